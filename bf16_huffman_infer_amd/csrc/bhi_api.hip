@@ -16,6 +16,16 @@ int bhi_launch_status(const char* what) {
     return (int)e;
 }
 
+extern "C" uint64_t bhi_stream_capture_id(void* stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo((hipStream_t)stream, &status, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return status == hipStreamCaptureStatusActive ? (uint64_t)id + 1 : 0;
+}
+
 extern "C" const char* bhi_last_error_string(void) { return g_err; }
 
 extern "C" int bhi_constants(int32_t* out, int n) {

@@ -20,6 +20,7 @@ import torch
 from torch import nn
 
 from .utils import shallow_copy_model
+from .workspace import Recording
 
 __all__ = ["GraphedCallable", "apply_graphed", "get_graphed_model"]
 
@@ -44,15 +45,18 @@ class GraphedCallable:
         # somebody else while replays still read it.
         self.fn = fn
         self.static_inputs = [a.clone() for a in sample_args]
+        # what the kernels need beside their operands: held here, so that no node of the graph
+        # has to prepare it at every replay
+        self.workspaces = Recording()
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(side), torch.no_grad():
+        with torch.cuda.stream(side), torch.no_grad(), self.workspaces.warmup():
             for _ in range(warmup):
                 fn(*self.static_inputs)
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
-        with torch.no_grad(), torch.cuda.graph(self.graph):
+        with torch.no_grad(), self.workspaces.capture(), torch.cuda.graph(self.graph):
             self.static_outputs = fn(*self.static_inputs)
 
     def __call__(self, *args: torch.Tensor):

@@ -15,6 +15,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
+from .workspace import workspace
 
 _LIB = torch.library.Library("bf16_huffman_infer", "DEF")
 _LIB.define("gemv_bf16_huffman(Tensor A_rem, Tensor A_exp, Tensor X, Tensor(a!) Y, Tensor offsets, "
@@ -382,6 +383,9 @@ def silu_mul(gate: Tensor, up: Tensor) -> Tensor:
     return out
 
 
+ATTENTION_COUNTER_BYTES = 4096       # of a workspace of the attention step: one per k/v head and tile of q heads
+
+
 def decode_attention(qk: Tensor, v: Tensor, norm_weight, cos: Tensor, sin: Tensor, pos: Tensor, k_cache: Tensor,
                      v_cache: Tensor, out: Tensor = None, eps: float = 1e-6, scale: float = None) -> Tensor:
     """The attention step of one new token of a decoder layer in one launch (no counterpart in the
@@ -409,14 +413,22 @@ def decode_attention(qk: Tensor, v: Tensor, norm_weight, cos: Tensor, sin: Tenso
     elif tuple(out.shape) != (q_heads, d):
         raise RuntimeError(f"out must be [{q_heads}, {d}]")
     lib = _lib.load()
+    stream = _stream(qk)
     with torch.cuda.device(qk.device):
-        rc = lib.bhi_decode_attention(
+        need = int(lib.bhi_decode_attention_workspace_bytes(q_heads, kv_heads, d, max_len))
+        if need < 0:
+            _lib.check(need, "decode_attention")
+        ws = workspace("attention", qk.device, stream, need, ATTENTION_COUNTER_BYTES) if need else None
+        rc = lib.bhi_decode_attention_split(
             _req(qk, torch.bfloat16, "qk"), _req(v, torch.bfloat16, "v", qk),
             None if norm_weight is None else _req(norm_weight, torch.bfloat16, "norm_weight", qk),
             _req(cos, torch.float32, "cos", qk), _req(sin, torch.float32, "sin", qk), pos.data_ptr(),
             _req(k_cache, torch.bfloat16, "k_cache", qk), _req(v_cache, torch.bfloat16, "v_cache", qk),
             _req(out, torch.bfloat16, "out", qk), q_heads, kv_heads, d, max_len, float(eps),
-            float(d ** -0.5 if scale is None else scale), _stream(qk))
+            float(d ** -0.5 if scale is None else scale),
+            None if ws is None else ws.data_ptr(), need, stream)
+        if rc != 0 and ws is not None:
+            ws[:ATTENTION_COUNTER_BYTES].zero_()
     _lib.check(rc, "decode_attention")
     return out
 

@@ -258,11 +258,25 @@ int bhi_reference_ans_decode(const void* A_rem, const void* A_exp, int64_t exp_w
  * for each q head (q heads h * q_heads / kv_heads .. share k/v head h), `out` bf16
  * [q_heads, head_dim].  `qk` is bf16 [q_heads + kv_heads, head_dim] (q heads first), `v` bf16
  * [kv_heads, head_dim]; `pos` points to one int64 in DEVICE memory (a recorded graph follows
- * it); head_dim must be 128, max_len at most 8192.  q, k, the softmax weights and the output
- * are rounded to BF16 where a chain of BF16 torch operations would round them. */
+ * it); head_dim must be 128, max_len at most 8192.  q, k and the output are
+ * rounded to BF16 where a chain of BF16 torch operations would round them; the softmax weights
+ * stay in fp32. */
 int bhi_decode_attention(const void* qk, const void* v, const void* norm_weight, const void* cos, const void* sin,
                          const void* pos, void* k_cache, void* v_cache, void* out, int q_heads, int kv_heads,
                          int head_dim, int max_len, float eps, float scale, void* stream);
+/* The same step with the visible slots dealt to several blocks per k/v head, whose sums meet in
+ * `workspace`: at least bhi_decode_attention_workspace_bytes(...) bytes of device memory, 16-byte
+ * aligned, whose first 4 KiB were zero before the first launch that used it (every launch leaves
+ * them at zero) and which no launch that may overlap uses.  0 bytes: the step is not split and
+ * `workspace` may be null, as for bhi_decode_attention. */
+int64_t bhi_decode_attention_workspace_bytes(int q_heads, int kv_heads, int head_dim, int max_len);
+int bhi_decode_attention_split(const void* qk, const void* v, const void* norm_weight, const void* cos, const void* sin,
+                               const void* pos, void* k_cache, void* v_cache, void* out, int q_heads, int kv_heads,
+                               int head_dim, int max_len, float eps, float scale, void* workspace, int64_t workspace_bytes,
+                               void* stream);
+/* A number for the capture that `stream` is part of (never 0), or 0 where it is not being captured.
+ * What a capture allocates belongs to its graph: callers keep workspaces per capture, not per stream. */
+uint64_t bhi_stream_capture_id(void* stream);
 
 /* No counterpart in the reference: a measurement helper.  Enqueues a kernel in which
  * `wavefronts` wavefronts (a positive multiple of 4) each load a contiguous span of `src`

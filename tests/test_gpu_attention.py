@@ -103,3 +103,86 @@ def test_rejections(cuda):
         c64, s64 = tables(64, 64)
         ops.decode_attention(qk[:, :64].contiguous(), v[:, :64].contiguous(), None, c64, s64,
                              torch.zeros(1, dtype=torch.int64, device="cuda"), kc[..., :64].contiguous(), kc[..., :64].contiguous())
+
+
+def _case(q_heads, kv_heads, max_len, seed):
+    d = 128
+    g = torch.Generator(device="cuda").manual_seed(seed)
+
+    def rand(*shape, scale=1.0):
+        return (torch.randn(*shape, generator=g, device="cuda") * scale).bfloat16()
+    return (rand(q_heads + kv_heads, d, scale=3), rand(kv_heads, d), rand(kv_heads, max_len, d), rand(kv_heads, max_len, d),
+            *tables(max_len, d))
+
+
+def _step_error(qk, v, cos, sin, p, kc, vc, q_heads, kv_heads, call):
+    """Largest difference of ``call``'s output to the torch formulation, in units of its bound: half a
+    BF16 step for the output, and 2**-6 of the largest |v| for what last-place flips of q (2**-8 of
+    scores of a few tens at most, through the softmax) and the BF16 weights of the torch formulation can do."""
+    kc_ref, vc_ref = kc.clone(), vc.clone()
+    pos = torch.tensor([p], device="cuda")
+    want = torch_step(qk, v, None, cos, sin, pos, kc_ref, vc_ref, q_heads, kv_heads, 1e-6)
+    got = call(pos).float()
+    assert torch.equal(vc, vc_ref)
+    torch.testing.assert_close(kc.float(), kc_ref.float(), rtol=2 ** -7, atol=1e-3)
+    return ((got - want).abs() / (want.abs() * 2 ** -8 + 2 ** -6 * vc_ref.float().abs().max())).max().item()
+
+
+@pytest.mark.parametrize("q_heads,kv_heads", [(28, 4), (31, 1), (32, 1), (6, 2), (20, 1), (16, 16), (128, 64)])
+@pytest.mark.parametrize("max_len,positions", [(64, (0, 63)), (1000, (14, 15, 16, 47, 62, 63, 64, 65, 127, 128, 190, 999)),
+                                               (8192, (255, 256, 3967, 3968, 6000, 8191))])
+def test_split_edges(cuda, q_heads, kv_heads, max_len, positions):
+    """Slots at the edges of matrix tiles (16), of a wavefront's share, of splits (64 and its
+    multiples) and of the cache; groups of q heads that fill no tile, and more than one tile."""
+    from bf16_huffman_infer_amd import ops
+    qk, v, kc, vc, cos, sin = _case(q_heads, kv_heads, max_len, q_heads + max_len)
+    for p in positions:
+        err = _step_error(qk, v, cos, sin, p, kc, vc, q_heads, kv_heads,
+                          lambda pos: ops.decode_attention(qk, v, None, cos, sin, pos, kc, vc, eps=1e-6))
+        assert err <= 1.0, (p, err)
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,max_len,positions", [(28, 4, 8192, (0, 63, 64, 255, 256, 257, 5000)), (3, 3, 300, (299,))])
+def test_entry_without_workspace(cuda, q_heads, kv_heads, max_len, positions):
+    """The C entry that takes no workspace walks all slots in one block per q head."""
+    from bf16_huffman_infer_amd import _lib
+    qk, v, kc, vc, cos, sin = _case(q_heads, kv_heads, max_len, 5)
+    out = torch.empty(q_heads, 128, dtype=torch.bfloat16, device="cuda")
+
+    def call(pos):
+        _lib.check(_lib.load().bhi_decode_attention(
+            qk.data_ptr(), v.data_ptr(), None, cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+            out.data_ptr(), q_heads, kv_heads, 128, max_len, 1e-6, 128 ** -0.5, torch.cuda.current_stream().cuda_stream), "attention")
+        return out
+    for p in positions:
+        assert _step_error(qk, v, cos, sin, p, kc, vc, q_heads, kv_heads, call) <= 1.0, p
+
+
+@pytest.mark.parametrize("recorder", ["torch", "package"])
+def test_second_graph_does_not_depend_on_the_first(cuda, recorder):
+    """Two graphs recorded one after the other (torch records both on one stream): the second is
+    replayed alone, then both in turn, against the eager bits."""
+    from bf16_huffman_infer_amd import ops
+    from bf16_huffman_infer_amd.cudagraph_utils import GraphedCallable
+    qk, v, kc, vc, cos, sin = _case(32, 8, 4096, 9)
+    pos = torch.tensor([3000], device="cuda")
+    want = ops.decode_attention(qk, v, None, cos, sin, pos, kc, vc).clone()
+    graphs, outs = [], []
+    for _ in range(2):
+        out = torch.zeros_like(want)
+
+        def step(out=out):
+            return ops.decode_attention(qk, v, None, cos, sin, pos, kc, vc, out=out)
+        if recorder == "package":
+            graph = GraphedCallable(step, ())
+        else:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                step()
+        graphs.append(graph)
+        outs.append(out)
+    for i in (1, 1, 0, 1, 0, 0):
+        outs[i].zero_()
+        graphs[i].replay()
+        assert torch.equal(outs[i], want), i
+        assert torch.equal(ops.decode_attention(qk, v, None, cos, sin, pos, kc, vc), want)
