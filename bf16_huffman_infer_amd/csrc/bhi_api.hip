@@ -96,23 +96,53 @@ extern "C" int64_t bhi_stream_read(const void* src, int64_t bytes, int wavefront
 // ---------------------------------------------------------------------------------------------
 // The two layer pieces the GEMV can take in front of its product, as kernels of their own: the
 // unfused form of the same arithmetic (same reduction order, same roundings), used where the
-// fused form does not apply (more than four rows) and as the reference the fused form is
+// fused form does not apply (more than four rows) or does not pay, and as the reference the fused form is
 // tested against bit for bit.
 namespace bhi {
-template <int BS>
+// One block per row: bound by latency (load, reduction, store; a row is a few KB), so a row of up to
+// 512 * N elements is requested at once, with its share of gamma, and stays in registers between the
+// sum and the product; longer rows are read twice.  Eight rows of 3584, two launches of four rows
+// whose blocks each summed every row: 9.2 us; this kernel 2.5 us (one row of 4096 2.9 -> 2.4 us), of
+// which 2.3 is what any launch takes inside a graph.
+template <int N>
 __global__ __launch_bounds__(kBlockThreads) void rms_norm_kernel(const uint16_t* __restrict__ X, const uint16_t* __restrict__ gamma,
                                                                  uint16_t* __restrict__ out, int K, float eps) {
-    __shared__ float part[kWavesPerBlock * BS];
-    float r[BS];
-    rms_scales_start<BS>(X, K, part);
-    __syncthreads();
-    rms_scales_finish<BS>(part, K, eps, r);
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;          // pair index
-    if (p < K / 2) {
-        const uint32_t g = ((const uint32_t*)gamma)[p];
+    __shared__ float part[kWavesPerBlock];
+    const uint32_t* x = (const uint32_t*)X + (size_t)blockIdx.x * (K / 2);
+    const uint32_t* g = (const uint32_t*)gamma;
+    uint32_t* y = (uint32_t*)out + (size_t)blockIdx.x * (K / 2);
+    constexpr int kHeld = N > 0 ? N : 1;
+    uint32_t xr[kHeld], gr[kHeld];
+    float r[1];
+    if (N > 0) {
+        float sq = 0.f;
 #pragma unroll
-        for (int b = 0; b < BS; ++b)
-            ((uint32_t*)out)[(size_t)b * (K / 2) + p] = rms_pair(((const uint32_t*)X)[(size_t)b * (K / 2) + p], r[b], g);
+        for (int i = 0; i < kHeld; ++i) {
+            const int p = (int)threadIdx.x + i * kBlockThreads;
+            xr[i] = p < K / 2 ? x[p] : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i) {
+            const int p = (int)threadIdx.x + i * kBlockThreads;
+            gr[i] = p < K / 2 ? g[p] : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i) add_squares(sq, xr[i]);
+        sq = wave_sum(sq);
+        if ((threadIdx.x & (kLanes - 1)) == 0) part[threadIdx.x / kLanes] = sq;
+    } else {
+        rms_scales_start<1>((const uint16_t*)x, K, part);
+    }
+    lds_barrier();
+    rms_scales_finish<1>(part, K, eps, r);
+    if (N > 0) {
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i) {
+            const int p = (int)threadIdx.x + i * kBlockThreads;
+            if (p < K / 2) y[p] = rms_pair(xr[i], r[0], gr[i]);
+        }
+    } else {
+        for (int p = threadIdx.x; p < K / 2; p += kBlockThreads) y[p] = rms_pair(x[p], r[0], g[p]);
     }
 }
 
@@ -126,16 +156,16 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const uint32_t* __restric
 extern "C" int bhi_rms_norm(const void* X, const void* gamma, void* out, int rows, int K, float eps, void* stream) {
     using namespace bhi;
     if (!X || !gamma || !out) return bhi_fail(BHI_EINVAL, "null pointer");
-    if (rows < 1 || rows > 4 || K < 2 || K % 2 != 0) return bhi_fail(BHI_EINVAL, "rms_norm takes 1 to 4 rows of an even length");
-    const dim3 grid((unsigned)((K / 2 + kBlockThreads - 1) / kBlockThreads)), block(kBlockThreads);
+    if (rows < 1 || K < 2 || K % 2 != 0) return bhi_fail(BHI_EINVAL, "rms_norm takes one or more rows of an even length");
+    const dim3 grid((unsigned)rows), block(kBlockThreads);
     const uint16_t *x = (const uint16_t*)X, *g = (const uint16_t*)gamma;
     uint16_t* o = (uint16_t*)out;
-    switch (rows) {
-        case 1: hipLaunchKernelGGL(rms_norm_kernel<1>, grid, block, 0, (hipStream_t)stream, x, g, o, K, eps); break;
-        case 2: hipLaunchKernelGGL(rms_norm_kernel<2>, grid, block, 0, (hipStream_t)stream, x, g, o, K, eps); break;
-        case 3: hipLaunchKernelGGL(rms_norm_kernel<3>, grid, block, 0, (hipStream_t)stream, x, g, o, K, eps); break;
-        default: hipLaunchKernelGGL(rms_norm_kernel<4>, grid, block, 0, (hipStream_t)stream, x, g, o, K, eps); break;
-    }
+    // the shortest row each is built for: 512 elements per held pair
+    if (K <= 512 * 4) hipLaunchKernelGGL(rms_norm_kernel<4>, grid, block, 0, (hipStream_t)stream, x, g, o, K, eps);
+    else if (K <= 512 * 8) hipLaunchKernelGGL(rms_norm_kernel<8>, grid, block, 0, (hipStream_t)stream, x, g, o, K, eps);
+    else if (K <= 512 * 16) hipLaunchKernelGGL(rms_norm_kernel<16>, grid, block, 0, (hipStream_t)stream, x, g, o, K, eps);
+    else if (K <= 512 * 40) hipLaunchKernelGGL(rms_norm_kernel<40>, grid, block, 0, (hipStream_t)stream, x, g, o, K, eps);
+    else hipLaunchKernelGGL(rms_norm_kernel<0>, grid, block, 0, (hipStream_t)stream, x, g, o, K, eps);
     return bhi_launch_status("rms_norm");
 }
 

@@ -78,14 +78,9 @@ constexpr int kAttnPartial = kAttnDim + 2;   // weighted sum, maximum, sum of we
 __device__ __forceinline__ float bf16_lo(uint32_t pair) { return __uint_as_float(pair << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t pair) { return __uint_as_float(pair & 0xFFFF0000u); }
 
-// Reductions over the lanes of a wavefront without a trip through the LDS crossbar (six dependent
-// __shfl_xor in a row are longer than the rest of a head's normalisation): rotations inside rows
-// of 16 lanes (DPP), then the two row-swap instructions of gfx950.
+// Reductions without a trip through the LDS crossbar (six dependent __shfl_xor in a row are longer
+// than the rest of a head's normalisation): the two row-swap instructions of gfx950.
 typedef uint32_t swapped_t __attribute__((ext_vector_type(2)));
-template <int CTRL>
-__device__ __forceinline__ float row_rotated(float v) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), CTRL, 0xF, 0xF, false));
-}
 template <class Op>
 __device__ __forceinline__ float across_halves(float v, Op op) {            // lanes l and l ^ 32
     const swapped_t p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -98,13 +93,6 @@ __device__ __forceinline__ float across_rows(float v, Op op) {              // t
 }
 struct Add { __device__ __forceinline__ float operator()(float x, float y) const { return x + y; } };
 struct Max { __device__ __forceinline__ float operator()(float x, float y) const { return fmaxf(x, y); } };
-__device__ __forceinline__ float wave_sum(float v) {
-    v += row_rotated<0x121>(v);
-    v += row_rotated<0x122>(v);
-    v += row_rotated<0x124>(v);
-    v += row_rotated<0x128>(v);
-    return across_rows(v, Add{});
-}
 
 // One head by one wavefront: RMSNorm (fp32, weight applied after the normalisation) and
 // rotation; lane l holds elements l and l + 64, the two halves the rotation pairs up.  Loads and

@@ -94,6 +94,26 @@ __device__ __forceinline__ float sum_over_column_blocks(float a) {
     return __uint_as_float(p.x) + __uint_as_float(p.y);
 }
 
+// Sum over all 64 lanes, left in every lane: the butterfly over lane distances 1, 2, 4, ..., 32 (each
+// lane adds what its partner holds, so the pairing and with it every bit of the sum is that of six
+// __shfl_xor steps), as DPP moves -- quad permutations, then mirrors of half rows and rows, whose
+// quads are equal by then -- and the two row swaps.
+template <int CTRL>
+__device__ __forceinline__ float dpp_partner(float v) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float wave_sum(float v) {
+    v += dpp_partner<0xB1>(v);               // quad_perm:[1,0,3,2]
+    v += dpp_partner<0x4E>(v);               // quad_perm:[2,3,0,1]
+    v += dpp_partner<0x141>(v);              // row_half_mirror
+    v += dpp_partner<0x140>(v);              // row_mirror
+    typedef uint32_t pair_t __attribute__((ext_vector_type(2)));
+    pair_t p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(p.x) + __uint_as_float(p.y);
+    p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(p.x) + __uint_as_float(p.y);
+}
+
 // A word of memory that nothing writes while the kernel runs (offsets, the format header),
 // read at a wave-uniform address: through the constant address space the compiler issues a
 // scalar load, which neither queues behind the vector loads in flight nor has to be waited

@@ -303,39 +303,51 @@ __device__ __forceinline__ uint32_t silu_mul_pair(uint32_t g, uint32_t u) {
     return f32_to_pair(f32x2_t{sf.x * uf.x, sf.y * uf.y});
 }
 
-// rsqrt(mean(x^2) + eps) of every batch row, by a whole block: thread t squares the pairs
-// t, t + T, ... of each row, a wavefront adds its lanes' sums by xor-shuffles, the
+__device__ __forceinline__ void add_squares(float& sum, uint32_t pair) {
+    const f32x2_t v = pair_to_f32(pair);
+    sum += v.x * v.x;
+    sum += v.y * v.y;
+}
+
+// rsqrt(mean(x^2) + eps) of every batch row, by a block of 256 threads: thread t squares the pairs
+// t, t + 256, ... of each row, a wavefront adds its lanes' sums (wave_sum), the
 // wavefronts' sums meet in `part` ([waves][BS] floats in LDS) and are added in order after
 // the caller's next barrier (rms_scales_finish).  The same code serves the stand-alone
 // RMSNorm kernel, which is what makes fused and unfused results identical.
 template <int BS>
 __device__ __forceinline__ void rms_scales_start(const uint16_t* __restrict__ X, int K, float* part) {
+    constexpr int kAhead = 8 / BS;                                // loads in flight: one round trip each would be most of the work
     const int lane = threadIdx.x & (kLanes - 1), wave = threadIdx.x / kLanes;
     float sq[BS];
 #pragma unroll
     for (int b = 0; b < BS; ++b) sq[b] = 0.f;
-    for (int p = threadIdx.x; p < K / 2; p += blockDim.x) {
+    for (int p0 = threadIdx.x; p0 < K / 2; p0 += kAhead * kBlockThreads) {
+        uint32_t x[kAhead][BS];
 #pragma unroll
-        for (int b = 0; b < BS; ++b) {
-            const f32x2_t v = pair_to_f32(((const uint32_t*)X)[(size_t)b * (K / 2) + p]);
-            sq[b] += v.x * v.x;
-            sq[b] += v.y * v.y;
+        for (int i = 0; i < kAhead; ++i) {
+            const int p = p0 + i * kBlockThreads;
+#pragma unroll
+            for (int b = 0; b < BS; ++b) x[i][b] = p < K / 2 ? ((const uint32_t*)X)[(size_t)b * (K / 2) + p] : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < kAhead; ++i) {
+#pragma unroll
+            for (int b = 0; b < BS; ++b) add_squares(sq[b], x[i][b]);
         }
     }
 #pragma unroll
     for (int b = 0; b < BS; ++b) {
-        float v = sq[b];
-        for (int o = 1; o < kLanes; o <<= 1) v += __shfl_xor(v, o);
+        const float v = wave_sum(sq[b]);
         if (lane == 0) part[wave * BS + b] = v;
     }
 }
 template <int BS>
 __device__ __forceinline__ void rms_scales_finish(const float* part, int K, float eps, float (&r)[BS]) {
-    const int waves = blockDim.x / kLanes;
 #pragma unroll
     for (int b = 0; b < BS; ++b) {
         float v = 0.f;
-        for (int w = 0; w < waves; ++w) v += part[w * BS + b];
+#pragma unroll
+        for (int w = 0; w < kWavesPerBlock; ++w) v += part[w * BS + b];
         r[b] = 1.0f / sqrtf(v / (float)K + eps);
     }
 }

@@ -357,16 +357,14 @@ def gemv_bf16_grouped(weights, X: Tensor, Ys, biases=None, residuals=None, x_mod
 def rms_norm(x: Tensor, gamma: Tensor, eps: float) -> Tensor:
     """``bf16(x * rsqrt(mean(x^2) + eps) * gamma)`` over the last dimension, one rounding: the
     arithmetic (reduction order included) of the RMSNorm that :func:`gemv_bf16_grouped` fuses."""
-    lib = _lib.load()
     K = x.shape[-1]
     flat = x.reshape(-1, K).contiguous()
     out = torch.empty_like(flat)
     g = _req(gamma.contiguous(), torch.bfloat16, "gamma", flat)
-    with torch.cuda.device(flat.device):
-        for r0 in range(0, flat.shape[0], X_TRANSFORM_MAX_ROWS):
-            rows = flat[r0:r0 + X_TRANSFORM_MAX_ROWS]
-            _lib.check(lib.bhi_rms_norm(_req(rows, torch.bfloat16, "x"), g, out[r0:].data_ptr(), rows.shape[0], K, float(eps),
-                                        _stream(flat)), "rms_norm")
+    if flat.shape[0] > 0:
+        with torch.cuda.device(flat.device):
+            _lib.check(_lib.load().bhi_rms_norm(_req(flat, torch.bfloat16, "x"), g, out.data_ptr(), flat.shape[0], K, float(eps),
+                                                _stream(flat)), "rms_norm")
     return out.view(x.shape)
 
 

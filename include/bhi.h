@@ -176,7 +176,7 @@ int bhi_gemv_bf16_huffman_grouped_x(const bhi_gemv_member* members, int n_member
 int bhi_gemv_bf16_ans_grouped_x(const bhi_gemv_member* members, int n_members, const void* X,
                                 int split_k, int Ks, int batch, int x_mode, const void* x_aux, float eps,
                                 void* stream);
-/* The same two pieces as kernels of their own (1..4 rows; out may not alias the inputs of
+/* The same two pieces as kernels of their own (any number of rows; out may not alias the inputs of
  * bhi_rms_norm): out = bf16(x * r * gamma) with one rounding; out = bf16(bf16(silu(gate)) * up). */
 int bhi_rms_norm(const void* X, const void* gamma, void* out, int rows, int K, float eps, void* stream);
 int bhi_silu_mul(const void* gate, const void* up, void* out, int64_t n, void* stream);
