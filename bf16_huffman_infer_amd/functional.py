@@ -401,6 +401,40 @@ class CompressedLinear(nn.Module):
         return F.linear(input, self.weight, self.bias)
 
 
+def fuses_input(rows: int, n_weights: int, norm: bool, huffman: bool) -> bool:
+    """Whether the RMSNorm (``norm``) or the SwiGLU product in front of a GEMV of ``n_weights`` weights
+    in all happens inside its launch or in a launch of its own.
+
+    A launch of its own costs 2.4 us.  Inside, every wavefront transforms the X of every step and row
+    it multiplies, in a kernel whose steps are short of issue slots as it is: the cost grows with rows
+    times weights.  Measured on MI355X in recorded graphs (us, inside / of its own):
+
+    ==================================  ===========  ===========  ===========  ===========
+    launch                              1 row        2 rows       3 rows       4 rows
+    ==================================  ===========  ===========  ===========  ===========
+    Huffman, norm, 1536x1024            5.9 / 7.0    6.2 / 7.6    6.6 / 7.5    6.9 / 7.7
+    Huffman, norm, 3072x2048            8.1 / 8.6    8.7 / 9.3    9.6 / 9.5    10.3 / 9.7
+    Huffman, norm, 4608x3584            11.3 / 11.4  12.5 / 12.1  14.3 / 12.9  16.2 / 13.6
+    Huffman, norm, 6144x4096            12.7 / 13.0  14.6 / 13.9  18.8 / 14.4  20.8 / 15.2
+    Huffman, norm, 24576x4096           34.4 / 32.6  38.8 / 34.9  46.9 / 36.6  50.8 / 34.2
+    Huffman, SwiGLU, 1024x3072          6.4 / 8.0    6.7 / 8.4    7.1 / 8.4    7.7 / 8.6
+    Huffman, SwiGLU, 2048x8192          11.3 / 12.6  13.2 / 12.9  14.9 / 13.2  16.7 / 13.5
+    Huffman, SwiGLU, 4096x12288         20.8 / 21.0  26.0 / 21.7  31.9 / 21.7  36.1 / 22.8
+    Huffman, SwiGLU, 3584x18944         28.8 / 26.3  34.9 / 28.0  42.6 / 29.5  49.6 / 30.3
+    rANS, norm, 6144x4096               16.0 / 16.1  18.4 / 17.2  21.7 / 17.6  24.6 / 18.2
+    rANS, norm, 24576x4096              44.0 / 40.7  49.7 / 43.5  57.6 / 46.0  65.2 / 43.7
+    rANS, SwiGLU, 1024x3072             7.1 / 8.8    7.6 / 9.0    8.1 / 9.2    8.6 / 9.4
+    rANS, SwiGLU, 2048x8192             14.6 / 15.0  16.1 / 15.2  17.7 / 15.4  19.2 / 15.8
+    rANS, SwiGLU, 4096x12288            28.8 / 26.1  34.1 / 27.0  38.9 / 27.4  42.4 / 28.2
+    ==================================  ===========  ===========  ===========  ===========
+    """
+    if rows > _ops.X_TRANSFORM_MAX_ROWS:
+        return False
+    if rows == 1:
+        return n_weights <= (28e6 if norm else 51e6 if huffman else 20e6)
+    return rows * n_weights <= (18e6 if norm else 22e6)
+
+
 def linear_grouped(input: Tensor, weights, biases=None, *, residuals=None, input_norm=None, input_gate=None,
                    outs=None) -> list:
     """``[F.linear(h, w, b) (+ r) for w, b, r in zip(weights, biases, residuals)]`` in ONE launch, where
@@ -415,7 +449,7 @@ def linear_grouped(input: Tensor, weights, biases=None, *, residuals=None, input
     separate BF16 addition would; ``outs[i]`` (bf16 ``[rows, M_i]``, contiguous -- a column slice of a
     one-row buffer qualifies) receives output ``i`` instead of a new tensor.  This is what the q/k/v (or gate/up) projections of a
     decoder layer need: the reference overlaps them on parallel streams
-    (``cudastream_utils.py:8-47``), here they are one grid.  Up to 4 rows (Huffman, rANS) the
+    (``cudastream_utils.py:8-47``), here they are one grid.  Where it pays (:func:`fuses_input`) the
     norm / gate product happens inside the kernel; otherwise it runs as this package's own
     elementwise kernel first -- the same arithmetic, the same bits.
     """
@@ -429,7 +463,8 @@ def linear_grouped(input: Tensor, weights, biases=None, *, residuals=None, input
     split_k, _, N = first.rem.shape
     mode, aux, eps = _ops.X_PLAIN, None, 0.0
     if input_norm is not None or input_gate is not None:
-        fusable = x.size(0) <= _ops.X_TRANSFORM_MAX_ROWS and not isinstance(first, NibbleWeight)
+        fusable = not isinstance(first, NibbleWeight) and fuses_input(
+            x.size(0), sum(w.rem.numel() for w in weights), input_norm is not None, hasattr(first, 'LUT1'))
         if input_norm is not None:
             gamma, eps = input_norm
             gamma = gamma.detach()
