@@ -44,6 +44,7 @@ struct AnsTable {
 
 struct AnsCodec {
     using Cursor = AnsCursor;
+    template <int RING> using TileCursor = AnsTileCursor<RING>;
     using Table = AnsTable;
     static constexpr bool kTransformsX = true;    // kernels with RMSNorm / SiLU*mul in front of the product are built
     static constexpr int kTableWords = kAnsTableWords;
@@ -164,6 +165,13 @@ extern "C" int bhi_gemm_bf16_ans(const bhi_gemv_member* weight, const void* X, i
     if (int rc = launch_mma<AnsCodec>(weight, 1, X, split_k, Ks, batch, workspace, workspace_bytes, 0, true,
                                       (hipStream_t)stream)) return rc;
     return bhi_launch_status("gemm_bf16_ans");
+}
+
+extern "C" int bhi_tile_bf16_ans(const bhi_gemv_member* weight, const void* X, int split_k, int Ks, int batch,
+                                 void* workspace, int64_t workspace_bytes, void* stream) {
+    if (int rc = launch_tile<AnsCodec>(weight, X, split_k, Ks, batch, workspace, workspace_bytes, 0, true,
+                                        (hipStream_t)stream)) return rc;
+    return bhi_launch_status("tile_bf16_ans");
 }
 
 extern "C" int bhi_gemm_bf16_ans_grouped(const bhi_gemv_member* members, int n_members, const void* X, int split_k,

@@ -176,7 +176,8 @@ constexpr int kSegLong = 4;
 #define BHI_RING_ROWS 16
 #endif
 constexpr int kRingRows = BHI_RING_ROWS;
-constexpr int kRingRowsLog2 = kRingRows == 8 ? 3 : kRingRows == 16 ? 4 : kRingRows == 32 ? 5 : -1;
+constexpr int ring_rows_log2(int rows) { return rows == 8 ? 3 : rows == 16 ? 4 : rows == 32 ? 5 : -1; }
+constexpr int kRingRowsLog2 = ring_rows_log2(kRingRows);
 static_assert(kRingRowsLog2 > 0, "ring of 8, 16 or 32 rows");
 #ifndef BHI_PRIME_ROWS
 #define BHI_PRIME_ROWS 8
@@ -408,7 +409,8 @@ struct AnsCursor : RowRingT<0> {
     }
 
     // one symbol: returns the second word of its table entry ((sym << 23) | rem), advances the state
-    __device__ __forceinline__ uint32_t symbol(const uint32_t* __restrict__ table) {
+    __device__ __forceinline__ uint32_t symbol(const uint32_t* __restrict__ table) { return symbol(table, xl, xh); }
+    static __device__ __forceinline__ uint32_t symbol(const uint32_t* __restrict__ table, uint32_t& xl, uint32_t& xh) {
         // byte 0 of the state, times eight, in one instruction (written as a mask and a shift
         // the compiler makes it two; eight symbols per step, the kernel is bound by VALU issue)
         uint32_t off;

@@ -12,6 +12,7 @@ namespace bhi {
 
 struct HuffCodec {
     using Cursor = HuffCursor;
+    template <int RING> using TileCursor = HuffTileCursor<RING>;
     static constexpr bool kTransformsX = true;    // kernels with RMSNorm / SiLU*mul in front of the product are built
     static constexpr int kTableWords = kTableEntries;
     using Table = PlainTable<kTableEntries>;
@@ -146,6 +147,13 @@ extern "C" int bhi_gemm_bf16_huffman(const bhi_gemv_member* weight, const void* 
     return bhi_launch_status("gemm_bf16_huffman");
 }
 
+extern "C" int bhi_tile_bf16_huffman(const bhi_gemv_member* weight, const void* X, int split_k, int Ks, int batch,
+                                 void* workspace, int64_t workspace_bytes, void* stream) {
+    if (int rc = launch_tile<HuffCodec>(weight, X, split_k, Ks, batch, workspace, workspace_bytes, (int64_t)kTableEntries * 4, false,
+                                        (hipStream_t)stream)) return rc;
+    return bhi_launch_status("tile_bf16_huffman");
+}
+
 extern "C" int bhi_gemm_bf16_huffman_grouped(const bhi_gemv_member* members, int n_members, const void* X, int split_k,
                                              int Ks, int batch, void* stream) {
     if (int rc = launch_mma<HuffCodec>(members, n_members, X, split_k, Ks, batch, nullptr, 0,
@@ -212,6 +220,13 @@ extern "C" int64_t bhi_gemm_workspace_bytes(int split_k, int M, int Ks, int batc
     if (batch < 1 || batch > kMmaMaxBatch) return bhi_fail(BHI_EBATCH, "the fused matrix product takes 1 to 32 rows of X");
     if (int rc = check_shape(split_k, M, Ks, kTailPadWords, &s)) return rc;
     return mma_workspace_bytes(s, batch);
+}
+
+extern "C" int64_t bhi_tile_workspace_bytes(int split_k, int M, int Ks, int batch) {
+    Shape s;
+    if (batch < kTileMinBatch || batch > kTileMaxBatch) return bhi_fail(BHI_EBATCH, "the tiled product takes 17 to 128 rows of X");
+    if (int rc = check_shape(split_k, M, Ks, kTailPadWords, &s)) return rc;
+    return tile_workspace_bytes(s, batch);
 }
 
 extern "C" int64_t bhi_encode_capacity(int n_steps) {

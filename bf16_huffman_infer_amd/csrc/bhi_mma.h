@@ -434,6 +434,24 @@ static inline bhi::Shape mma_group_shape(const bhi::Shape& first, long long rows
     return s;
 }
 
+// One member of a launch from the caller's description of it, not cut along K.
+static inline int fill_mma_member(bhi::MmaArgs& a, const bhi_gemv_member& m, int split_k, int Ks, int batch,
+                                  int64_t table_bytes_expected, bool header_is_table) {
+    using namespace bhi;
+    if (!m.A_rem || !m.A_exp || !m.Y || !m.offsets || !m.table || (!header_is_table && !m.header))
+        return bhi_fail(BHI_EINVAL, "null pointer in a group member");
+    if (table_bytes_expected > 0 && m.table_bytes != table_bytes_expected)
+        return bhi_fail(BHI_ELAYOUT, "decode table has the wrong size");
+    if (int rc = check_shape(split_k, m.M, Ks, m.exp_words, &a.s)) return rc;
+    a.rem = (const uint8_t*)m.A_rem; a.exp = (const uint32_t*)m.A_exp; a.Y = (uint16_t*)m.Y;
+    a.offsets = (const uint32_t*)m.offsets; a.table = (const uint32_t*)m.table;
+    a.header = (const uint8_t*)(header_is_table ? m.table : m.header); a.bias = (const uint16_t*)m.bias;
+    a.residual = (const uint16_t*)m.residual;
+    a.batch = batch; a.slices = 1;
+    a.counters = nullptr; a.partial = nullptr;
+    return 0;
+}
+
 template <class Codec>
 static inline int launch_mma(const bhi_gemv_member* members, int n_members, const void* X, int split_k, int Ks, int batch,
                              void* workspace, int64_t workspace_bytes, int64_t table_bytes_expected, bool header_is_table,
@@ -445,20 +463,8 @@ static inline int launch_mma(const bhi_gemv_member* members, int n_members, cons
     MmaGroup grp = {};
     long long rows = 0;
     for (int i = 0; i < n_members; ++i) {
-        const bhi_gemv_member& m = members[i];
-        if (!m.A_rem || !m.A_exp || !m.Y || !m.offsets || !m.table || (!header_is_table && !m.header))
-            return bhi_fail(BHI_EINVAL, "null pointer in a group member");
-        if (table_bytes_expected > 0 && m.table_bytes != table_bytes_expected)
-            return bhi_fail(BHI_ELAYOUT, "decode table has the wrong size");
-        MmaArgs& a = grp.m[i];
-        if (int rc = check_shape(split_k, m.M, Ks, m.exp_words, &a.s)) return rc;
-        a.rem = (const uint8_t*)m.A_rem; a.exp = (const uint32_t*)m.A_exp; a.Y = (uint16_t*)m.Y;
-        a.offsets = (const uint32_t*)m.offsets; a.table = (const uint32_t*)m.table;
-        a.header = (const uint8_t*)(header_is_table ? m.table : m.header); a.bias = (const uint16_t*)m.bias;
-        a.residual = (const uint16_t*)m.residual;
-        a.batch = batch; a.slices = 1;
-        a.counters = nullptr; a.partial = nullptr;
-        rows += m.M;
+        if (int rc = fill_mma_member(grp.m[i], members[i], split_k, Ks, batch, table_bytes_expected, header_is_table)) return rc;
+        rows += members[i].M;
     }
     if (rows > 0x7FFFFFFFll) return bhi_fail(BHI_EINVAL, "group too large for one launch");
     const int Q = (batch + 3) / 4;

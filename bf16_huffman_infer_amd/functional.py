@@ -733,6 +733,58 @@ def prefers_matrix_cores(rows: int, M: int, K: int) -> bool:
     return rows >= 3 and M >= 32768 and K >= 3584
 
 
+def prefers_tiles(rows: int, M: int, K: int) -> bool:
+    """Whether ``rows`` > 16 rows of activations go through the tiled product (``bhi_tile.h``) rather than
+    the matrix-core kernel (up to 32 rows) or decoding and a dense GEMM (above).  Measured on MI355X (us,
+    before / tiled; more in ``bhi_tile.h``):
+
+    ====================  ===========  ===========  ============  ===========
+    M x K                 17 rows      48 rows      96 rows       128 rows
+    ====================  ===========  ===========  ============  ===========
+    512x3584              14.7 / 12.9  18.0 / 14.4  19.0 / 21.8   19.7 / 25.4
+    1536x1024             12.6 / 10.0  12.7 / 11.3  12.8 / 17.5   12.9 / 20.1
+    1024x4096             15.8 / 14.0  23.7 / 16.0  17.4 / 24.7   20.4 / 27.5
+    2048x8192             23.5 / 18.3  28.7 / 20.2  31.8 / 29.6   32.9 / 34.0
+    4096x4096             22.2 / 16.9  26.9 / 18.7  32.4 / 25.3   34.4 / 31.0
+    4096x11008 (rANS)     37.8 / 41.0  56.0 / 42.8  71.2 / 51.1
+    3584x18944            42.1 / 47.5  119 / 52.0   108 / 62.4    117 / 91.7
+    ====================  ===========  ===========  ============  ===========
+
+    A small layer's weight stays in the caches between the decoder and the GEMM, whose library kernel
+    gains on this one with every row; long rows in few row groups leave the tiled kernel few wavefronts,
+    and at 17 to 20 rows the other one needs five quads of batch rows only."""
+    if rows <= 20:
+        return K < 11008
+    if rows <= 64:
+        return True
+    return M * K >= 16 << 20
+
+
+def _fuses_above_32_rows(input: Tensor, bias: Optional[Tensor]) -> bool:
+    """Decoding and ``F.linear`` pass gradients, forward-mode tangents, function transforms, autocast and
+    dispatch modes on to the input (and the bias); a fused product does not, and takes over only where none
+    of them is in play."""
+    if torch.is_grad_enabled() and (input.requires_grad or (bias is not None and bias.requires_grad)):
+        return False
+    if torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    if torch.is_autocast_enabled('cuda') or torch._C._len_torch_dispatch_stack():
+        return False
+    return type(input) in (Tensor, nn.Parameter)
+
+
+def _tiled(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool:
+    rows = input.size(0)
+    if not _ops.TILE_MIN_ROWS <= rows <= _ops.TILE_MAX_ROWS or isinstance(weight, NibbleWeight):
+        return False
+    split_k, M, N = weight.rem.shape
+    if input.dtype != torch.bfloat16 or (bias is not None and bias.dtype != torch.bfloat16) or not input.is_cuda:
+        return False
+    if input.size(1) != split_k * N or input.numel() >= 2 ** 31 or not prefers_tiles(rows, M, split_k * N):
+        return False
+    return rows <= GEMM_MAX_ROWS or ((bias is None or tuple(bias.shape) == (M,)) and _fuses_above_32_rows(input, bias))
+
+
 def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], fused) -> Tensor:
     assert input.dim() >= 2, input
     shape = input.shape
@@ -749,6 +801,14 @@ def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tens
         output = fused(input)
         if bias is not None:
             output += bias[None, :]
+    elif _tiled(input, weight, bias):
+        # 17..128 rows where the rule says so: as below, sixteen weight rows at a time
+        x = (input if input.size(0) <= GEMM_MAX_ROWS else input.contiguous()).view(-1, split_k, N).contiguous()
+        if x.data_ptr() % 16:
+            x = x.clone()
+        _check_weight_call(weight.rem, weight.exp, x)
+        output = torch.empty((x.size(0), M), dtype=torch.bfloat16, device=x.device)
+        _ops.tile_bf16(weight, x, output, None if bias is None else bias.detach().contiguous())
     elif wide or (input.size(0) <= GEMM_MAX_ROWS and not isinstance(weight, NibbleWeight) and input.dtype == torch.bfloat16
                   and (bias is None or bias.dtype == torch.bfloat16)):
         # 9..32 rows (and fewer where the rule above says so): decode inside the matrix-core kernel,
@@ -763,8 +823,8 @@ def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tens
 
 
 def linear_huffman(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor] = None) -> Tensor:
-    """``F.linear`` with a :class:`HuffmanWeight`: fused kernel up to 8 rows, else decode +
-    dense GEMM (reference ``functional.py:390-411``)."""
+    """``F.linear`` with a :class:`HuffmanWeight`: fused kernels up to 32 rows and, where they are faster,
+    up to 128, else decode + dense GEMM (reference ``functional.py:390-411``)."""
     return _linear_compressed(input, weight, bias, lambda x: mv_huffman(
         weight.rem, weight.exp, x, weight.offsets,
         weight.LUT1, weight.LUT2, weight.LUT3, weight.LUT4, weight.code_lengths))

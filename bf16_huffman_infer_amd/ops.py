@@ -528,6 +528,38 @@ def gemm_bf16(weight, X: Tensor, Y: Tensor, bias=None, static_workspace: bool = 
     _lib.check(rc, name)
 
 
+TILE_MIN_ROWS, TILE_MAX_ROWS = 17, 128
+TILE_COUNTER_BYTES = 1024            # of a workspace of the tiled product: one per row block of a product cut along K
+
+
+def tile_bf16(weight, X: Tensor, Y: Tensor, bias=None) -> None:
+    """``Y = X @ W.T (+ bias)`` for 17 to 128 rows of ``X`` with ``W`` held compressed (:class:`HuffmanWeight`
+    or :class:`ANSWeight`), decoded inside a matrix-core kernel that multiplies sixteen weight rows at a
+    time.  Arguments as :func:`gemm_bf16`; partial sums of K slices meet in a workspace of the
+    (device, stream) or of the capture (:mod:`.workspace`)."""
+    lib = _lib.load()
+    split_k, M, Ks = _weight_dims(weight.rem, weight.offsets)
+    if X.dim() != 3 or X.shape[1] != split_k or X.shape[2] != Ks:
+        raise RuntimeError(f"X must be [rows, {split_k}, {Ks}], got {tuple(X.shape)}")
+    rows = X.shape[0]
+    if tuple(Y.shape) != (rows, M):
+        raise RuntimeError(f"Y must be [{rows}, {M}], got {tuple(Y.shape)}")
+    member = (_lib.GemvMember * 1)()
+    x_ptr = _req(X, torch.bfloat16, "X", weight.rem)
+    name = "tile_bf16_huffman" if _fill_member(member[0], weight, Y, bias, weight.rem) else "tile_bf16_ans"
+    device = weight.rem.device
+    stream = _stream(weight.rem)
+    with torch.cuda.device(device):
+        need = int(lib.bhi_tile_workspace_bytes(split_k, M, Ks, rows))
+        if need < 0:
+            _lib.check(need, name)
+        ws = workspace("tile", device, stream, need, TILE_COUNTER_BYTES) if need else None
+        rc = getattr(lib, "bhi_" + name)(member, x_ptr, split_k, Ks, rows, None if ws is None else ws.data_ptr(), need, stream)
+        if rc != 0 and ws is not None:
+            ws[:TILE_COUNTER_BYTES].zero_()
+    _lib.check(rc, name)
+
+
 def gemm_bf16_grouped(weights, X: Tensor, Ys, biases=None, residuals=None) -> None:
     """:func:`gemm_bf16` for up to four weights of one class (Huffman or rANS) and one ``split_k`` / ``Ks``
     that multiply the same ``X``: one grid when their rows together are enough for the kernel to

@@ -210,6 +210,17 @@ int bhi_gemm_bf16_ans_grouped(const bhi_gemv_member* members, int n_members, con
 /* Workspace bytes a call with these dimensions needs (0: none); negative on a rejected shape. */
 int64_t bhi_gemm_workspace_bytes(int split_k, int M, int Ks, int batch);
 
+/* The product for 17..128 rows of X (no counterpart in the reference, which decodes to a BF16 matrix
+ * and calls a dense GEMM): one weight as above, workspace under the same rules, its size from
+ * bhi_tile_workspace_bytes (1 KiB of counters, then partial sums).  Above 32 rows a bias is added
+ * before the product is rounded to BF16 (a dense GEMM's rounding), up to 32 after.  X must be 16-byte
+ * aligned for full speed. */
+int bhi_tile_bf16_huffman(const bhi_gemv_member* weight, const void* X, int split_k, int Ks, int batch,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+int bhi_tile_bf16_ans(const bhi_gemv_member* weight, const void* X, int split_k, int Ks, int batch,
+                      void* workspace, int64_t workspace_bytes, void* stream);
+int64_t bhi_tile_workspace_bytes(int split_k, int M, int Ks, int batch);
+
 /* bhi_gemm_bf16_huffman without a workspace argument -- no counterpart in the reference.  For
  * callers that cannot allocate device memory at all (code under stream capture that has no
  * workspace yet, serving loops and harnesses that forbid it): the partial sums and counters
