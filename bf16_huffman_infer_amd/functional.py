@@ -76,8 +76,8 @@ def _check_weight_call(A_rem: Tensor, A_exp: Tensor, X: Tensor):
     assert N % 128 == 0
     assert X.dim() == 3 and X.size(-1) == N
     assert X.dtype == torch.bfloat16
-    assert A_rem.device.type == A_exp.device.type == X.device.type == 'cuda'
-    assert A_rem.device == A_exp.device == X.device
+    assert A_rem.is_cuda and A_exp.is_cuda and X.is_cuda
+    assert A_rem.get_device() == A_exp.get_device() == X.get_device()
 
 
 def mv_huffman(
@@ -777,7 +777,7 @@ def _tiled(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool
     rows = input.size(0)
     if not _ops.TILE_MIN_ROWS <= rows <= _ops.TILE_MAX_ROWS or isinstance(weight, NibbleWeight):
         return False
-    split_k, M, N = weight.rem.shape
+    split_k, M, N = _ops._buffer(weight, 'rem').shape
     if input.dtype != torch.bfloat16 or (bias is not None and bias.dtype != torch.bfloat16) or not input.is_cuda:
         return False
     if input.size(1) != split_k * N or input.numel() >= 2 ** 31 or not prefers_tiles(rows, M, split_k * N):
@@ -788,49 +788,58 @@ def _tiled(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool
 def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], fused) -> Tensor:
     assert input.dim() >= 2, input
     shape = input.shape
-    input = input.flatten(0, -2)
-    if input.size(0) == 0:                       # no rows: nothing to launch
-        return input.new_empty((*shape[:-1], weight.rem.shape[1]))
-    split_k, M, N = weight.rem.shape
-    wide = (input.size(0) <= MAX_FUSED_BATCH and not isinstance(weight, NibbleWeight) and input.dtype == torch.bfloat16
-            and (bias is None or bias.dtype == torch.bfloat16) and prefers_matrix_cores(input.size(0), M, split_k * N))
-    if input.size(0) <= MAX_FUSED_BATCH and not wide:
+    if len(shape) > 2:
+        input = input.flatten(0, -2)
+    rows = input.size(0)
+    split_k, M, N = _ops._buffer(weight, 'rem').shape
+    if rows == 0:                       # no rows: nothing to launch
+        return input.new_empty((*shape[:-1], M))
+    matrix_cores = (not isinstance(weight, NibbleWeight) and input.dtype == torch.bfloat16
+                    and (bias is None or bias.dtype == torch.bfloat16))
+    wide = rows <= MAX_FUSED_BATCH and matrix_cores and prefers_matrix_cores(rows, M, split_k * N)
+    if rows <= MAX_FUSED_BATCH and not wide:
         if bias is not None and bias.dtype == torch.bfloat16:
             # the grouped entry point adds the bias in the kernel's last store (same bits, one launch less)
-            return linear_grouped(input, [weight], [bias])[0].unflatten(0, shape[:-1])
-        output = fused(input)
-        if bias is not None:
-            output += bias[None, :]
-    elif _tiled(input, weight, bias):
+            x = input.view(-1, split_k, N)
+            _check_weight_call(weight.rem, weight.exp, x)
+            output = torch.empty((rows, M), dtype=torch.bfloat16, device=x.device)
+            gemv_bf16_grouped([weight], x.contiguous(), [output], [bias.detach().contiguous()])
+        else:
+            output = fused(input)
+            if bias is not None:
+                output += bias[None, :]
+    elif matrix_cores and rows > MAX_FUSED_BATCH and _tiled(input, weight, bias):
         # 17..128 rows where the rule says so: as below, sixteen weight rows at a time
-        x = (input if input.size(0) <= GEMM_MAX_ROWS else input.contiguous()).view(-1, split_k, N).contiguous()
+        x = (input if rows <= GEMM_MAX_ROWS else input.contiguous()).view(-1, split_k, N).contiguous()
         if x.data_ptr() % 16:
             x = x.clone()
         _check_weight_call(weight.rem, weight.exp, x)
-        output = torch.empty((x.size(0), M), dtype=torch.bfloat16, device=x.device)
+        output = torch.empty((rows, M), dtype=torch.bfloat16, device=x.device)
         _ops.tile_bf16(weight, x, output, None if bias is None else bias.detach().contiguous())
-    elif wide or (input.size(0) <= GEMM_MAX_ROWS and not isinstance(weight, NibbleWeight) and input.dtype == torch.bfloat16
-                  and (bias is None or bias.dtype == torch.bfloat16)):
+    elif wide or (rows <= GEMM_MAX_ROWS and matrix_cores):
         # 9..32 rows (and fewer where the rule above says so): decode inside the matrix-core kernel,
         # no BF16 weight in memory
         x = input.view(-1, split_k, N)
         _check_weight_call(weight.rem, weight.exp, x)
-        output = torch.empty((x.size(0), M), dtype=torch.bfloat16, device=x.device)
+        output = torch.empty((rows, M), dtype=torch.bfloat16, device=x.device)
         gemm_bf16(weight, x.contiguous(), output, None if bias is None else bias.detach().contiguous())
     else:
         output = F.linear(input, weight.get_weight(), bias)
-    return output.unflatten(0, shape[:-1])
+    return output if len(shape) == 2 else output.unflatten(0, shape[:-1])
 
 
 def linear_huffman(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor] = None) -> Tensor:
     """``F.linear`` with a :class:`HuffmanWeight`: fused kernels up to 32 rows and, where they are faster,
     up to 128, else decode + dense GEMM (reference ``functional.py:390-411``)."""
-    return _linear_compressed(input, weight, bias, lambda x: mv_huffman(
-        weight.rem, weight.exp, x, weight.offsets,
-        weight.LUT1, weight.LUT2, weight.LUT3, weight.LUT4, weight.code_lengths))
+    def fused(x):
+        b = weight._buffers
+        return mv_huffman(b['rem'], b['exp'], x, b['offsets'], b['LUT1'], b['LUT2'], b['LUT3'], b['LUT4'], b['code_lengths'])
+    return _linear_compressed(input, weight, bias, fused)
 
 
 def linear_ans(input: Tensor, weight: ANSWeight, bias: Optional[Tensor] = None) -> Tensor:
     """rANS counterpart of :func:`linear_huffman` (reference ``functional.py:447-466``)."""
-    return _linear_compressed(input, weight, bias, lambda x: mv_ans(
-        weight.rem, weight.exp, x, weight.offsets, weight.LUT))
+    def fused(x):
+        b = weight._buffers
+        return mv_ans(b['rem'], b['exp'], x, b['offsets'], b['LUT'])
+    return _linear_compressed(input, weight, bias, fused)

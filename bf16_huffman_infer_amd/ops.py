@@ -11,6 +11,8 @@ reference rejects them with asserts.
 Every op mutates caller-allocated outputs and returns nothing; nothing here
 synchronises or allocates, so the ops can be captured in a HIP graph.
 """
+import contextlib
+
 import torch
 from torch import Tensor
 
@@ -42,13 +44,21 @@ def _stream(t: Tensor) -> int:
     """The current torch stream of ``t``'s device.  The first op on a device also lets the
     library do its once-per-device lookups: whatever comes first in a process is an eager call
     (a conversion, a warm-up), so none of them is left for a call under stream capture."""
-    device = t.device
-    if device not in _ready_devices:
+    index = t.get_device()
+    if index not in _ready_devices:
         if not torch.cuda.is_current_stream_capturing():
-            with torch.cuda.device(device):
+            with torch.cuda.device(index):
                 _lib.check(_lib.load().bhi_device_init(), "device_init")
-            _ready_devices.add(device)
-    return torch.cuda.current_stream(device).cuda_stream
+            _ready_devices.add(index)
+    return torch._C._cuda_getCurrentRawStream(index)
+
+
+_here = contextlib.nullcontext()
+
+
+def _on_device(index: int):
+    """Makes device ``index`` current for a ``with`` block; nothing to do where it already is."""
+    return _here if torch._C._cuda_getDevice() == index else torch.cuda.device(index)
 
 
 def _req(t: Tensor, dtype, name: str, ref: Tensor = None) -> int:
@@ -56,9 +66,16 @@ def _req(t: Tensor, dtype, name: str, ref: Tensor = None) -> int:
         raise RuntimeError(f"{name}: expected {dtype}, got {t.dtype}")
     if not t.is_contiguous():
         raise RuntimeError(f"{name}: must be contiguous")
-    if ref is not None and t.device != ref.device:
+    if ref is not None and t.get_device() != ref.get_device():
         raise RuntimeError(f"{name}: on {t.device}, expected {ref.device}")
     return t.data_ptr()
+
+
+def _buffer(w, name: str) -> Tensor:
+    """``w.name`` of a weight module, without the walk through ``nn.Module.__getattr__``."""
+    found = w.__dict__.get("_buffers")
+    t = None if found is None else found.get(name)
+    return getattr(w, name) if t is None else t
 
 
 def _weight_dims(A_rem: Tensor, offsets: Tensor):
@@ -83,7 +100,7 @@ def _gemv_common(A_rem, A_exp, X, Y, offsets):
 def _gemv_bf16_huffman(A_rem, A_exp, X, Y, offsets, LUT1, LUT2, LUT3, LUT4, code_lengths):
     lib = _lib.load()
     split_k, M, Ks, batch = _gemv_common(A_rem, A_exp, X, Y, offsets)
-    with torch.cuda.device(A_rem.device):
+    with _on_device(A_rem.get_device()):
         rc = lib.bhi_gemv_bf16_huffman(
             _req(A_rem, torch.uint8, "A_rem"), _req(A_exp, torch.int32, "A_exp", A_rem), A_exp.numel(),
             _req(X, torch.bfloat16, "X", A_rem), _req(Y, torch.bfloat16, "Y", A_rem),
@@ -100,7 +117,7 @@ def _huffman_decode(A_rem, A_exp, Y, offsets, LUT1, LUT2, LUT3, LUT4, code_lengt
     split_k, M, Ks = _weight_dims(A_rem, offsets)
     if tuple(Y.shape) != (M, split_k * Ks):
         raise RuntimeError(f"Y must be [{M}, {split_k * Ks}], got {tuple(Y.shape)}")
-    with torch.cuda.device(A_rem.device):
+    with _on_device(A_rem.get_device()):
         rc = lib.bhi_huffman_decode(
             _req(A_rem, torch.uint8, "A_rem"), _req(A_exp, torch.int32, "A_exp", A_rem), A_exp.numel(),
             _req(Y, torch.bfloat16, "Y", A_rem), _req(offsets, torch.int32, "offsets", A_rem),
@@ -125,7 +142,7 @@ def _huffman_encode(data, LUT, output, output_lengths):
     n_tasks, n_steps = _encode_dims(data, output, output_lengths)
     if LUT.numel() != 65537:
         raise RuntimeError("LUT must hold 65537 encoder entries")
-    with torch.cuda.device(data.device):
+    with _on_device(data.get_device()):
         rc = lib.bhi_huffman_encode(
             _req(data, torch.uint8, "data"), _req(LUT, torch.int32, "LUT", data),
             _req(output, torch.int32, "output", data), _req(output_lengths, torch.int32, "output_lengths", data),
@@ -138,7 +155,7 @@ def _gemv_bf16_ans(A_rem, A_exp, X, Y, offsets, LUT):
     split_k, M, Ks, batch = _gemv_common(A_rem, A_exp, X, Y, offsets)
     if LUT.numel() != 256:
         raise RuntimeError("LUT must hold 256 rANS slots")
-    with torch.cuda.device(A_rem.device):
+    with _on_device(A_rem.get_device()):
         rc = lib.bhi_gemv_bf16_ans(
             _req(A_rem, torch.uint8, "A_rem"), _req(A_exp, torch.int32, "A_exp", A_rem), A_exp.numel(),
             _req(X, torch.bfloat16, "X", A_rem), _req(Y, torch.bfloat16, "Y", A_rem),
@@ -154,7 +171,7 @@ def _ans_decode(A_rem, A_exp, Y, offsets, LUT):
         raise RuntimeError(f"Y must be [{M}, {split_k * Ks}], got {tuple(Y.shape)}")
     if LUT.numel() != 256:
         raise RuntimeError("LUT must hold 256 rANS slots")
-    with torch.cuda.device(A_rem.device):
+    with _on_device(A_rem.get_device()):
         rc = lib.bhi_ans_decode(
             _req(A_rem, torch.uint8, "A_rem"), _req(A_exp, torch.int32, "A_exp", A_rem), A_exp.numel(),
             _req(Y, torch.bfloat16, "Y", A_rem), _req(offsets, torch.int32, "offsets", A_rem),
@@ -167,7 +184,7 @@ def _ans_encode(data, freq, cum, output, output_lengths):
     n_tasks, n_steps = _encode_dims(data, output, output_lengths)
     if freq.numel() != 256 or cum.numel() != 256:
         raise RuntimeError("freq and cum must hold 256 entries")
-    with torch.cuda.device(data.device):
+    with _on_device(data.get_device()):
         rc = lib.bhi_ans_encode(
             _req(data, torch.uint8, "data"), _req(freq, torch.int32, "freq", data), _req(cum, torch.int32, "cum", data),
             _req(output, torch.int32, "output", data), _req(output_lengths, torch.int32, "output_lengths", data),
@@ -180,7 +197,7 @@ def _gemv_bf16_nibble(A_rem, A_exp, X, Y, offsets, LUT):
     split_k, M, Ks, batch = _gemv_common(A_rem, A_exp, X, Y, offsets)
     if LUT.numel() != 256:
         raise RuntimeError("LUT must hold 256 entries")
-    with torch.cuda.device(A_rem.device):
+    with _on_device(A_rem.get_device()):
         rc = lib.bhi_gemv_bf16_nibble(
             _req(A_rem, torch.uint8, "A_rem"), _req(A_exp, torch.int32, "A_exp", A_rem), A_exp.numel(),
             _req(X, torch.bfloat16, "X", A_rem), _req(Y, torch.bfloat16, "Y", A_rem),
@@ -196,7 +213,7 @@ def _nibble_decode(A_rem, A_exp, Y, offsets, LUT):
         raise RuntimeError(f"Y must be [{M}, {split_k * Ks}], got {tuple(Y.shape)}")
     if LUT.numel() != 256:
         raise RuntimeError("LUT must hold 256 entries")
-    with torch.cuda.device(A_rem.device):
+    with _on_device(A_rem.get_device()):
         rc = lib.bhi_nibble_decode(
             _req(A_rem, torch.uint8, "A_rem"), _req(A_exp, torch.int32, "A_exp", A_rem), A_exp.numel(),
             _req(Y, torch.bfloat16, "Y", A_rem), _req(offsets, torch.int32, "offsets", A_rem),
@@ -209,7 +226,7 @@ def _nibble_encode(data, LUT, output, output_lengths):
     n_tasks, n_steps = _encode_dims(data, output, output_lengths)
     if LUT.numel() != 256:
         raise RuntimeError("LUT must hold 256 entries")
-    with torch.cuda.device(data.device):
+    with _on_device(data.get_device()):
         rc = lib.bhi_nibble_encode(
             _req(data, torch.uint8, "data"), _req(LUT, torch.int32, "LUT", data),
             _req(output, torch.int32, "output", data), _req(output_lengths, torch.int32, "output_lengths", data),
@@ -308,17 +325,17 @@ def gemv_bf16_grouped(weights, X: Tensor, Ys, biases=None, residuals=None, x_mod
     if not 1 <= len(weights) <= 4 or len(weights) != len(Ys):
         raise RuntimeError("a group has 1 to 4 weights and one output per weight")
     first = weights[0]
-    huffman = hasattr(first, "LUT1")
-    if huffman:
+    rem = _buffer(first, "rem")
+    if "LUT1" in first.__dict__.get("_buffers", ()) or hasattr(first, "LUT1"):
         entry = "gemv_bf16_huffman_grouped"
     elif int(getattr(first, "MAGIC", 0)) != 0:
         entry = "gemv_bf16_nibble_grouped"
     else:
         entry = "gemv_bf16_ans_grouped"
-    split_k, _, Ks = _weight_dims(first.rem, first.offsets)
+    split_k, _, Ks = _weight_dims(rem, _buffer(first, "offsets"))
     if X.dim() != 3 or X.shape[1] != split_k or X.shape[2] != Ks:
         raise RuntimeError(f"X must be [batch, {split_k}, {Ks}], got {tuple(X.shape)}")
-    x_ptr = _req(X, torch.bfloat16, "X", first.rem)
+    x_ptr = _req(X, torch.bfloat16, "X", rem)
     batch = X.shape[0]
     members = (_lib.GemvMember * len(weights))()
     if biases is None:
@@ -328,20 +345,20 @@ def gemv_bf16_grouped(weights, X: Tensor, Ys, biases=None, residuals=None, x_mod
     for m, w, Y, b, r in zip(members, weights, Ys, biases, residuals):
         if type(w) is not type(first):
             raise RuntimeError("the weights of a group must use one codec")
-        sk, M, ks = _weight_dims(w.rem, w.offsets)
+        sk, M, ks = _weight_dims(_buffer(w, "rem"), _buffer(w, "offsets"))
         if (sk, ks) != (split_k, Ks):
             raise RuntimeError("the weights of a group must share split_k and Ks")
         if tuple(Y.shape) != (batch, M):
             raise RuntimeError(f"Y must be [{batch}, {M}], got {tuple(Y.shape)}")
-        _fill_member(m, w, Y, b, first.rem)
+        _fill_member(m, w, Y, b, rem)
         if r is not None:
             if tuple(r.shape) != (batch, M):
                 raise RuntimeError(f"residual must be [{batch}, {M}], got {tuple(r.shape)}")
-            m.residual = _req(r, torch.bfloat16, "residual", first.rem)
+            m.residual = _req(r, torch.bfloat16, "residual", rem)
     lib = _lib.load()
-    with torch.cuda.device(first.rem.device):
+    with _on_device(rem.get_device()):
         if x_mode == X_PLAIN:
-            rc = getattr(lib, "bhi_" + entry)(members, len(weights), x_ptr, split_k, Ks, batch, _stream(first.rem))
+            rc = getattr(lib, "bhi_" + entry)(members, len(weights), x_ptr, split_k, Ks, batch, _stream(rem))
         else:
             if entry == "gemv_bf16_nibble_grouped":
                 raise RuntimeError("the nibble codec's kernels take X as it is")
@@ -350,7 +367,7 @@ def gemv_bf16_grouped(weights, X: Tensor, Ys, biases=None, residuals=None, x_mod
                 raise RuntimeError(f"x_aux must hold {want} values")
             entry += "_x"
             rc = getattr(lib, "bhi_" + entry)(members, len(weights), x_ptr, split_k, Ks, batch, int(x_mode),
-                                              _req(x_aux, torch.bfloat16, "x_aux", first.rem), float(eps), _stream(first.rem))
+                                              _req(x_aux, torch.bfloat16, "x_aux", rem), float(eps), _stream(rem))
     _lib.check(rc, entry)
 
 
@@ -433,20 +450,23 @@ def decode_attention(qk: Tensor, v: Tensor, norm_weight, cos: Tensor, sin: Tenso
 
 def _fill_member(m, w, Y: Tensor, bias, ref: Tensor) -> bool:
     """Fills one ``bhi_gemv_member`` from a weight module; returns whether it is a Huffman weight."""
-    huffman = hasattr(w, "LUT1")
-    _, M, _ = _weight_dims(w.rem, w.offsets)
-    m.A_rem = _req(w.rem, torch.uint8, "A_rem", ref)
-    m.A_exp = _req(w.exp, torch.int32, "A_exp", ref)
-    m.exp_words = w.exp.numel()
+    rem, exp, offsets = _buffer(w, "rem"), _buffer(w, "exp"), _buffer(w, "offsets")
+    huffman = "LUT1" in w.__dict__.get("_buffers", ()) or hasattr(w, "LUT1")
+    _, M, _ = _weight_dims(rem, offsets)
+    m.A_rem = _req(rem, torch.uint8, "A_rem", ref)
+    m.A_exp = _req(exp, torch.int32, "A_exp", ref)
+    m.exp_words = exp.numel()
     m.Y = _req(Y, torch.bfloat16, "Y", ref)
-    m.offsets = _req(w.offsets, torch.int32, "offsets", ref)
+    m.offsets = _req(offsets, torch.int32, "offsets", ref)
     if huffman:
-        m.table = _req(w.LUT1, torch.uint8, "LUT1", ref)
-        m.table_bytes = w.LUT1.numel()
-        m.header = _req(w.code_lengths, torch.uint8, "code_lengths", ref)
+        table = _buffer(w, "LUT1")
+        m.table = _req(table, torch.uint8, "LUT1", ref)
+        m.table_bytes = table.numel()
+        m.header = _req(_buffer(w, "code_lengths"), torch.uint8, "code_lengths", ref)
     else:
-        m.table = _req(w.LUT, torch.int32, "LUT", ref)
-        m.table_bytes = w.LUT.numel() * 4
+        table = _buffer(w, "LUT")
+        m.table = _req(table, torch.int32, "LUT", ref)
+        m.table_bytes = table.numel() * 4
         m.header = None
     m.M = M
     if bias is not None:
@@ -490,23 +510,24 @@ def gemm_bf16(weight, X: Tensor, Y: Tensor, bias=None, static_workspace: bool = 
     weights) allocates nothing and uses the array built into the library instead: ONE array per
     GPU, so launches that take it and may overlap on the GPU (different streams) race."""
     lib = _lib.load()
-    split_k, M, Ks = _weight_dims(weight.rem, weight.offsets)
+    rem = _buffer(weight, "rem")
+    split_k, M, Ks = _weight_dims(rem, _buffer(weight, "offsets"))
     if X.dim() != 3 or X.shape[1] != split_k or X.shape[2] != Ks:
         raise RuntimeError(f"X must be [rows, {split_k}, {Ks}], got {tuple(X.shape)}")
     rows = X.shape[0]
     if tuple(Y.shape) != (rows, M):
         raise RuntimeError(f"Y must be [{rows}, {M}], got {tuple(Y.shape)}")
     member = (_lib.GemvMember * 1)()
-    x_ptr = _req(X, torch.bfloat16, "X", weight.rem)
-    huffman = _fill_member(member[0], weight, Y, bias, weight.rem)
+    x_ptr = _req(X, torch.bfloat16, "X", rem)
+    huffman = _fill_member(member[0], weight, Y, bias, rem)
     if residual is not None:
         if tuple(residual.shape) != (rows, M):
             raise RuntimeError(f"residual must be [{rows}, {M}], got {tuple(residual.shape)}")
-        member[0].residual = _req(residual, torch.bfloat16, "residual", weight.rem)
+        member[0].residual = _req(residual, torch.bfloat16, "residual", rem)
     name = "gemm_bf16_huffman" if huffman else "gemm_bf16_ans"
-    device = weight.rem.device
-    stream = _stream(weight.rem)
-    with torch.cuda.device(device):
+    device = rem.device
+    stream = _stream(rem)
+    with _on_device(rem.get_device()):
         need = int(lib.bhi_gemm_workspace_bytes(split_k, M, Ks, rows))
         if need < 0:
             _lib.check(need, name)
@@ -516,7 +537,7 @@ def gemm_bf16(weight, X: Tensor, Y: Tensor, bias=None, static_workspace: bool = 
         elif static_workspace:
             if not huffman:
                 raise RuntimeError("gemm_bf16: the built-in workspace serves Huffman weights only")
-            if device not in _ready_devices:
+            if device.index not in _ready_devices:
                 raise RuntimeError("gemm_bf16: the library has not been used on this device outside a stream capture yet")
             rc = lib.bhi_gemm_bf16_huffman_static(member, x_ptr, split_k, Ks, rows, stream)
         else:
@@ -538,18 +559,19 @@ def tile_bf16(weight, X: Tensor, Y: Tensor, bias=None) -> None:
     time.  Arguments as :func:`gemm_bf16`; partial sums of K slices meet in a workspace of the
     (device, stream) or of the capture (:mod:`.workspace`)."""
     lib = _lib.load()
-    split_k, M, Ks = _weight_dims(weight.rem, weight.offsets)
+    rem = _buffer(weight, "rem")
+    split_k, M, Ks = _weight_dims(rem, _buffer(weight, "offsets"))
     if X.dim() != 3 or X.shape[1] != split_k or X.shape[2] != Ks:
         raise RuntimeError(f"X must be [rows, {split_k}, {Ks}], got {tuple(X.shape)}")
     rows = X.shape[0]
     if tuple(Y.shape) != (rows, M):
         raise RuntimeError(f"Y must be [{rows}, {M}], got {tuple(Y.shape)}")
     member = (_lib.GemvMember * 1)()
-    x_ptr = _req(X, torch.bfloat16, "X", weight.rem)
-    name = "tile_bf16_huffman" if _fill_member(member[0], weight, Y, bias, weight.rem) else "tile_bf16_ans"
-    device = weight.rem.device
-    stream = _stream(weight.rem)
-    with torch.cuda.device(device):
+    x_ptr = _req(X, torch.bfloat16, "X", rem)
+    name = "tile_bf16_huffman" if _fill_member(member[0], weight, Y, bias, rem) else "tile_bf16_ans"
+    device = rem.device
+    stream = _stream(rem)
+    with _on_device(rem.get_device()):
         need = int(lib.bhi_tile_workspace_bytes(split_k, M, Ks, rows))
         if need < 0:
             _lib.check(need, name)
