@@ -50,13 +50,20 @@ __all__ = [
 ]
 
 
-def _lane_order(plane: Tensor, split_k: int) -> Tensor:
-    """[M, K] byte plane -> [split_k, G, S, 64, 8]: (split, row group, step, lane, column)."""
-    M, K = plane.shape
-    Ks = K // split_k
-    G, S = M // GROUP_ROWS, Ks // STEP_COLS
-    x = plane.view(G, GROUP_ROWS, split_k, S, STEP_COLS // LANE_COLS, LANE_COLS)     # g i k t b j
-    return x.permute(2, 0, 3, 4, 1, 5).reshape(split_k, G, S, LANES, LANE_COLS)
+def _single_counts(pairs: Tensor) -> Tensor:
+    """int64 ``[256]`` occurrences of every exponent from those of the pairs."""
+    pairs = pairs.view(256, 256)                 # [second, first]
+    return pairs.sum(0) + pairs.sum(1)
+
+
+def _to_host(t: Tensor) -> Tensor:
+    """``t`` in host memory.  Copying into memory that was never touched runs at the pace of its page faults,
+    taken one by one (50 MB: 11.6 ms); a fill takes them on all threads first."""
+    if not t.is_cuda:
+        return t.cpu()
+    host = torch.empty(t.shape, dtype=t.dtype)
+    host.zero_()
+    return host.copy_(t)
 
 
 def _promote_single_split(A_rem: Tensor, offsets: Tensor):
@@ -160,36 +167,21 @@ class HuffmanWeight(nn.Module):
     @classmethod
     def get_codec(cls, a: Tensor) -> LUTHuffmanEncoder:
         """One code per weight matrix, built from the histogram of exponent pairs."""
-        device = torch.device('cuda', 0)
-        _, exp = split_bf16(a.detach().to(device))
-        counts = cls._pair_counts(exp)
+        _, exp = split_bf16(a.detach().to(torch.device('cuda', 0)))
+        return cls._codec_of(cls._pair_counts(exp))
+
+    @classmethod
+    def _codec_of(cls, counts: Tensor) -> LUTHuffmanEncoder:
+        """The code for int64 ``[65536]`` pair counts."""
         codec = LUTHuffmanEncoder()
         codec.build_lut(counts.cpu())
         return codec
 
     @staticmethod
     def _pair_counts(exp: Tensor) -> Tensor:
-        """int64 [65536]: occurrences of every exponent pair ``a | b << 8`` (a = even column).
-
-        A histogram over 65536 bins runs on global atomics (25 ms for a 4096x12288 layer); real
-        weights use a few dozen exponent values, so the pairs are counted over the ranks of
-        the values that occur (at most 64 x 64 bins, which the histogram kernel keeps in
-        shared memory) and scattered back."""
-        single = torch.bincount(exp.flatten().to(torch.int32), minlength=256)
-        present = torch.nonzero(single).flatten()                      # exponent values that occur, ascending
-        a, b = exp[:, 0::2], exp[:, 1::2]
-        if present.numel() > 64:
-            pairs = a.to(torch.int32) | (b.to(torch.int32) << 8)
-            return torch.bincount(pairs.flatten(), minlength=65536)
-        rank = torch.zeros(256, dtype=torch.int32, device=exp.device)
-        rank[present] = torch.arange(present.numel(), dtype=torch.int32, device=exp.device)
-        dense = rank[a.to(torch.int64)] | (rank[b.to(torch.int64)] << 6)
-        small = torch.bincount(dense.flatten(), minlength=4096)        # [rank_b * 64 + rank_a]
-        counts = torch.zeros(65536, dtype=torch.int64, device=exp.device)
-        ra, rb = torch.meshgrid(torch.arange(present.numel(), device=exp.device),
-                                torch.arange(present.numel(), device=exp.device), indexing='ij')
-        counts[(present[ra] | (present[rb] << 8)).flatten()] = small[(ra | (rb << 6)).flatten()]
-        return counts
+        """int64 [65536]: occurrences of every exponent pair ``a | b << 8`` (a = even column) of ``[M, K]``
+        exponents, K a multiple of eight."""
+        return _ops.pair_histogram(exp.contiguous())
 
     @classmethod
     def get_lut_kwargs(cls, codec: LUTHuffmanEncoder) -> dict[str, Tensor]:
@@ -222,7 +214,11 @@ class HuffmanWeight(nn.Module):
         """Compress ``a`` with ``n`` column splits (the reference's ``compress_split_n``,
         ``functional.py:195-238``)."""
         assert a.dim() == 2 and a.dtype == torch.bfloat16
-        a = a.detach()
+        return cls(**{name: _to_host(t) for name, t in cls._compress_on_device(a, n).items()})
+
+    @classmethod
+    def _compress_on_device(cls, a: Tensor, n: int) -> dict[str, Tensor]:
+        """The buffers of the compressed ``a``, on the GPU."""
         M, K = a.shape
         assert M % 128 == 0 and K % n == 0 and (K // n) % STEP_COLS == 0, a.shape
         Ks = K // n
@@ -232,22 +228,22 @@ class HuffmanWeight(nn.Module):
         consts = _lib.constants()
         nc = lib.bhi_chunks_per_group(M, Ks, n)
 
-        codec = cls.get_codec(a)
-        rem, exp = split_bf16(a.to(device))
-        rem = _lane_order(rem, n).reshape(n, M, Ks).contiguous()
-        sym = _lane_order(exp, n)                                           # [n, G, S, 64, 8]
-        del exp
+        rem, sym = _ops.split_planes(a.detach().to(device).contiguous(), n)
+        codec = cls._codec_of(_ops.pair_histogram(sym))
 
         lengths = torch.zeros(n, G, nc, dtype=torch.int64, device=device)
         pieces = []                                                          # (chunk, first task, streams, lengths)
+        done = 0
         for c in range(nc):
             t0, t1 = (S * c) // nc, (S * (c + 1)) // nc
-            tasks = sym[:, :, t0:t1].reshape(n * G, (t1 - t0) * LANES * LANE_COLS)
+            size = (t1 - t0) * LANES * LANE_COLS
+            tasks = sym[done:done + n * G * size].view(n * G, size)
+            done += tasks.numel()
             per_call = max(1, ENCODE_PART_BYTES // (4 * cls.capacity(t1 - t0)))
             for first in range(0, n * G, per_call):
-                out, ln = cls.compress_groups(tasks[first:first + per_call].contiguous(), codec)
+                out, ln = cls.compress_groups(tasks[first:first + per_call], codec)
                 used = int(ln.max().item())
-                pieces.append((c, first, out[:, :used].clone(), ln.to(torch.int64)))
+                pieces.append((c, first, out[:, :used].clone(), ln))
                 lengths.view(n * G, nc)[first:first + ln.numel(), c] = ln
         del sym
 
@@ -256,19 +252,10 @@ class HuffmanWeight(nn.Module):
         starts = (torch.cumsum(lengths.flatten(), 0) - lengths.flatten()).view(n * G, nc)
         words = torch.zeros(total + consts['tail_pad_words'], dtype=torch.int32, device=device)
         for c, first, out, ln in pieces:
-            cols = torch.arange(out.size(1), device=device)[None, :]
-            keep = cols < ln[:, None]
-            dest = (starts[first:first + ln.numel(), c][:, None] + cols)[keep]
-            words[dest] = out[keep]
+            _ops.place_streams(out, ln, starts[first:first + ln.numel(), c], words)
         offsets = torch.zeros(n, G, GROUP_ROWS, dtype=torch.int32, device=device)
         offsets[:, :, :nc] = starts.view(n, G, nc).to(torch.int32)
-
-        return cls(
-            rem=rem.cpu(),
-            exp=words.cpu(),
-            offsets=offsets.view(n, M).cpu(),
-            **cls.get_lut_kwargs(codec),
-        )
+        return dict(rem=rem, exp=words, offsets=offsets.view(n, M), **cls.get_lut_kwargs(codec))
 
     @classmethod
     def compress(cls, a: Tensor):
@@ -303,6 +290,10 @@ class ANSWeight(HuffmanWeight):
         _, exp = split_bf16(a.detach().to(device))
         counts = torch.bincount(exp.flatten().to(torch.int32), minlength=256)
         return RANSEncoder(counts.tolist(), precision=ANS_PRECISION)
+
+    @classmethod
+    def _codec_of(cls, counts: Tensor) -> RANSEncoder:
+        return RANSEncoder(_single_counts(counts).tolist(), precision=ANS_PRECISION)
 
     @classmethod
     def get_lut_kwargs(cls, codec: RANSEncoder) -> dict[str, Tensor]:
@@ -366,6 +357,10 @@ class NibbleWeight(ANSWeight):
         device = torch.device('cuda', 0)
         _, exp = split_bf16(a.detach().to(device))
         return NibbleCodec(torch.bincount(exp.flatten().to(torch.int32), minlength=256))
+
+    @classmethod
+    def _codec_of(cls, counts: Tensor) -> NibbleCodec:
+        return NibbleCodec(_single_counts(counts))
 
     @classmethod
     def get_lut_kwargs(cls, codec: NibbleCodec) -> dict[str, Tensor]:
@@ -570,29 +565,30 @@ def convert(linear: nn.Linear, name, disable_precision_check=True, algo='huffman
     random GEMV deviates by 2 % or more from the dense layer.
     """
     assert algo in ('huffman', 'ans', 'smallest', 'nibble')
-    if algo == 'huffman':
-        weight = HuffmanWeight.compress(linear.weight)
-    elif algo == 'ans':
-        weight = ANSWeight.compress(linear.weight)
-    elif algo == 'nibble':
-        weight = NibbleWeight.compress(linear.weight)
-    else:
-        weight = min([HuffmanWeight.compress(linear.weight), ANSWeight.compress(linear.weight)], key=_weight_bytes)
+    # The weight goes to the GPU once and the compressed buffers come back once; the layer itself stays
+    # where it is until the end.
+    weight = linear.weight
+    n = get_block_size_n(weight)[0]
+    assert weight.dim() == 2 and weight.dtype == torch.bfloat16
+    dense = weight.detach().to(torch.device('cuda', 0)).contiguous()
+    classes = {'huffman': [HuffmanWeight], 'ans': [ANSWeight], 'nibble': [NibbleWeight],
+               'smallest': [HuffmanWeight, ANSWeight]}[algo]
+    compressed = min([cls(**cls._compress_on_device(dense, n)) for cls in classes], key=_weight_bytes)
 
-    module = CompressedLinear(weight=weight, bias=linear.bias)
+    module = CompressedLinear(weight=compressed, bias=linear.bias)
     ori_size = linear.weight.nelement() * linear.weight.element_size()
     ratio = _weight_bytes(module.weight) / ori_size
 
-    linear.cuda()
-    module.cuda()
+    compressed.cuda()
+    dense = dense.cuda()
+    bias = None if linear.bias is None else linear.bias.detach().cuda()
     x = torch.randn(1, linear.in_features, dtype=torch.bfloat16, device='cuda')
     with torch.no_grad():
-        y1 = linear(x)
-        y2 = module(x)
-        lossless = torch.equal(module.weight.get_weight().view(torch.int16), linear.weight.view(torch.int16))
+        y1 = F.linear(x, dense, bias)
+        y2 = F.linear(x, compressed, bias)
+        lossless = torch.equal(compressed.get_weight().view(torch.int16), dense.view(torch.int16))
     max_rtol = ((y2 - y1).abs() / y1.abs().clamp(min=1e-4)).max().item()
     linear.cpu()
-    module.cpu()
 
     fallback = False
     if ratio >= 1:
@@ -607,6 +603,7 @@ def convert(linear: nn.Linear, name, disable_precision_check=True, algo='huffman
     if fallback:
         print('Fallback to regular nn.Linear')
         return linear
+    compressed._apply(_to_host)
     return module
 
 

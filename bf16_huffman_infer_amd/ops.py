@@ -280,6 +280,40 @@ def ans_decode(A_rem: Tensor, A_exp: Tensor, Y: Tensor, offsets: Tensor, LUT: Te
     torch.ops.bf16_huffman_infer.ans_decode.default(A_rem, A_exp, Y, offsets, LUT)
 
 
+def split_planes(w: Tensor, split_k: int):
+    """bf16 ``[M, K]`` -> (rem uint8 ``[split_k, M, K/split_k]`` as stored, exponents uint8 ``[M*K]`` in task
+    order: the tasks of chunk 0, then of chunk 1, ...)."""
+    M, K = w.shape
+    rem = torch.empty((split_k, M, K // split_k), dtype=torch.uint8, device=w.device)
+    exp = torch.empty(M * K, dtype=torch.uint8, device=w.device)
+    with _on_device(w.get_device()):
+        _lib.check(_lib.load().bhi_split_planes(_req(w, torch.bfloat16, "weight"), rem.data_ptr(), exp.data_ptr(), split_k, M,
+                                                K // split_k, _stream(w)), "split_planes")
+    return rem, exp
+
+
+def pair_histogram(exp: Tensor) -> Tensor:
+    """int64 ``[65536]``: occurrences of every pair ``a | b << 8`` of neighbouring bytes of ``exp`` (uint8, a
+    multiple of eight)."""
+    counts = torch.zeros(65536, dtype=torch.int64, device=exp.device)
+    with _on_device(exp.get_device()):
+        _lib.check(_lib.load().bhi_pair_histogram(_req(exp, torch.uint8, "exp"), exp.numel(), counts.data_ptr(), _stream(exp)),
+                   "pair_histogram")
+    return counts
+
+
+def place_streams(streams: Tensor, lengths: Tensor, starts: Tensor, words: Tensor) -> None:
+    """Copies the first ``lengths[i]`` words of row ``i`` of ``streams`` to ``words[starts[i]:]``; ``starts`` is
+    int64 ``[n]`` of any stride."""
+    if starts.dtype != torch.int64 or starts.dim() != 1 or starts.numel() != streams.shape[0]:
+        raise RuntimeError("starts must be one int64 per stream")
+    with _on_device(streams.get_device()):
+        _lib.check(_lib.load().bhi_place_streams(
+            _req(streams, torch.int32, "streams"), streams.shape[1], _req(lengths, torch.int32, "lengths", streams),
+            starts.data_ptr(), starts.stride(0), streams.shape[0], _req(words, torch.int32, "words", streams), words.numel(),
+            _stream(streams)), "place_streams")
+
+
 def encode_capacity(n_steps: int) -> int:
     """Words to reserve per task row of ``huffman_encode``'s output."""
     return int(_lib.load().bhi_encode_capacity(n_steps))

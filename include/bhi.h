@@ -243,6 +243,18 @@ int64_t bhi_gemm_static_workspace_bytes(void);
 int bhi_device_init(void);
 int bhi_gemm_workspace_reset(void* workspace, int64_t workspace_bytes, void* stream);
 
+/* The passes of a conversion around the encoders (the reference's are tensor operations,
+ * functional.py:195-238).  bhi_split_planes: bf16 W [M, split_k*Ks] -> rem uint8
+ * [split_k, M, Ks] as stored and exp uint8 [split_k*M*Ks]: the exponents of chunk 0's tasks, then chunk
+ * 1's, ... as the encoders take them.  bhi_pair_histogram: adds the occurrences of every pair of
+ * neighbouring bytes to counts int64 [65536] (index first | second << 8).  bhi_place_streams: copies the
+ * first lengths[i] (int32) words of row i of streams int32 [n_tasks, stride] to words + starts[i *
+ * starts_stride] (int64); a row that does not fit words int32 [n_words] is left out. */
+int bhi_split_planes(const void* W, void* rem, void* exp, int split_k, int M, int Ks, void* stream);
+int bhi_pair_histogram(const void* exp, int64_t bytes, void* counts, void* stream);
+int bhi_place_streams(const void* streams, int64_t stride, const void* lengths, const void* starts, int64_t starts_stride,
+                      int n_tasks, void* words, int64_t n_words, void* stream);
+
 /* Readers for weights that were compressed by the reference package itself: same tensors
  * as the reference's huffman_decode / ans_decode ops (kernel.cu:534-587, 878-919) IN THE
  * REFERENCE'S OWN LAYOUT (functional.py:129-242: 64 streams per row, LUT1..4 uint8 [256],

@@ -1,0 +1,48 @@
+"""The conversion passes around the encoders (needs a GPU) against tensor operations on the CPU."""
+import pytest
+import torch
+
+from helpers import gaussian_weight, random_bits_weight
+
+pytestmark = pytest.mark.gpu
+
+
+def _lane_order(plane, n):
+    """[M, K] bytes -> [split, group, step, lane, column]."""
+    M, K = plane.shape
+    x = plane.view(M // 4, 4, n, K // n // 128, 16, 8)
+    return x.permute(2, 0, 3, 4, 1, 5).reshape(n, M // 4, K // n // 128, 512)
+
+
+@pytest.mark.parametrize("make", [gaussian_weight, random_bits_weight])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("M,K,n", [(128, 128, 1), (128, 1152, 1), (256, 2176, 1), (128, 3456, 3), (640, 1024, 2), (28672, 384, 3)])
+def test_split_planes_and_histogram(cuda, make, offset, M, K, n):
+    """Whole weights and, one element on, weights that are aligned to two bytes only; one to four chunks of
+    steps that do not divide evenly; a workgroup that is not full."""
+    from bf16_huffman_infer_amd import _lib, ops
+    from bf16_huffman_infer_amd.utils import split_bf16
+    w = make(M, K, seed=M + K)
+    held = torch.empty(M * K + 1, dtype=torch.bfloat16, device="cuda")[offset:offset + M * K].view(M, K)
+    held.copy_(w)
+    rem, exp = ops.split_planes(held, n)
+    wrem, wexp = split_bf16(w)
+    assert torch.equal(rem.cpu().view(-1), _lane_order(wrem, n).reshape(-1))
+    order, S = _lane_order(wexp, n), K // n // 128
+    nc = _lib.load().bhi_chunks_per_group(M, K // n, n)
+    want = torch.cat([order[:, :, S * c // nc:S * (c + 1) // nc].reshape(-1) for c in range(nc)])
+    assert torch.equal(exp.cpu(), want)
+    pairs = wexp[:, 0::2].to(torch.int64) | wexp[:, 1::2].to(torch.int64) << 8
+    assert torch.equal(ops.pair_histogram(exp).cpu(), torch.bincount(pairs.flatten(), minlength=65536))
+
+
+@pytest.mark.parametrize("algo", ["huffman", "ans", "smallest", "nibble"])
+def test_convert_leaves_the_layer_alone_and_returns_host_buffers(cuda, algo):
+    from bf16_huffman_infer_amd.functional import convert
+    w = gaussian_weight(4096, 1024, seed=5)
+    linear = torch.nn.Linear(1024, 4096, dtype=torch.bfloat16)
+    linear.weight.data.copy_(w)
+    module = convert(linear, "layer", algo=algo)
+    assert torch.equal(linear.weight.data, w) and not linear.weight.is_cuda
+    assert all(not b.is_cuda for b in module.buffers()) and module.bias is linear.bias
+    assert torch.equal(module.cuda().weight.get_weight().cpu().view(torch.int16), w.view(torch.int16))
