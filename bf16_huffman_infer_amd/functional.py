@@ -814,7 +814,7 @@ def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tens
         output = torch.empty((rows, M), dtype=torch.bfloat16, device=x.device)
         _ops.tile_bf16(weight, x, output, None if bias is None else bias.detach().contiguous())
     elif wide or (rows <= GEMM_MAX_ROWS and matrix_cores):
-        # 9..32 rows (and fewer where the rule above says so): decode inside the matrix-core kernel,
+        # up to 32 rows that neither the GEMV nor the tiled product takes: decode inside the matrix-core kernel,
         # no BF16 weight in memory
         x = input.view(-1, split_k, N)
         _check_weight_call(weight.rem, weight.exp, x)

@@ -181,8 +181,8 @@ int bhi_gemv_bf16_ans_grouped_x(const bhi_gemv_member* members, int n_members, c
 int bhi_rms_norm(const void* X, const void* gamma, void* out, int rows, int K, float eps, void* stream);
 int bhi_silu_mul(const void* gate, const void* up, void* out, int64_t n, void* stream);
 
-/* Fused decode + matrix product for 1..32 rows of X (meant for 9..32; up to 8 the GEMV
- * entry points are faster): Y = X W^T (+ bias) with the weights going from the decoder's
+/* Fused decode + matrix product for 1..32 rows of X (meant for 9..16; up to 8 the GEMV
+ * entry points are faster, above 16 mostly bhi_tile_bf16_*): Y = X W^T (+ bias) with the weights going from the decoder's
  * registers straight into matrix-core instructions.  Replaces the reference's path above
  * eight rows, huffman_decode / ans_decode to a BF16 matrix followed by a dense GEMM
  * (functional.py:405-407, 460-462; kernel.cu:510-587, 851-919), which writes and re-reads

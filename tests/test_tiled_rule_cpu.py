@@ -1,0 +1,43 @@
+"""Where the tiled product may take the place of decoding and ``F.linear``, and the workspace it asks for."""
+import torch
+import torch.autograd.forward_ad as forward_ad
+
+
+def test_only_where_nothing_but_the_value_is_asked_for():
+    from bf16_huffman_infer_amd.functional import _fuses_above_32_rows as fuses
+    x, bias = torch.zeros(40, 128), torch.zeros(64)
+    assert fuses(x, None) and fuses(x, bias) and fuses(torch.nn.Parameter(x, requires_grad=False), bias)
+    wants = x.clone().requires_grad_()
+    assert not fuses(wants, None) and not fuses(x, bias.clone().requires_grad_())
+    with torch.no_grad():
+        assert fuses(wants, None)
+    with forward_ad.dual_level():
+        assert not fuses(x, None)
+    seen = []
+    torch.func.vmap(lambda v: (seen.append(fuses(x, None)), v)[1])(x)
+    assert seen == [False]
+    with torch.utils._python_dispatch.TorchDispatchMode():
+        assert not fuses(x, None)
+
+    class Sub(torch.Tensor):
+        pass
+    assert not fuses(x.as_subclass(Sub), None)
+
+
+def test_workspace_follows_the_slice_choice():
+    """Counters, then whole blocks of sixteen-row tiles per slice; nothing where K is not cut; never more
+    row blocks than there are counters."""
+    from bf16_huffman_infer_amd import _lib
+    lib = _lib.load()
+    for split_k, M, Ks in [(1, 128, 128), (1, 1024, 4096), (3, 4096, 4096), (4, 3584, 4736), (1, 18944, 3584), (1, 12288, 4096),
+                           (2, 65536, 2048), (1, 132, 512)]:
+        per_group = split_k * lib.bhi_chunks_per_group(M, Ks, split_k)
+        for rows in (17, 32, 33, 64, 65, 80, 81, 96, 97, 112, 128):
+            need = lib.bhi_tile_workspace_bytes(split_k, M, Ks, rows)
+            assert need >= 0
+            if need:
+                tiles = (rows + 15) // 16
+                choices = [(nw, d) for nw in (4, 6, 8) for d in range(2, 9) if per_group % d == 0
+                           and -(-M // (16 * nw)) <= 256 and 1024 + -(-M // (16 * nw)) * 16 * nw * tiles * 64 * d == need]
+                assert choices, (split_k, M, Ks, rows, need)
+        assert lib.bhi_tile_workspace_bytes(split_k, M, Ks, 16) < 0 and lib.bhi_tile_workspace_bytes(split_k, M, Ks, 129) < 0
