@@ -758,14 +758,14 @@ def prefers_tiles(rows: int, M: int, K: int) -> bool:
 
 
 def _fuses_above_32_rows(input: Tensor, bias: Optional[Tensor]) -> bool:
-    """Decoding and ``F.linear`` pass gradients, forward-mode tangents, function transforms, autocast and
-    dispatch modes on to the input (and the bias); a fused product does not, and takes over only where none
-    of them is in play."""
+    """Decoding and ``F.linear`` pass gradients, forward-mode tangents, function transforms, autocast, dispatch
+    modes and tracing on to the input (and the bias); a fused product does not, and takes over only where
+    none of them is in play."""
     if torch.is_grad_enabled() and (input.requires_grad or (bias is not None and bias.requires_grad)):
         return False
     if torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
         return False
-    if torch.is_autocast_enabled('cuda') or torch._C._len_torch_dispatch_stack():
+    if torch.is_autocast_enabled('cuda') or torch._C._len_torch_dispatch_stack() or torch.compiler.is_compiling():
         return False
     return type(input) in (Tensor, nn.Parameter)
 
