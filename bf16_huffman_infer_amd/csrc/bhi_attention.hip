@@ -190,9 +190,12 @@ __global__ __launch_bounds__(kAttnThreads, 2) void decode_attention_kernel(const
     const int w0 = first + wave * share, w1 = min(w0 + share, first + slots);
     const bool has_own = newest && w0 < w1 && w1 == n;           // the token's own slot is this wavefront's
 
-    const uint16_t* kc = a.k_cache + (size_t)kh * a.max_len * kAttnDim;
-    const uint16_t* vc = a.v_cache + (size_t)kh * a.max_len * kAttnDim;
     const uint16_t* v_own = a.v + (size_t)kh * kAttnDim;
+    // With nothing cached yet (n == 1) the token's own v row stands in for both: the only slot of
+    // the cache is then one that was never written and that another block may be writing.
+    const uint16_t* kc = n > 1 ? a.k_cache + (size_t)kh * a.max_len * kAttnDim : v_own;
+    const uint16_t* vc = n > 1 ? a.v_cache + (size_t)kh * a.max_len * kAttnDim : v_own;
+    const int cached = min(w1, n - 1);                           // end of this wavefront's slots whose rows are in the cache
     const int col = lane & 15, quarter = lane >> 4, half = lane >> 5;
 
     // this position's cosines and sines ahead of the rows: vector loads return in issue order
@@ -214,7 +217,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void decode_attention_kernel(const
         uint2 vr[NT][8];                                         // [tile][two slots]: 4 elements of one of them
         const int last = n > 1 ? n - 2 : 0;
         auto load = [&](int b0) __attribute__((always_inline)) {
-            // slots past the visible ones read a valid row whose weight will be 0
+            // slots past the visible ones read a valid row, whose score and values are dropped below
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 int j = b0 + t * kAttnTile + col;
@@ -222,7 +225,10 @@ __global__ __launch_bounds__(kAttnThreads, 2) void decode_attention_kernel(const
                 // 32-bit offsets from a uniform base: a head of the cache is at most 2 MiB
                 const char* row = (const char*)kc + (uint32_t)(j * (2 * kAttnDim) + quarter * 16);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) kr[t][c] = *(const uint4*)(row + 64 * c);
+                for (int c = 0; c < 4; ++c) {
+                    const row16_t r = *(const row16_t*)(row + 64 * c);
+                    kr[t][c] = make_uint4(r.x, r.y, r.z, r.w);
+                }
             }
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
@@ -305,7 +311,10 @@ __global__ __launch_bounds__(kAttnThreads, 2) void decode_attention_kernel(const
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const float* w = weights[wave][t * kAttnTile + 2 * i + half];
-                    const f32x4a_t v = {bf16_lo(vr[t][i].x), bf16_hi(vr[t][i].x), bf16_lo(vr[t][i].y), bf16_hi(vr[t][i].y)};
+                    // dropped by value: a weight of 0 would make NaN of an Inf or NaN in the row
+                    const bool in = b0 + t * kAttnTile + 2 * i + half < cached;
+                    const uint32_t lo = in ? vr[t][i].x : 0u, hi = in ? vr[t][i].y : 0u;
+                    const f32x4a_t v = {bf16_lo(lo), bf16_hi(lo), bf16_lo(hi), bf16_hi(hi)};
 #pragma unroll
                     for (int h = 0; h < GT; ++h) acc[h] += w[h] * v;
                 }
@@ -409,9 +418,11 @@ __global__ __launch_bounds__(kAttnThreads, 2) void decode_attention_kernel(const
             o *= f;
 #pragma unroll
             for (int i = 0; i < kAttnAhead; ++i) {
-                const float w = s0 + i < used ? rescale(ml[i].x, m) : 0.f;
-                l += w * ml[i].y;
-                o += w * x[i];
+                if (s0 + i < used) {                             // else the last split once more
+                    const float w = rescale(ml[i].x, m);
+                    l += w * ml[i].y;
+                    o += w * x[i];
+                }
             }
         }
         store_row8(a.out + (size_t)(h0 + h) * kAttnDim + d, o, 1.0f / l);

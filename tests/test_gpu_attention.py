@@ -186,3 +186,59 @@ def test_second_graph_does_not_depend_on_the_first(cuda, recorder):
         graphs[i].replay()
         assert torch.equal(outs[i], want), i
         assert torch.equal(ops.decode_attention(qk, v, None, cos, sin, pos, kc, vc), want)
+
+
+def _without_workspace(qk, v, cos, sin, pos, kc, vc, q_heads, kv_heads, out):
+    from bf16_huffman_infer_amd import _lib
+    _lib.check(_lib.load().bhi_decode_attention(
+        qk.data_ptr(), v.data_ptr(), None, cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+        out.data_ptr(), q_heads, kv_heads, 128, kc.shape[1], 1e-6, 128 ** -0.5, torch.cuda.current_stream().cuda_stream), "attention")
+
+
+@pytest.mark.parametrize("q_heads,kv_heads", [(8, 2), (31, 1), (3, 3)])
+@pytest.mark.parametrize("max_len,positions", [(1, (0,)), (64, (0, 1, 15, 63)), (1000, (0, 16, 130, 700)), (4096, (0, 4000))])
+@pytest.mark.parametrize("split", [True, False])
+def test_slots_from_the_position_on_are_not_read(cuda, q_heads, kv_heads, max_len, positions, split):
+    """A cache is allocated once and filled token by token: whatever lies in the slots from the token's
+    own on (here NaN, Inf) has no part in the result, which is that of a cache of zeros there, bit for bit."""
+    from bf16_huffman_infer_amd import ops
+    qk, v, kc, vc, cos, sin = _case(q_heads, kv_heads, max_len, 3 + max_len)
+    for p in positions:
+        pos = torch.tensor([p], device="cuda")
+        results = []
+        for filler in (0.0, float("nan"), float("inf")):
+            k, w = kc.clone(), vc.clone()
+            k[:, p:], w[:, p:] = filler, filler
+            out = torch.full((q_heads, 128), 7.0, dtype=torch.bfloat16, device="cuda")
+            if split:
+                ops.decode_attention(qk, v, None, cos, sin, pos, k, w, out=out)
+            else:
+                _without_workspace(qk, v, cos, sin, pos, k, w, q_heads, kv_heads, out)
+            assert torch.equal(w[:, p], v) and bool(k[:, p].isfinite().all())
+            results.append(out)
+        assert bool(results[0].isfinite().all())
+        assert torch.equal(results[1], results[0]) and torch.equal(results[2], results[0]), p
+
+
+@pytest.mark.parametrize("split", [True, False])
+def test_infinite_values_in_the_last_cached_row_stay_infinite(cuda, split):
+    """Slots that fill up a matrix tile read the last cached row again; Inf there is Inf in the output
+    (as of any softmax with a weight above 0), not the NaN of 0 * Inf."""
+    from bf16_huffman_infer_amd import ops
+    q_heads, kv_heads, max_len, p = 8, 2, 512, 70
+    qk, v, kc, vc, cos, sin = _case(q_heads, kv_heads, max_len, 11)
+    pos = torch.tensor([p], device="cuda")
+    want = torch.empty(q_heads, 128, dtype=torch.bfloat16, device="cuda")
+    got = torch.empty_like(want)
+
+    def call(out):
+        if split:
+            ops.decode_attention(qk, v, None, cos, sin, pos, kc, vc, out=out)
+        else:
+            _without_workspace(qk, v, cos, sin, pos, kc, vc, q_heads, kv_heads, out)
+    call(want)
+    vc[:, p - 1, 5] = float("inf")
+    call(got)
+    assert bool((got[:, 5] == float("inf")).all())
+    others = torch.arange(128, device="cuda") != 5
+    assert torch.equal(got[:, others], want[:, others])
