@@ -765,7 +765,9 @@ def _fuses_above_32_rows(input: Tensor, bias: Optional[Tensor]) -> bool:
         return False
     if torch.autograd.forward_ad._current_level >= 0 or torch._C._functorch.peek_interpreter_stack() is not None:
         return False
-    if torch.is_autocast_enabled('cuda') or torch._C._len_torch_dispatch_stack() or torch.compiler.is_compiling():
+    if torch.is_autocast_enabled('cuda') or torch._C._len_torch_dispatch_stack():
+        return False
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None:       # torch.compile / export; torch.jit.trace
         return False
     return type(input) in (Tensor, nn.Parameter)
 

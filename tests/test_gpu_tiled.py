@@ -110,3 +110,17 @@ def test_tiled_product_rejections(cuda):
     ops._fill_member(member[0], mod, y, None, mod.rem)
     rc = _lib.load().bhi_tile_bf16_huffman(member, x.data_ptr(), 1, 1024, 40, None, 0, None)
     assert rc != 0 and b"workspace" in _lib.load().bhi_last_error_string()
+
+
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
+def test_traced_call_records_the_product(cuda):
+    """``torch.jit.trace`` at a row count of the tiled product: the module it returns computes."""
+    from bf16_huffman_infer_amd.functional import CompressedLinear
+    M, K, rows = 1024, 1024, 40
+    w = gaussian_weight(M, K, seed=8)
+    lin = CompressedLinear(_cls("huffman").compress(w), None).cuda().eval()
+    a, b = (torch.randn(rows, K, generator=torch.Generator().manual_seed(i)).bfloat16().cuda() for i in range(2))
+    with torch.no_grad():
+        traced = torch.jit.trace(lambda x: torch.nn.functional.linear(x, lin.weight), (a,), check_trace=False)
+        assert "linear" in str(traced.graph)
+        _check(traced(b), b, w)

@@ -41,3 +41,18 @@ def test_workspace_follows_the_slice_choice():
                            and -(-M // (16 * nw)) <= 256 and 1024 + -(-M // (16 * nw)) * 16 * nw * tiles * 64 * d == need]
                 assert choices, (split_k, M, Ks, rows, need)
         assert lib.bhi_tile_workspace_bytes(split_k, M, Ks, 16) < 0 and lib.bhi_tile_workspace_bytes(split_k, M, Ks, 129) < 0
+
+
+def test_not_while_the_call_is_traced(monkeypatch):
+    """A tracer records what goes through the dispatcher: of the tiled product that is the empty output alone."""
+    from bf16_huffman_infer_amd.functional import _fuses_above_32_rows as fuses
+    x, seen = torch.zeros(40, 8), []
+
+    def step(v):
+        seen.append((torch.jit.is_tracing(), fuses(v, None)))
+        return v + 1
+    torch.jit.trace(step, (x,), check_trace=False)
+    assert seen == [(True, False)]
+    assert fuses(x, None)
+    monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
+    assert not fuses(x, None)
