@@ -40,11 +40,19 @@ LANE_BYTES_PER_STEP = 512          # 64 lanes x 8 exponent bytes
 _ready_devices = set()
 
 
+def _not_on_a_gpu():
+    """For an index that ``Tensor.get_device()`` gives where there is none, -1.  torch's device switches and stream
+    lookups take that for the current device, and a kernel would get host addresses."""
+    raise ValueError("expected tensors on a GPU")
+
+
 def _stream(t: Tensor) -> int:
     """The current torch stream of ``t``'s device.  The first op on a device also lets the
     library do its once-per-device lookups: whatever comes first in a process is an eager call
     (a conversion, a warm-up), so none of them is left for a call under stream capture."""
     index = t.get_device()
+    if index < 0:
+        _not_on_a_gpu()
     if index not in _ready_devices:
         if not torch.cuda.is_current_stream_capturing():
             with torch.cuda.device(index):
@@ -58,6 +66,8 @@ _here = contextlib.nullcontext()
 
 def _on_device(index: int):
     """Makes device ``index`` current for a ``with`` block; nothing to do where it already is."""
+    if index < 0:
+        _not_on_a_gpu()
     return _here if torch._C._cuda_getDevice() == index else torch.cuda.device(index)
 
 
@@ -307,6 +317,8 @@ def place_streams(streams: Tensor, lengths: Tensor, starts: Tensor, words: Tenso
     int64 ``[n]`` of any stride."""
     if starts.dtype != torch.int64 or starts.dim() != 1 or starts.numel() != streams.shape[0]:
         raise RuntimeError("starts must be one int64 per stream")
+    if starts.get_device() != streams.get_device() or lengths.numel() != streams.shape[0]:
+        raise RuntimeError("starts must be on the device of streams, and lengths one per stream")
     with _on_device(streams.get_device()):
         _lib.check(_lib.load().bhi_place_streams(
             _req(streams, torch.int32, "streams"), streams.shape[1], _req(lengths, torch.int32, "lengths", streams),

@@ -226,3 +226,53 @@ def test_workspace_of_the_fused_product_follows_the_slice_choice():
             assert per_group % d == 0
             if (M // 4 // (8 if rows <= 16 else 16)) * d <= 256:
                 assert lib.bhi_gemm_workspace_bytes(split_k, M, Ks, rows) <= static
+
+
+def test_direct_wrappers_refuse_cpu_tensors_before_any_launch(monkeypatch):
+    """The functions that bypass the dispatcher hand raw pointers to kernels: tensors that all lie in host memory
+    agree with each other, and must be refused all the same."""
+    from bf16_huffman_infer_amd import _lib, ops
+
+    class NoLaunch:
+        def __getattr__(self, name):
+            fn = getattr(lib, name)
+            if name.endswith("_bytes") or name.endswith("_capacity"):      # host arithmetic
+                return fn
+
+            def launch(*args):
+                raise AssertionError(f"{name} was reached")
+            return launch
+    lib = _lib.load()
+    monkeypatch.setattr(_lib, "load", lambda: NoLaunch())
+    huffman, ans = _huffman_weight(128, 384), _ans_weight(128, 768)
+    bf16 = dict(dtype=torch.bfloat16)
+
+    def x(w, rows):
+        return torch.zeros(rows, w.rem.shape[0], w.rem.shape[2], **bf16)
+
+    def y(rows):
+        return torch.empty(rows, 128, **bf16)
+    calls = []
+    for w in (huffman, ans):
+        calls += [lambda w=w: ops.gemv_bf16_grouped([w], x(w, 1), [y(1)]),
+                  lambda w=w: ops.gemv_bf16_grouped([w, w], x(w, 2), [y(2), y(2)], x_mode=ops.X_RMS,
+                                                    x_aux=torch.ones(w.rem.shape[0] * w.rem.shape[2], **bf16)),
+                  lambda w=w: ops.gemm_bf16(w, x(w, 12), y(12)),
+                  lambda w=w: ops.gemm_bf16_grouped([w, w], x(w, 12), [y(12), y(12)]),
+                  lambda w=w: ops.tile_bf16(w, x(w, 40), y(40))]
+    streams, starts = torch.zeros(2, 8, dtype=torch.int32), torch.zeros(2, dtype=torch.int64)
+    words, lengths = torch.zeros(64, dtype=torch.int32), torch.zeros(2, dtype=torch.int32)
+    cache, tables = torch.zeros(1, 16, 128, **bf16), torch.zeros(16, 128)
+    calls += [lambda: ops.split_planes(torch.zeros(128, 128, **bf16), 1),
+              lambda: ops.pair_histogram(torch.zeros(64, dtype=torch.uint8)),
+              lambda: ops.place_streams(streams, lengths, starts, words),
+              lambda: ops.rms_norm(torch.zeros(2, 64, **bf16), torch.ones(64, **bf16), 1e-6),
+              lambda: ops.silu_mul(torch.zeros(2, 64, **bf16), torch.zeros(2, 64, **bf16)),
+              lambda: ops.decode_attention(torch.zeros(2, 128, **bf16), torch.zeros(1, 128, **bf16), None, tables, tables,
+                                           torch.zeros(1, dtype=torch.int64), cache, cache.clone())]
+    for i, call in enumerate(calls):
+        with pytest.raises(ValueError):
+            call()
+    assert -1 not in ops._ready_devices
+    with pytest.raises(RuntimeError, match="one per stream"):
+        ops.place_streams(streams, lengths[:1], starts, words)
