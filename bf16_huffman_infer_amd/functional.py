@@ -23,7 +23,7 @@ from .ops import (GEMM_MAX_ROWS, ans_decode, ans_encode, ans_encode_capacity, en
                   gemm_bf16_grouped,
                   gemv_bf16_ans, gemv_bf16_grouped, gemv_bf16_huffman, gemv_bf16_nibble, huffman_decode, huffman_encode,
                   nibble_decode, nibble_encode, nibble_encode_capacity)
-from .utils import get_block_size_n, split_bf16
+from .utils import get_block_size_n
 
 ANS_PRECISION = 8
 MAX_FUSED_BATCH = 8
@@ -50,10 +50,25 @@ __all__ = [
 ]
 
 
-def _single_counts(pairs: Tensor) -> Tensor:
-    """int64 ``[256]`` occurrences of every exponent from those of the pairs."""
-    pairs = pairs.view(256, 256)                 # [second, first]
-    return pairs.sum(0) + pairs.sum(1)
+def _exponents(a: Tensor) -> Tensor:
+    """The exponent bytes of BF16 ``a`` on the GPU (:func:`.utils.split_bf16`'s, without the other plane and the
+    32-bit integers)."""
+    assert a.dtype == torch.bfloat16
+    return (a.detach().to(torch.device('cuda', 0)).contiguous().view(torch.int16) >> 7).to(torch.uint8)
+
+
+def _kernel_counts(exp: Tensor) -> bool:
+    """Whether the histogram kernel takes ``exp``: eight-byte loads of GPU memory."""
+    return exp.is_cuda and exp.numel() > 0 and exp.numel() % 8 == 0 and exp.data_ptr() % 8 == 0
+
+
+def _exponent_counts(exp: Tensor) -> Tensor:
+    """int64 ``[256]`` occurrences of every exponent."""
+    exp = exp.flatten()
+    if _kernel_counts(exp):
+        pairs = _ops.pair_histogram(exp).view(256, 256)          # [second, first]
+        return pairs.sum(0) + pairs.sum(1)
+    return torch.bincount(exp.to(torch.int32), minlength=256)
 
 
 def _to_host(t: Tensor) -> Tensor:
@@ -167,21 +182,19 @@ class HuffmanWeight(nn.Module):
     @classmethod
     def get_codec(cls, a: Tensor) -> LUTHuffmanEncoder:
         """One code per weight matrix, built from the histogram of exponent pairs."""
-        _, exp = split_bf16(a.detach().to(torch.device('cuda', 0)))
-        return cls._codec_of(cls._pair_counts(exp))
-
-    @classmethod
-    def _codec_of(cls, counts: Tensor) -> LUTHuffmanEncoder:
-        """The code for int64 ``[65536]`` pair counts."""
         codec = LUTHuffmanEncoder()
-        codec.build_lut(counts.cpu())
+        codec.build_lut(cls._pair_counts(_exponents(a)).cpu())
         return codec
 
     @staticmethod
     def _pair_counts(exp: Tensor) -> Tensor:
         """int64 [65536]: occurrences of every exponent pair ``a | b << 8`` (a = even column) of ``[M, K]``
-        exponents, K a multiple of eight."""
-        return _ops.pair_histogram(exp.contiguous())
+        exponents, K even."""
+        exp = exp.contiguous()
+        if exp.size(1) % 2 == 0 and _kernel_counts(exp):
+            return _ops.pair_histogram(exp)
+        pairs = exp[:, 0::2].to(torch.int32) | (exp[:, 1::2].to(torch.int32) << 8)
+        return torch.bincount(pairs.flatten(), minlength=65536)
 
     @classmethod
     def get_lut_kwargs(cls, codec: LUTHuffmanEncoder) -> dict[str, Tensor]:
@@ -228,8 +241,10 @@ class HuffmanWeight(nn.Module):
         consts = _lib.constants()
         nc = lib.bhi_chunks_per_group(M, Ks, n)
 
-        rem, sym = _ops.split_planes(a.detach().to(device).contiguous(), n)
-        codec = cls._codec_of(_ops.pair_histogram(sym))
+        a = a.detach().to(device).contiguous()
+        codec = cls.get_codec(a)
+        rem, sym = _ops.split_planes(a, n)
+        del a
 
         lengths = torch.zeros(n, G, nc, dtype=torch.int64, device=device)
         pieces = []                                                          # (chunk, first task, streams, lengths)
@@ -286,14 +301,7 @@ class ANSWeight(HuffmanWeight):
 
     @classmethod
     def get_codec(cls, a: Tensor) -> RANSEncoder:
-        device = torch.device('cuda', 0)
-        _, exp = split_bf16(a.detach().to(device))
-        counts = torch.bincount(exp.flatten().to(torch.int32), minlength=256)
-        return RANSEncoder(counts.tolist(), precision=ANS_PRECISION)
-
-    @classmethod
-    def _codec_of(cls, counts: Tensor) -> RANSEncoder:
-        return RANSEncoder(_single_counts(counts).tolist(), precision=ANS_PRECISION)
+        return RANSEncoder(_exponent_counts(_exponents(a)).tolist(), precision=ANS_PRECISION)
 
     @classmethod
     def get_lut_kwargs(cls, codec: RANSEncoder) -> dict[str, Tensor]:
@@ -354,13 +362,7 @@ class NibbleWeight(ANSWeight):
 
     @classmethod
     def get_codec(cls, a: Tensor) -> NibbleCodec:
-        device = torch.device('cuda', 0)
-        _, exp = split_bf16(a.detach().to(device))
-        return NibbleCodec(torch.bincount(exp.flatten().to(torch.int32), minlength=256))
-
-    @classmethod
-    def _codec_of(cls, counts: Tensor) -> NibbleCodec:
-        return NibbleCodec(_single_counts(counts))
+        return NibbleCodec(_exponent_counts(_exponents(a)))
 
     @classmethod
     def get_lut_kwargs(cls, codec: NibbleCodec) -> dict[str, Tensor]:

@@ -46,3 +46,50 @@ def test_convert_leaves_the_layer_alone_and_returns_host_buffers(cuda, algo):
     assert torch.equal(linear.weight.data, w) and not linear.weight.is_cuda
     assert all(not b.is_cuda for b in module.buffers()) and module.bias is linear.bias
     assert torch.equal(module.cuda().weight.get_weight().cpu().view(torch.int16), w.view(torch.int16))
+
+
+@pytest.mark.parametrize("algo", ["huffman", "ans", "nibble"])
+@pytest.mark.parametrize("M,K", [(128, 384), (3, 6), (7, 10), (1, 2)])
+def test_get_codec_takes_any_even_width(cuda, algo, M, K):
+    """A code for a matrix of any even width, from host or GPU memory, equal to the one of a histogram on the CPU."""
+    from bf16_huffman_infer_amd.functional import (ANS_PRECISION, ANSWeight, HuffmanWeight, LUTHuffmanEncoder, NibbleCodec,
+                                                   NibbleWeight, RANSEncoder)
+    from bf16_huffman_infer_amd.utils import split_bf16
+    w = gaussian_weight(M, K, seed=K)
+    exp = split_bf16(w)[1].to(torch.int64)
+    counts = torch.bincount(exp.flatten(), minlength=256)
+    for a in (w, w.cuda(), w.cuda().T.contiguous().T):
+        if algo == "huffman":
+            want = LUTHuffmanEncoder()
+            want.build_lut(torch.bincount((exp[:, 0::2] | exp[:, 1::2] << 8).flatten(), minlength=65536))
+            got = HuffmanWeight.get_codec(a)
+            assert (got.enc_table == want.enc_table).all() and (got.LUT1 == want.LUT1).all()
+        elif algo == "ans":
+            want = RANSEncoder(counts.tolist(), precision=ANS_PRECISION)
+            got = ANSWeight.get_codec(a)
+            assert list(got.freq) == list(want.freq) and list(got.cum) == list(want.cum)
+        else:
+            want, got = NibbleCodec(counts), NibbleWeight.get_codec(a)
+            assert (got.base, got.has_escapes) == (want.base, want.has_escapes)
+
+
+@pytest.mark.parametrize("algo", ["huffman", "ans", "nibble"])
+def test_compress_uses_the_class_own_codec(cuda, algo):
+    """``get_codec`` is where a subclass chooses the code: here one built from another matrix."""
+    from bf16_huffman_infer_amd import functional
+    base = {"huffman": functional.HuffmanWeight, "ans": functional.ANSWeight, "nibble": functional.NibbleWeight}[algo]
+    other = gaussian_weight(128, 1024, seed=9, std=0.1)
+    asked = []
+
+    class Own(base):
+        @classmethod
+        def get_codec(cls, a):
+            asked.append(a.shape)
+            # every exponent of `a` occurs in the code as well
+            return base.get_codec(torch.cat([other, a.detach().cpu()]))
+    w = gaussian_weight(256, 1024, seed=4)
+    mod = Own.compress(w)
+    want = base.get_lut_kwargs(base.get_codec(torch.cat([other, w])))
+    assert asked == [w.shape] and type(mod) is Own
+    assert all(torch.equal(getattr(mod, name), t) for name, t in want.items())
+    assert torch.equal(mod.cuda().get_weight().cpu().view(torch.int16), w.view(torch.int16))

@@ -276,3 +276,14 @@ def test_direct_wrappers_refuse_cpu_tensors_before_any_launch(monkeypatch):
     assert -1 not in ops._ready_devices
     with pytest.raises(RuntimeError, match="one per stream"):
         ops.place_streams(streams, lengths[:1], starts, words)
+
+
+@pytest.mark.parametrize("M,K", [(3, 6), (128, 384), (5, 130)])
+def test_pair_counts_of_host_tensors_and_any_even_width(M, K):
+    exp = torch.randint(0, 256, (M, K), generator=torch.Generator().manual_seed(M), dtype=torch.int32).to(torch.uint8)
+    counts = HuffmanWeight._pair_counts(exp)
+    want = torch.zeros(65536, dtype=torch.int64)
+    for row in exp.tolist():
+        for a, b in zip(row[0::2], row[1::2]):
+            want[a | b << 8] += 1
+    assert counts.dtype == torch.int64 and torch.equal(counts, want)
