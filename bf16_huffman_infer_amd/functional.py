@@ -8,6 +8,7 @@ Public surface of the reference's ``bf16_huffman_infer/functional.py``:
 bytes inside ``rem``/``exp``/``offsets``/``LUT1`` follow the wave64 layout of this
 package's HIP kernels.
 """
+import contextlib
 from typing import Optional
 
 import torch
@@ -559,6 +560,19 @@ def _weight_bytes(w: nn.Module) -> int:
     return sum(b.nelement() * b.element_size() for b in w.buffers())
 
 
+@contextlib.contextmanager
+def _visiting_gpu(module: nn.Module):
+    """``module`` on the current GPU for a while, then in host memory.  Parameters that lay there get their
+    own storage back: nothing is copied, and the pages of a copy (:func:`_to_host`) need not be touched."""
+    at_home = [(p, p.data) for p in module.parameters() if not p.is_cuda]
+    try:
+        yield module.cuda()
+    finally:
+        for p, data in at_home:
+            p.data = data
+        module.cpu()
+
+
 def convert(linear: nn.Linear, name, disable_precision_check=True, algo='huffman') -> nn.Module:
     """Compress one ``nn.Linear`` (reference ``functional.py:323-375``).
 
@@ -567,30 +581,24 @@ def convert(linear: nn.Linear, name, disable_precision_check=True, algo='huffman
     random GEMV deviates by 2 % or more from the dense layer.
     """
     assert algo in ('huffman', 'ans', 'smallest', 'nibble')
-    # The weight goes to the GPU once and the compressed buffers come back once; the layer itself stays
-    # where it is until the end.
-    weight = linear.weight
-    n = get_block_size_n(weight)[0]
-    assert weight.dim() == 2 and weight.dtype == torch.bfloat16
-    dense = weight.detach().to(torch.device('cuda', 0)).contiguous()
+    n = get_block_size_n(linear.weight)[0]
+    assert linear.weight.dim() == 2 and linear.weight.dtype == torch.bfloat16
     classes = {'huffman': [HuffmanWeight], 'ans': [ANSWeight], 'nibble': [NibbleWeight],
                'smallest': [HuffmanWeight, ANSWeight]}[algo]
-    compressed = min([cls(**cls._compress_on_device(dense, n)) for cls in classes], key=_weight_bytes)
-
-    module = CompressedLinear(weight=compressed, bias=linear.bias)
-    ori_size = linear.weight.nelement() * linear.weight.element_size()
-    ratio = _weight_bytes(module.weight) / ori_size
-
-    compressed.cuda()
-    dense = dense.cuda()
-    bias = None if linear.bias is None else linear.bias.detach().cuda()
-    x = torch.randn(1, linear.in_features, dtype=torch.bfloat16, device='cuda')
-    with torch.no_grad():
-        y1 = F.linear(x, dense, bias)
-        y2 = F.linear(x, compressed, bias)
-        lossless = torch.equal(compressed.get_weight().view(torch.int16), dense.view(torch.int16))
-    max_rtol = ((y2 - y1).abs() / y1.abs().clamp(min=1e-4)).max().item()
-    linear.cpu()
+    with _visiting_gpu(linear):
+        dense = linear.weight.detach()
+        compressed = min([cls(**cls._compress_on_device(dense, n)) for cls in classes], key=_weight_bytes)
+        ratio = _weight_bytes(compressed) / (dense.nelement() * dense.element_size())
+        module = CompressedLinear(weight=compressed.cuda(), bias=linear.bias)
+        x = torch.randn(1, linear.in_features, dtype=torch.bfloat16, device='cuda')
+        with torch.no_grad():
+            # the layer itself: a subclass's forward and whatever hooks it has are part of the comparison
+            y1 = linear(x)
+            y2 = module(x)
+            lossless = torch.equal(compressed.get_weight().view(torch.int16), dense.view(torch.int16))
+        max_rtol = ((y2 - y1).abs() / y1.abs().clamp(min=1e-4)).max().item()
+        del dense
+    module.bias = linear.bias
 
     fallback = False
     if ratio >= 1:

@@ -93,3 +93,37 @@ def test_compress_uses_the_class_own_codec(cuda, algo):
     assert asked == [w.shape] and type(mod) is Own
     assert all(torch.equal(getattr(mod, name), t) for name, t in want.items())
     assert torch.equal(mod.cuda().get_weight().cpu().view(torch.int16), w.view(torch.int16))
+
+
+def test_convert_compares_with_the_layer_itself(cuda):
+    """The precision check runs the layer that would be replaced, a subclass's forward, its further parameters and
+    hooks included; the layer keeps its storage."""
+    from bf16_huffman_infer_amd.functional import CompressedLinear, convert
+
+    class Adapted(torch.nn.Linear):
+        def __init__(self, *args, **kwargs):
+            super().__init__(*args, **kwargs)
+            self.gain = torch.nn.Parameter(torch.ones(self.out_features, dtype=torch.bfloat16))
+            self.register_buffer("shift", torch.zeros(self.out_features, dtype=torch.bfloat16))
+
+        def forward(self, x):
+            return super().forward(x) * self.gain + self.shift
+    w = gaussian_weight(4096, 1024, seed=6)
+    for change, accepted in ((None, True), ("gain", False), ("shift", False), ("hook", False)):
+        linear = Adapted(1024, 4096, dtype=torch.bfloat16)
+        linear.weight.data.copy_(w)
+        linear.bias.data.fill_(10)               # outputs around 10: their BF16 steps are 0.6 %, the check's bound is 2 %
+        if change == "hook":
+            linear.register_forward_hook(lambda module, args, out: out + 1)
+        elif change:
+            getattr(linear, change).data.add_(1)
+        held = {name: p.data_ptr() for name, p in linear.named_parameters()}
+        module = convert(linear, "layer", disable_precision_check=False)
+        assert (type(module) is CompressedLinear) == accepted, change
+        assert module.bias is linear.bias
+        assert {name: p.data_ptr() for name, p in linear.named_parameters()} == held
+        assert not linear.shift.is_cuda and torch.equal(linear.weight.data, w)
+    on_gpu = torch.nn.Linear(1024, 4096, dtype=torch.bfloat16).cuda()
+    on_gpu.weight.data.copy_(w)
+    module = convert(on_gpu, "layer")
+    assert type(module) is CompressedLinear and not on_gpu.weight.is_cuda and torch.equal(on_gpu.weight.data, w)
