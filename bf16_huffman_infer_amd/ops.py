@@ -17,7 +17,7 @@ import torch
 from torch import Tensor
 
 from . import _lib
-from .workspace import workspace
+from .workspace import captured, workspace
 
 _LIB = torch.library.Library("bf16_huffman_infer", "DEF")
 _LIB.define("gemv_bf16_huffman(Tensor A_rem, Tensor A_exp, Tensor X, Tensor(a!) Y, Tensor offsets, "
@@ -527,7 +527,7 @@ _workspaces = {}          # (device, stream) -> [zero-initialised uint8 tensors]
 
 
 def _gemm_workspace(device: torch.device, stream: int, nbytes: int, allocate=None) -> Tensor:
-    """The fused matrix product's workspace for launches on ``stream`` of ``device``: partial
+    """The fused matrix product's workspace for eager launches on ``stream`` of ``device``: partial
     sums of K slices and the arrival counters of their row blocks.  One per (device, stream):
     launches on one stream run one after the other and may share it, launches on different
     streams may overlap and must not.  Grown by replacement; the old one is kept alive because
@@ -541,6 +541,17 @@ def _gemm_workspace(device: torch.device, stream: int, nbytes: int, allocate=Non
     return held[-1]
 
 
+GEMM_COUNTER_BYTES = 1024            # at the front of that workspace
+
+
+def _workspace_of_launch(device: torch.device, stream: int, nbytes: int) -> Tensor:
+    """For the next launch on ``stream``.  Under capture it belongs to the capture (or to the recorded program),
+    not to the stream: torch records every graph on one stream, and a second graph that used the first one's
+    would find counters that only the first one's replay sets to zero."""
+    ws = captured("gemm", device, stream, nbytes, GEMM_COUNTER_BYTES)
+    return _gemm_workspace(device, stream, nbytes) if ws is None else ws
+
+
 def gemm_bf16(weight, X: Tensor, Y: Tensor, bias=None, static_workspace: bool = False, residual=None) -> None:
     """``Y = X @ W.T (+ bias)`` for up to 32 rows of ``X`` with ``W`` held compressed
     (:class:`HuffmanWeight` or :class:`ANSWeight`), decoded inside the matrix-core kernel.
@@ -550,9 +561,9 @@ def gemm_bf16(weight, X: Tensor, Y: Tensor, bias=None, static_workspace: bool = 
     ``[rows, M]`` written; ``bias`` (bf16 ``[M]``) and then ``residual`` (bf16 ``[rows, M]``) are added
     as separate BF16 additions would.  Plain function: only enqueues on the current stream.  Products that
     are cut along K keep their partial sums in a workspace that belongs to the (device, stream)
-    pair of the call and is allocated (and zeroed by a fill kernel) at the first such call on
-    that stream -- also under stream capture, where the allocation comes from the graph's own
-    pool and the fill becomes a node in front of the product.  ``static_workspace=True`` (Huffman
+    pair of the call and is allocated (and zeroed) at the first such call on that stream.  Under stream
+    capture it belongs to the capture or to the recorded program (:mod:`.workspace`).
+    ``static_workspace=True`` (Huffman
     weights) allocates nothing and uses the array built into the library instead: ONE array per
     GPU, so launches that take it and may overlap on the GPU (different streams) race."""
     lib = _lib.load()
@@ -587,7 +598,7 @@ def gemm_bf16(weight, X: Tensor, Y: Tensor, bias=None, static_workspace: bool = 
                 raise RuntimeError("gemm_bf16: the library has not been used on this device outside a stream capture yet")
             rc = lib.bhi_gemm_bf16_huffman_static(member, x_ptr, split_k, Ks, rows, stream)
         else:
-            ws = _gemm_workspace(device, stream, need)
+            ws = _workspace_of_launch(device, stream, need)
             rc = getattr(lib, "bhi_" + name)(member, x_ptr, split_k, Ks, rows, ws.data_ptr(), ws.numel(), stream)
         if rc != 0 and ws is not None:
             # the launch did not happen or was cut short: its counters may not be zero any more

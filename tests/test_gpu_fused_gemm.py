@@ -227,3 +227,37 @@ def test_built_in_workspace_on_request(cuda):
         assert torch.equal(rec.view(torch.int16), want.view(torch.int16)), f"replay {i}"
     with pytest.raises(RuntimeError, match="Huffman"):
         ops.gemm_bf16(_cls("ans").compress(w).cuda(), x, got, static_workspace=True)
+
+
+@pytest.mark.parametrize("algo", ["huffman", "ans"])
+@pytest.mark.parametrize("recorder", ["torch", "package"])
+def test_second_graph_does_not_depend_on_the_first(cuda, algo, recorder):
+    """Two graphs recorded one after the other (torch records both on one stream): the second is replayed
+    alone, then both in turn, with eager products between the replays, against the eager bits."""
+    from bf16_huffman_infer_amd.cudagraph_utils import GraphedCallable
+    w = gaussian_weight(1024, 4096, seed=13)
+    mod = _cls(algo).compress(w).cuda()
+    x = torch.randn(16, 4096, generator=torch.Generator().manual_seed(6)).bfloat16().cuda()
+    eager = torch.nn.functional.linear(x, mod)
+    torch.testing.assert_close(eager.float(), x.float() @ w.cuda().float().T, rtol=RTOL, atol=ATOL)
+    graphs, outs = [], []
+    for _ in range(2):
+        out = torch.zeros_like(eager)
+
+        def step(out=out):
+            out.copy_(torch.nn.functional.linear(x, mod))
+            return out
+        if recorder == "package":
+            graph = GraphedCallable(step, ())
+        else:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                step()
+        graphs.append(graph)
+        outs.append(out)
+    for i in (1, 1, 0, 1, 0, 0):
+        outs[i].zero_()
+        graphs[i].replay()
+        assert torch.equal(outs[i].view(torch.int16), eager.view(torch.int16)), i
+        again = torch.nn.functional.linear(x, mod)
+        assert torch.equal(again.view(torch.int16), eager.view(torch.int16))

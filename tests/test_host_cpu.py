@@ -287,3 +287,28 @@ def test_pair_counts_of_host_tensors_and_any_even_width(M, K):
         for a, b in zip(row[0::2], row[1::2]):
             want[a | b << 8] += 1
     assert counts.dtype == torch.int64 and torch.equal(counts, want)
+
+
+def test_gemm_workspace_of_a_capture_is_its_own(monkeypatch):
+    """Two captures on one stream get two workspaces, each zeroed on its own, and neither is the eager one."""
+    from bf16_huffman_infer_amd import ops, workspace
+    cpu, state = torch.device("cpu"), [0]
+    monkeypatch.setattr(workspace, "capture_id", lambda stream: state[0])
+    monkeypatch.setattr(workspace, "_captured", {})
+    monkeypatch.setattr(ops, "_workspaces", {})
+
+    def take(capture, nbytes=4096):
+        state[0] = capture
+        return ops._workspace_of_launch(cpu, 7, nbytes)
+    eager = take(0)
+    first = take(1)
+    assert take(1, 2048) is first and take(0) is eager
+    first.fill_(1)
+    second = take(2)
+    assert len({t.data_ptr() for t in (eager, first, second)}) == 3
+    assert not bool(second[:ops.GEMM_COUNTER_BYTES].any()) and second.numel() >= 4096
+    assert take(2, 1 << 20).numel() >= 1 << 20
+    recording = workspace.Recording()
+    with recording.warmup():
+        assert take(0) is eager
+    assert recording._needs == {("gemm", cpu): (4096, ops.GEMM_COUNTER_BYTES)}
