@@ -13,7 +13,10 @@ needs from them.
 :class:`GraphedCallable` is the model-independent part: any function of tensors whose
 launches stay on the current stream can be recorded with it.
 """
+import contextlib
+import gc
 import inspect
+import threading
 from typing import Callable, Sequence
 
 import torch
@@ -23,6 +26,30 @@ from .utils import shallow_copy_model
 from .workspace import Recording
 
 __all__ = ["GraphedCallable", "apply_graphed", "get_graphed_model"]
+
+
+_collector = threading.Lock()
+_captures = [0, False]          # recordings under way, whether the collector was on before the first
+
+
+@contextlib.contextmanager
+def _no_collection():
+    """No automatic garbage collection while a step is recorded.  A recording usually sits in a reference cycle
+    (an object that holds the recording of its own method), so a dead one waits for the collector, and the
+    destructor of its graph synchronises the device: within a capture, of this thread or another, that fails and
+    ends the process."""
+    with _collector:
+        if _captures[0] == 0:
+            _captures[1] = gc.isenabled()
+            gc.disable()
+        _captures[0] += 1
+    try:
+        yield
+    finally:
+        with _collector:
+            _captures[0] -= 1
+            if _captures[0] == 0 and _captures[1]:
+                gc.enable()
 
 
 class GraphedCallable:
@@ -56,7 +83,7 @@ class GraphedCallable:
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
-        with torch.no_grad(), self.workspaces.capture(), torch.cuda.graph(self.graph):
+        with torch.no_grad(), self.workspaces.capture(), _no_collection(), torch.cuda.graph(self.graph):
             self.static_outputs = fn(*self.static_inputs)
 
     def __call__(self, *args: torch.Tensor):

@@ -106,3 +106,62 @@ def test_patched_forward_with_both_model_signatures(with_cache_position, style):
     assert cache.resets == 2 and log[0]["cache"] is cache
     assert log[0]["generate_kwargs"] in ([], ["disable_compile"])
     assert [e["ids"].shape[1] for e in log[1:]] == [2, 1, 1]
+
+
+def test_no_garbage_collection_during_a_capture(monkeypatch):
+    """The destructor of a graph waits for the device, which no one may while a stream is being captured: a dead
+    recording that hangs in a reference cycle (an object whose method was recorded) must not be found by the
+    collector while the next one records."""
+    import contextlib
+    import gc
+    from bf16_huffman_infer_amd import cudagraph_utils
+    log, capturing = [], [False]
+
+    class FakeGraph:
+        def __del__(self):
+            log.append(("freed", capturing[0]))
+
+    @contextlib.contextmanager
+    def fake_capture(graph):
+        capturing[0] = True
+        try:
+            yield
+        finally:
+            capturing[0] = False
+    stream = types.SimpleNamespace(wait_stream=lambda other: None)
+    for name, value in dict(Stream=lambda: stream, current_stream=lambda: stream, stream=lambda s: contextlib.nullcontext(),
+                            synchronize=lambda: None, CUDAGraph=FakeGraph, graph=fake_capture).items():
+        monkeypatch.setattr(torch.cuda, name, value)
+
+    class Layer:                              # holds its recording, which holds the method, which holds the layer
+        def __init__(self, fail=False):
+            self.fail = fail
+            self.recorded = cudagraph_utils.GraphedCallable(self.step, (torch.zeros(1),), warmup=1)
+
+        def step(self, x):
+            if capturing[0]:
+                [[] for _ in range(5000)]     # objects the collector keeps count of
+            if self.fail and capturing[0]:
+                raise RuntimeError("not recordable")
+            return x
+    threshold = gc.get_threshold()
+    gc.collect()
+    gc.freeze()                               # little is left that would delay full collections
+    gc.collect()
+    gc.set_threshold(500, 1, 1)
+    try:
+        for _ in range(5):
+            Layer()
+        assert gc.isenabled()
+        with pytest.raises(RuntimeError, match="not recordable"):
+            Layer(fail=True)
+        assert gc.isenabled()
+        gc.disable()                          # a program that has switched it off finds it off
+        Layer()
+        assert not gc.isenabled()
+    finally:
+        gc.enable()
+        gc.set_threshold(*threshold)
+        gc.unfreeze()
+    gc.collect()
+    assert len(log) == 7 and not any(during for _, during in log)
