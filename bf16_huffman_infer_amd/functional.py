@@ -63,12 +63,17 @@ def _kernel_counts(exp: Tensor) -> bool:
     return exp.is_cuda and exp.numel() > 0 and exp.numel() % 8 == 0 and exp.data_ptr() % 8 == 0
 
 
+def _single_counts(pairs: Tensor) -> Tensor:
+    """int64 ``[256]`` occurrences of every exponent from those of the pairs."""
+    pairs = pairs.view(256, 256)                 # [second, first]
+    return pairs.sum(0) + pairs.sum(1)
+
+
 def _exponent_counts(exp: Tensor) -> Tensor:
     """int64 ``[256]`` occurrences of every exponent."""
     exp = exp.flatten()
     if _kernel_counts(exp):
-        pairs = _ops.pair_histogram(exp).view(256, 256)          # [second, first]
-        return pairs.sum(0) + pairs.sum(1)
+        return _single_counts(_ops.pair_histogram(exp))
     return torch.bincount(exp.to(torch.int32), minlength=256)
 
 
@@ -183,8 +188,13 @@ class HuffmanWeight(nn.Module):
     @classmethod
     def get_codec(cls, a: Tensor) -> LUTHuffmanEncoder:
         """One code per weight matrix, built from the histogram of exponent pairs."""
+        return cls._codec_of(cls._pair_counts(_exponents(a)))
+
+    @classmethod
+    def _codec_of(cls, counts: Tensor) -> LUTHuffmanEncoder:
+        """The code for int64 ``[65536]`` pair counts."""
         codec = LUTHuffmanEncoder()
-        codec.build_lut(cls._pair_counts(_exponents(a)).cpu())
+        codec.build_lut(counts.cpu())
         return codec
 
     @staticmethod
@@ -243,8 +253,12 @@ class HuffmanWeight(nn.Module):
         nc = lib.bhi_chunks_per_group(M, Ks, n)
 
         a = a.detach().to(device).contiguous()
-        codec = cls.get_codec(a)
         rem, sym = _ops.split_planes(a, n)
+        if getattr(cls.get_codec, '__func__', None) in _COUNTING_CODECS:
+            # what get_codec(a) gives, from the exponents at hand: another pass over `a` and its memory are 0.9 ms
+            codec = cls._codec_of(_ops.pair_histogram(sym))
+        else:
+            codec = cls.get_codec(a)                                         # a subclass chooses its own
         del a
 
         lengths = torch.zeros(n, G, nc, dtype=torch.int64, device=device)
@@ -303,6 +317,10 @@ class ANSWeight(HuffmanWeight):
     @classmethod
     def get_codec(cls, a: Tensor) -> RANSEncoder:
         return RANSEncoder(_exponent_counts(_exponents(a)).tolist(), precision=ANS_PRECISION)
+
+    @classmethod
+    def _codec_of(cls, counts: Tensor) -> RANSEncoder:
+        return RANSEncoder(_single_counts(counts).tolist(), precision=ANS_PRECISION)
 
     @classmethod
     def get_lut_kwargs(cls, codec: RANSEncoder) -> dict[str, Tensor]:
@@ -366,6 +384,10 @@ class NibbleWeight(ANSWeight):
         return NibbleCodec(_exponent_counts(_exponents(a)))
 
     @classmethod
+    def _codec_of(cls, counts: Tensor) -> NibbleCodec:
+        return NibbleCodec(_single_counts(counts))
+
+    @classmethod
     def get_lut_kwargs(cls, codec: NibbleCodec) -> dict[str, Tensor]:
         lut = torch.zeros(256, dtype=torch.int32)
         lut[0], lut[1], lut[2] = codec.base, int(codec.has_escapes), cls.MAGIC
@@ -383,6 +405,9 @@ class NibbleWeight(ANSWeight):
         lengths = torch.zeros(x.size(0), dtype=torch.int32, device=device)
         nibble_encode(x, cls.get_lut_kwargs(codec)['LUT'].to(device), out, lengths)
         return out, lengths
+
+
+_COUNTING_CODECS = [c.get_codec.__func__ for c in (HuffmanWeight, ANSWeight, NibbleWeight)]
 
 
 class CompressedLinear(nn.Module):
