@@ -765,31 +765,50 @@ def prefers_matrix_cores(rows: int, M: int, K: int) -> bool:
     return rows >= 3 and M >= 32768 and K >= 3584
 
 
-def prefers_tiles(rows: int, M: int, K: int) -> bool:
+def prefers_tiles(rows: int, M: int, K: int, split_k: int = 1, huffman: bool = True) -> bool:
     """Whether ``rows`` > 16 rows of activations go through the tiled product (``bhi_tile.h``) rather than
-    the matrix-core kernel (up to 32 rows) or decoding and a dense GEMM (above).  Measured on MI355X (us,
-    before / tiled; more in ``bhi_tile.h``):
+    the matrix-core kernel (up to 32 rows) or decoding and a dense GEMM (above).  Measured on MI355X in
+    recorded graphs, 37 shapes of 13 row counts and both codecs (us, the other path / tiled; four copies of
+    a weight in turn):
 
-    ====================  ===========  ===========  ============  ===========
-    M x K                 17 rows      48 rows      96 rows       128 rows
-    ====================  ===========  ===========  ============  ===========
-    512x3584              14.7 / 12.9  18.0 / 14.4  19.0 / 21.8   19.7 / 25.4
-    1536x1024             12.6 / 10.0  12.7 / 11.3  12.8 / 17.5   12.9 / 20.1
-    1024x4096             15.8 / 14.0  23.7 / 16.0  17.4 / 24.7   20.4 / 27.5
-    2048x8192             23.5 / 18.3  28.7 / 20.2  31.8 / 29.6   32.9 / 34.0
-    4096x4096             22.2 / 16.9  26.9 / 18.7  32.4 / 25.3   34.4 / 31.0
-    4096x11008 (rANS)     37.8 / 41.0  56.0 / 42.8  71.2 / 51.1
-    3584x18944            42.1 / 47.5  119 / 52.0   108 / 62.4    117 / 91.7
-    ====================  ===========  ===========  ============  ===========
-
-    A small layer's weight stays in the caches between the decoder and the GEMM, whose library kernel
-    gains on this one with every row; long rows in few row groups leave the tiled kernel few wavefronts,
-    and at 17 to 20 rows the other one needs five quads of batch rows only."""
-    if rows <= 20:
-        return K < 11008
+    =======================  ===========  ===========  ===========  ===========  ===========
+    M x K                    17 rows      24 rows      32 rows      64 rows      96 rows
+    =======================  ===========  ===========  ===========  ===========  ===========
+    640x1024 Huffman         12.9 / 9.8   14.2 / 9.8   16.6 / 10.0  12.3 / 12.1  11.8 / 14.4
+    640x1024 rANS            13.8 / 11.3  15.1 / 11.2  17.3 / 11.4  12.6 / 13.6  12.4 / 15.9
+    4096x4096 Huffman        22.2 / 16.9  24.5 / 16.6  28.6 / 16.7  27.4 / 20.2  32.6 / 24.5
+    12288x4096 Huffman       28.3 / 27.7  29.7 / 27.1  33.7 / 27.5  56.4 / 33.6  57.3 / 40.7
+    12288x4096 rANS          35.6 / 37.3  36.5 / 36.7  40.0 / 37.0  59.0 / 41.5  59.0 / 51.7
+    4096x11008 rANS          37.5 / 40.7  40.0 / 40.4  44.8 / 40.4  58.2 / 44.8  69.0 / 51.4
+    4096x12288 rANS          42.4 / 37.6  44.6 / 37.2  50.4 / 37.2  62.0 / 44.1  76.6 / 53.1
+    1024x18944 rANS          31.7 / 35.2  34.5 / 35.3  37.9 / 35.3  67.8 / 39.7  68.9 / 46.1
+    3584x18944 Huffman       41.2 / 47.7  44.8 / 47.6  50.7 / 48.1  102 / 58.3   108 / 63.9
+    3584x18944 rANS          50.7 / 70.5  53.6 / 70.3  60.1 / 70.7  104 / 76.3   109 / 75.7
+    16384x3584 Huffman       29.7 / 38.9  31.1 / 38.7  35.1 / 39.0  56.1 / 45.8  58.0 / 46.9
+    18944x3584 Huffman       44.5 / 36.2  47.5 / 36.2  55.2 / 36.5  65.1 / 43.9  67.6 / 59.6
+    18944x3584 rANS          56.4 / 53.1  59.7 / 53.2  66.5 / 53.5  66.4 / 57.9  69.2 / 80.6
+    =======================  ===========  ===========  ===========  ===========  ===========
+    """
+    tasks = split_k * _lib.load().bhi_chunks_per_group(M, K // split_k, split_k)      # of a row group
+    steps = K / (STEP_COLS * tasks)                                                   # of a task
+    if rows <= 32:
+        # The other kernel is at its best with 12 to 16 wavefronts for every compute unit (it is cut along K
+        # below 8192 rows only) and pays for each four rows of X; this one lags on long tasks, whose lanes
+        # drift out of the ring, and its rANS steps cost more.
+        waves = (M if M >= 8192 else M * tasks) / (4 * 256)
+        if 12 < waves <= 16 and steps > 24:
+            return huffman and rows > 28 and tasks > 1
+        if huffman or rows > 20:
+            return True
+        return waves > 16 or (M >= 8192 and waves > 12) or (steps < 13 and K < 16384)
     if rows <= 64:
-        return True
-    return M * K >= 16 << 20
+        # a small layer's weight stays in the caches between the decoder and the GEMM
+        return huffman or rows <= 48 or M * K >= 7 << 18
+    # Above, the library's kernel gains on this one with every row.  With one task per row group and four to
+    # five wavefronts for a unit, blocks of six or eight leave a quarter of the units idle.
+    if M * K < 16 << 20:
+        return False
+    return huffman or rows <= 80 or not (tasks == 1 and 4 * 4096 < M < 5 * 4096)
 
 
 def _fuses_above_32_rows(input: Tensor, bias: Optional[Tensor]) -> bool:
@@ -814,7 +833,9 @@ def _tiled(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool
     split_k, M, N = _ops._buffer(weight, 'rem').shape
     if input.dtype != torch.bfloat16 or (bias is not None and bias.dtype != torch.bfloat16) or not input.is_cuda:
         return False
-    if input.size(1) != split_k * N or input.numel() >= 2 ** 31 or not prefers_tiles(rows, M, split_k * N):
+    if input.size(1) != split_k * N or input.numel() >= 2 ** 31:
+        return False
+    if not prefers_tiles(rows, M, split_k * N, split_k, 'LUT1' in weight._buffers):
         return False
     return rows <= GEMM_MAX_ROWS or ((bias is None or tuple(bias.shape) == (M,)) and _fuses_above_32_rows(input, bias))
 

@@ -1,4 +1,5 @@
 """Where the tiled product may take the place of decoding and ``F.linear``, and the workspace it asks for."""
+import pytest
 import torch
 import torch.autograd.forward_ad as forward_ad
 
@@ -56,3 +57,27 @@ def test_not_while_the_call_is_traced(monkeypatch):
     assert fuses(x, None)
     monkeypatch.setattr(torch.compiler, "is_compiling", lambda: True)
     assert not fuses(x, None)
+
+
+# (M, K, rows, Huffman, rANS): whether the tiled product was the faster one by more than 2 % (None: about equal)
+MEASURED = [
+    (640, 1024, 17, True, True), (640, 1024, 48, True, None), (640, 1024, 64, None, False), (640, 1024, 65, False, False),
+    (1024, 4096, 17, True, None), (4096, 4096, 17, True, True), (4096, 4096, 96, True, True),
+    (12288, 4096, 17, None, False), (12288, 4096, 32, True, True), (12288, 4096, 128, True, True),
+    (11008, 4096, 20, None, False), (13824, 5120, 20, True, True), (4096, 11008, 17, None, False), (4096, 11008, 32, True, True),
+    (4096, 12288, 17, True, True), (2048, 11008, 17, True, True), (1024, 18944, 17, None, False), (1024, 18944, 32, True, True),
+    (3584, 18944, 17, False, False), (3584, 18944, 24, False, False), (3584, 18944, 32, True, False), (3584, 18944, 33, True, True),
+    (4096, 14336, 24, False, False), (16384, 3584, 17, False, False), (16384, 3584, 32, False, False), (16384, 3584, 33, True, True),
+    (16384, 4096, 24, False, False), (18944, 3584, 17, True, True), (18944, 3584, 80, True, True), (18944, 3584, 96, True, False),
+    (24576, 4096, 17, True, True), (24576, 4096, 96, True, True), (8192, 8192, 17, True, False), (8192, 8192, 24, True, None),
+    (1536, 6784, 17, True, False), (9216, 5504, 20, True, False), (5120, 13824, 17, True, True), (16384, 1024, 112, True, True),
+]
+
+
+@pytest.mark.parametrize("M,K,rows,huffman,rans", MEASURED)
+def test_tiled_product_is_chosen_where_it_was_faster(M, K, rows, huffman, rans):
+    from bf16_huffman_infer_amd.functional import prefers_tiles
+    from bf16_huffman_infer_amd.utils import get_block_size_n
+    split_k, = get_block_size_n(torch.empty(1, K, device="meta"))
+    assert huffman is None or prefers_tiles(rows, M, K, split_k, True) == huffman
+    assert rans is None or prefers_tiles(rows, M, K, split_k, False) == rans
