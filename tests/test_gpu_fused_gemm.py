@@ -73,12 +73,13 @@ def test_row_counts_that_fill_no_whole_block(cuda, algo, rows, M, K):
     w = gaussian_weight(M, K, seed=M + rows)
     mod = _cls(algo).compress(w).cuda()
     x = torch.randn(rows, K, generator=torch.Generator().manual_seed(rows)).bfloat16().cuda()
-    y = torch.full((rows, M), float("nan"), dtype=torch.bfloat16, device="cuda")
-    guard = torch.full((4096,), 7.0, dtype=torch.bfloat16, device="cuda")       # allocated right behind y
+    held = torch.full((rows * M + 8192,), 7.0, dtype=torch.bfloat16, device="cuda")      # Y in the middle
+    y = held[4096:-4096].view(rows, M)
+    y.fill_(float("nan"))
     ops.gemm_bf16(mod, x.view(rows, *mod.rem.shape[::2]), y)
     ref = x.float() @ w.cuda().float().T
     torch.testing.assert_close(y.float(), ref, rtol=RTOL, atol=ATOL)
-    assert bool((guard == 7.0).all())
+    assert bool((held[:4096] == 7.0).all()) and bool((held[-4096:] == 7.0).all())
 
 
 @pytest.mark.parametrize("algo", ["huffman", "ans"])

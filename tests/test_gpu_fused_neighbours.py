@@ -45,6 +45,56 @@ def test_silu_mul_kernel_against_torch(cuda):
     torch.testing.assert_close(got.float(), want.float(), rtol=2.0 ** -6, atol=1e-6)
 
 
+@pytest.mark.parametrize("rows", [1, 5])
+@pytest.mark.parametrize("K", [2, 126, 2046, 2048, 2050, 4096, 4098, 5120, 8192, 8194, 18944, 20480, 20482, 24576])
+def test_rms_norm_kernel_row_lengths(cuda, rows, K):
+    """Rows that a block holds in registers (up to 2048, 4096, 8192 and 20480 elements) and longer ones, which it reads
+    twice; each row on its own scale, and nothing written past the last."""
+    from bf16_huffman_infer_amd import _lib
+    g = torch.Generator().manual_seed(K + rows)
+    x = (torch.randn(rows, K, generator=g) * torch.arange(1, rows + 1)[:, None]).bfloat16().cuda()
+    gamma = (1 + 0.1 * torch.randn(K, generator=g)).bfloat16().cuda()
+    held = torch.full((rows * K + 512,), 7.0, dtype=torch.bfloat16, device="cuda")
+    got = held[256:-256].view(rows, K)
+    _lib.check(_lib.load().bhi_rms_norm(x.data_ptr(), gamma.data_ptr(), got.data_ptr(), rows, K, 1e-6,
+                                        torch.cuda.current_stream().cuda_stream), "rms_norm")
+    want = x.double() * torch.rsqrt(x.double().pow(2).mean(-1, keepdim=True) + 1e-6) * gamma.double()
+    # one rounding to BF16's eight significant bits (half a step of 2^-7 at 1: 2^-8), and fp32 sums of up to 24576
+    # squares, each thread's at most 96 in a row, 14 more to join them, a handful of roundings after: 128 * 2^-24
+    assert bool(((got.double() - want).abs() <= (2.0 ** -8 + 2.0 ** -17) * want.abs()).all())
+    assert bool((held[:256] == 7.0).all()) and bool((held[-256:] == 7.0).all())
+
+
+def _fused(mods, x, mode, aux, residuals=None, eps=0.0):
+    """The launch with the transform inside, whatever :func:`fuses_input` would choose."""
+    from bf16_huffman_infer_amd import ops
+    rows = x.shape[0]
+    ys = [torch.full((rows, m.rem.shape[1]), float("nan"), dtype=torch.bfloat16, device="cuda") for m in mods]
+    ops.gemv_bf16_grouped(mods, x.view(rows, *mods[0].rem.shape[::2]), ys, None, residuals, mode, aux, eps)
+    return ys
+
+
+@pytest.mark.parametrize("algo", ["huffman", "ans"])
+@pytest.mark.parametrize("rows", [1, 2, 3, 4])
+@pytest.mark.parametrize("K", [1024, 4096, 5120, 12288, 22528])
+def test_transforms_inside_the_launch(cuda, algo, rows, K):
+    """Both transforms inside the GEMV at every row count, on short and long tasks and rows of every kind that
+    the RMSNorm kernel tells apart: the bits of the kernels of their own."""
+    from bf16_huffman_infer_amd import ops
+    from bf16_huffman_infer_amd.functional import linear_grouped
+    mods = [_cls(algo).compress(gaussian_weight(M, K, seed=M + K)).cuda() for M in (256, 128)]
+    g = torch.Generator().manual_seed(rows + K)
+    x = (torch.randn(rows, K, generator=g) * 2).bfloat16().cuda()
+    gamma = (1 + 0.1 * torch.randn(K, generator=g)).bfloat16().cuda()
+    gate = (torch.randn(rows, K, generator=g) * 1.5).bfloat16().cuda()
+    res = [torch.randn(rows, m.rem.shape[1], generator=g).bfloat16().cuda() for m in mods]
+    for inside, own in ((_fused(mods, x, ops.X_RMS, gamma, eps=1e-6), linear_grouped(ops.rms_norm(x, gamma, 1e-6), mods)),
+                        (_fused(mods, x, ops.X_SILU_MUL, gate, res),
+                         linear_grouped(ops.silu_mul(gate, x), mods, residuals=res))):
+        for a, b in zip(inside, own):
+            assert torch.equal(_bits(a), _bits(b))
+
+
 @pytest.mark.parametrize("algo", ["huffman", "ans"])
 @pytest.mark.parametrize("rows", [1, 2, 3, 4])
 def test_norm_in_front_of_grouped_gemv(cuda, algo, rows):
@@ -57,7 +107,9 @@ def test_norm_in_front_of_grouped_gemv(cuda, algo, rows):
     g = torch.Generator().manual_seed(rows)
     x = (torch.randn(rows, K, generator=g) * 2).bfloat16().cuda()
     gamma = (1 + 0.1 * torch.randn(K, generator=g)).bfloat16().cuda()
-    fused = linear_grouped(x, mods, input_norm=(gamma, 1e-6))
+    fused = _fused(mods, x, ops.X_RMS, gamma, eps=1e-6)
+    for a, b in zip(fused, linear_grouped(x, mods, input_norm=(gamma, 1e-6))):
+        assert torch.equal(_bits(a), _bits(b))                  # wherever the rule puts the norm
     h = ops.rms_norm(x, gamma, 1e-6)
     unfused = linear_grouped(h, mods)
     for w, a, b in zip(ws, fused, unfused):
@@ -79,9 +131,11 @@ def test_gate_product_in_front_and_residual_behind(cuda, algo, rows, M, K):
     gate = (torch.randn(rows, K, generator=g) * 1.5).bfloat16().cuda()
     up = torch.randn(rows, K, generator=g).bfloat16().cuda()
     res = torch.randn(rows, M, generator=g).bfloat16().cuda()
-    fused, = linear_grouped(up, [mod], input_gate=gate, residuals=[res])
+    fused, = _fused([mod], up, ops.X_SILU_MUL, gate, [res])
+    chosen, = linear_grouped(up, [mod], input_gate=gate, residuals=[res])
     h = ops.silu_mul(gate, up)
     plain, = linear_grouped(h, [mod])
+    assert torch.equal(_bits(fused), _bits(chosen))             # wherever the rule puts the product
     assert torch.equal(_bits(fused), _bits(plain + res))        # a separate BF16 addition gives the same bits
     prod = h.float() @ w.cuda().float().T
     bound = ATOL + RTOL * (prod + res.float()).abs() + 2.0 ** -8 * prod.abs()

@@ -49,13 +49,14 @@ def test_tiled_product(cuda, algo, make, M, K, n):
     mod = _cls(algo).compress_split_n(w, n=n).cuda()
     for rows in (17, 32, 33, 48, 49, 64, 65, 80, 81, 96, 97, 112, 113, 128):
         x = torch.randn(rows, K, generator=torch.Generator().manual_seed(rows)).bfloat16().cuda()
-        y = torch.full((rows, M), float("nan"), dtype=torch.bfloat16, device="cuda")
-        guard = torch.full((4096,), 7.0, dtype=torch.bfloat16, device="cuda")
+        held = torch.full((rows * M + 8192,), 7.0, dtype=torch.bfloat16, device="cuda")      # Y in the middle
+        y = held[4096:-4096].view(rows, M)
+        y.fill_(float("nan"))
         bias = (0.1 * torch.randn(M, device="cuda")).bfloat16() if rows % 2 else None
         for _ in range(2):                     # the second launch finds the first one's counters
             ops.tile_bf16(mod, x.view(rows, n, K // n), y, bias)
             _check(y, x, w, bias)
-        assert bool((guard == 7.0).all())
+        assert bool((held[:4096] == 7.0).all()) and bool((held[-4096:] == 7.0).all())
 
 
 @pytest.mark.parametrize("rows", [24, 40, 100])
