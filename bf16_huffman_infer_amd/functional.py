@@ -835,7 +835,7 @@ def _tiled(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool
         return False
     if input.size(1) != split_k * N or input.numel() >= 2 ** 31:
         return False
-    if not prefers_tiles(rows, M, split_k * N, split_k, 'LUT1' in weight._buffers):
+    if not prefers_tiles(rows, M, split_k * N, split_k, not isinstance(weight, ANSWeight)):
         return False
     return rows <= GEMM_MAX_ROWS or ((bias is None or tuple(bias.shape) == (M,)) and _fuses_above_32_rows(input, bias))
 
@@ -887,14 +887,23 @@ def linear_huffman(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor] 
     """``F.linear`` with a :class:`HuffmanWeight`: fused kernels up to 32 rows and, where they are faster,
     up to 128, else decode + dense GEMM (reference ``functional.py:390-411``)."""
     def fused(x):
-        b = weight._buffers
-        return mv_huffman(b['rem'], b['exp'], x, b['offsets'], b['LUT1'], b['LUT2'], b['LUT3'], b['LUT4'], b['code_lengths'])
+        b = weight._buffers          # without nn.Module's attribute lookups, a microsecond of the call
+        try:
+            args = (b['rem'], b['exp'], x, b['offsets'], b['LUT1'], b['LUT2'], b['LUT3'], b['LUT4'], b['code_lengths'])
+        except KeyError:             # a parametrization takes a buffer out and puts a property in its place
+            w = weight
+            args = (w.rem, w.exp, x, w.offsets, w.LUT1, w.LUT2, w.LUT3, w.LUT4, w.code_lengths)
+        return mv_huffman(*args)
     return _linear_compressed(input, weight, bias, fused)
 
 
 def linear_ans(input: Tensor, weight: ANSWeight, bias: Optional[Tensor] = None) -> Tensor:
     """rANS counterpart of :func:`linear_huffman` (reference ``functional.py:447-466``)."""
     def fused(x):
-        b = weight._buffers
-        return mv_ans(b['rem'], b['exp'], x, b['offsets'], b['LUT'])
+        b = weight._buffers          # as above
+        try:
+            args = (b['rem'], b['exp'], x, b['offsets'], b['LUT'])
+        except KeyError:
+            args = (weight.rem, weight.exp, x, weight.offsets, weight.LUT)
+        return mv_ans(*args)
     return _linear_compressed(input, weight, bias, fused)

@@ -312,3 +312,25 @@ def test_gemm_workspace_of_a_capture_is_its_own(monkeypatch):
     with recording.warmup():
         assert take(0) is eager
     assert recording._needs == {("gemm", cpu): (4096, ops.GEMM_COUNTER_BYTES)}
+
+
+@pytest.mark.parametrize("make,name", [(lambda: _huffman_weight(128, 384), "mv_huffman"), (lambda: _ans_weight(128, 768), "mv_ans")])
+def test_a_weight_whose_buffer_is_parametrized_reaches_the_kernel(monkeypatch, make, name):
+    """A parametrization takes the tensor out of the module's buffers and puts a property in its place."""
+    from bf16_huffman_infer_amd import functional
+    weight, seen = make(), []
+
+    def mv(rem, exp, x, offsets, *tables):
+        seen.append(rem)
+        return torch.zeros(x.shape[0], rem.shape[1], dtype=torch.bfloat16)
+    monkeypatch.setattr(functional, name, mv)
+    x = torch.zeros(2, weight.rem.shape[0] * weight.rem.shape[2], dtype=torch.bfloat16)
+    torch.nn.functional.linear(x, weight)
+
+    class Same(torch.nn.Module):
+        def forward(self, t):
+            return t
+    rem = weight.rem
+    torch.nn.utils.parametrize.register_parametrization(weight, "rem", Same())
+    torch.nn.functional.linear(x, weight)
+    assert len(seen) == 2 and all(t.data_ptr() == rem.data_ptr() for t in seen)
