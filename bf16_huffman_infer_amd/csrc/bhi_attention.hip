@@ -32,10 +32,12 @@
 //    of the K-sliced matrix product (bhi_mma.h), for the reasons and with the costs given there.
 //
 // Measured in a recorded graph, cache rows not in any cache, us (one block per q head walking all
-// slots with dot products before -> now): 28 / 4 heads at 6001 slots 149 -> 17.1, 32 / 8 heads at 301
-// slots 14.5 -> 8.8, at 1024 slots 10.0 now; 6.0 at one slot is what launch, position, rows and
+// slots with dot products before -> now): 28 / 4 heads at 6001 slots 149 -> 15.9, 32 / 8 heads at 301
+// slots 14.3 -> 7.5, at 1001 slots 8.8 now; 4.8 at one slot is what launch, position, rows and
 // output take in a row, and a hand-over costs 2.5 more.  Splits of 32 or 128 slots at least, and at
-// most 16 or 32 splits, were within 1 us of this or slower.
+// most 16 or 32 splits, were within 1 us of this or slower.  Without a workspace (one block per q
+// head, the looping kernel): 154 -> 81 at 6001 slots of 28 / 4 heads, 30.2 -> 22.5 and 14.3 -> 12.5 at
+// 1001 and 301 of 32 / 8, 5.5 -> 4.3 at one.
 #include <type_traits>
 #include "bhi_common.h"
 #include "bhi_host.h"
@@ -145,8 +147,8 @@ __device__ __forceinline__ float rescale(float m, float top) { return m == -INFI
 
 // GT: q heads a block is built for (1, 2 or 4): sums and weights are kept for that many.
 // LOOP: a wavefront's share may be more slots than it has in flight at once.  Built for one q head
-// only, for launches without a workspace: the loop keeps both ends of its registers alive (256 and
-// spills where 190 do), and with splits no share is that long.
+// only, for launches without a workspace: the loop keeps both ends of its registers alive (254 where
+// 218 do; above 256 a compute unit would hold one block, not two), and with splits no share is that long.
 template <int GT, bool LOOP>
 __global__ __launch_bounds__(kAttnThreads, 2) void decode_attention_kernel(const AttnArgs a) {
     constexpr int kRow = kAttnDim + 8;                           // q rows 16 bytes apart in bank order
@@ -301,6 +303,19 @@ __global__ __launch_bounds__(kAttnThreads, 2) void decode_attention_kernel(const
                     }
                 }
             }
+            // Rows that are not this wavefront's are dropped by value: a weight of 0 would make NaN of an Inf
+            // or NaN in them.  In the loop once, at the end of the walk (at 6001 slots 85.5 us with the
+            // selects in every batch, 80.6 so); without a loop where they are used (0.2 us of 15.9; a branch
+            // around them 0.1 more).
+            if (LOOP && b0 + NT * kAttnTile > cached) {
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        if (b0 + t * kAttnTile + 2 * i + half >= cached) vr[t][i] = make_uint2(0, 0);
+                    }
+                }
+            }
             if (LOOP && b0 != w0) {                              // earlier slots were weighted against an older maximum
                 if (lane < GT) factor[wave][lane] = scale_old;
 #pragma unroll
@@ -311,8 +326,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void decode_attention_kernel(const
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const float* w = weights[wave][t * kAttnTile + 2 * i + half];
-                    // dropped by value: a weight of 0 would make NaN of an Inf or NaN in the row
-                    const bool in = b0 + t * kAttnTile + 2 * i + half < cached;
+                    const bool in = LOOP || b0 + t * kAttnTile + 2 * i + half < cached;
                     const uint32_t lo = in ? vr[t][i].x : 0u, hi = in ? vr[t][i].y : 0u;
                     const f32x4a_t v = {bf16_lo(lo), bf16_hi(lo), bf16_lo(hi), bf16_hi(hi)};
 #pragma unroll

@@ -1,5 +1,5 @@
-// Fused decode + matrix product for up to 32 rows of X (F.linear's path for 9..16 rows, for 17..20 on
-// long rows, and from 3 rows on large layers; bhi_tile.h serves the others): the weights go from the decoder's
+// Fused decode + matrix product for up to 32 rows of X (F.linear's path for 9..16 rows, from 3 rows on
+// large layers, and for 17..32 rows where functional.prefers_tiles keeps a layer here): the weights go from the decoder's
 // registers straight into matrix-core instructions, the compressed bytes are read once
 // and no BF16 weight ever reaches HBM.
 //

@@ -24,9 +24,14 @@
 //   4096x12288     37.4 / 30.1   45.4 / 30.6   59.2 / 34.2   63.5 / 38.5   76.2 / 47.6   84.5 / 54.5
 //   18944x3584     45.9 / 36.4   57.2 / 37     65.8 / 39.9   66.1 / 45     68.8 / 60.2   71.0 / 64.3
 //
-// What bounds it now is the decoding itself: a step of four groups takes 0.83 us with one wavefront
-// per SIMD and 1.1 us with two, whatever the loads (rem bytes from cache: no change) and 30 % less
-// with them and X taken out.  Decoding step t + 1 between the products of step t gained nothing.
+// What bounds it now.  With two tiles of X the decoding: a step of four groups takes 0.83 us with one
+// wavefront per SIMD and 1.1 us with two, rem bytes from cache or not.  Every further tile adds 0.13 to 0.16 us
+// to a step of eight wavefronts, for which they read 32 KB of X from LDS, each of them all of it for its
+// sixteen weight rows: 0.11 us at the 128 bytes a clock that LDS delivers.  At five tiles X staged and read
+// is 16 of 72 us (measured with both taken out).  Decoding step t + 1 between the products of step t
+// gained nothing.  Long tasks pay more per step: at 28 steps and more lanes drift out of the ring, and where the
+// other kernel fills the compute units it is ahead up to 32 rows (16384x3584 at 20 rows: 29.2 there, 38.7 here;
+// functional.prefers_tiles).
 #pragma once
 // (included by bhi_task.h users after bhi_mma.h, whose argument block and workspace it shares)
 
