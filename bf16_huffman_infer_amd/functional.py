@@ -25,6 +25,7 @@ from .ops import (GEMM_MAX_ROWS, ans_decode, ans_encode, ans_encode_capacity, en
                   gemv_bf16_ans, gemv_bf16_grouped, gemv_bf16_huffman, gemv_bf16_nibble, huffman_decode, huffman_encode,
                   nibble_decode, nibble_encode, nibble_encode_capacity)
 from .utils import get_block_size_n
+from .workspace import recorded
 
 ANS_PRECISION = 8
 MAX_FUSED_BATCH = 8
@@ -424,7 +425,7 @@ class CompressedLinear(nn.Module):
         return F.linear(input, self.weight, self.bias)
 
 
-def fuses_input(rows: int, n_weights: int, norm: bool, huffman: bool) -> bool:
+def fuses_input(rows: int, n_weights: int, norm: bool, huffman: bool, in_graph: bool = True) -> bool:
     """Whether the RMSNorm (``norm``) or the SwiGLU product in front of a GEMV of ``n_weights`` weights
     in all happens inside its launch or in a launch of its own.
 
@@ -450,9 +451,26 @@ def fuses_input(rows: int, n_weights: int, norm: bool, huffman: bool) -> bool:
     rANS, SwiGLU, 2048x8192             14.6 / 15.0  16.1 / 15.2  17.7 / 15.4  19.2 / 15.8
     rANS, SwiGLU, 4096x12288            28.8 / 26.1  34.1 / 27.0  38.9 / 27.4  42.4 / 28.2
     ==================================  ===========  ===========  ===========  ===========
+
+    Outside a graph (``in_graph=False``) another launch is 8 to 11 us of host time, and most of these calls are bound by
+    the host (us per call):
+
+    ==================================  ===========  ===========  ===========
+    eager call                          1 row        2 rows       4 rows
+    ==================================  ===========  ===========  ===========
+    Huffman, norm, 4608x3584            20.7 / 31.6  20.8 / 31.0  22.3 / 31.2
+    Huffman, norm, 24576x4096           30.8 / 38.9  34.7 / 39.2  45.2 / 45.7
+    Huffman, SwiGLU, 4096x12288         20.9 / 28.8  22.4 / 28.9  33.7 / 28.9
+    Huffman, SwiGLU, 3584x18944         23.7 / 28.9  29.7 / 28.9  46.3 / 33.6
+    rANS, norm, 24576x4096              38.5 / 41.1  42.5 / 42.1  58.4 / 46.2
+    rANS, SwiGLU, 4096x12288            24.2 / 30.9  29.7 / 30.0  40.7 / 30.3
+    rANS, SwiGLU, 3584x18944            33.2 / 30.5  42.1 / 30.9  57.8 / 34.4
+    ==================================  ===========  ===========  ===========
     """
     if rows > _ops.X_TRANSFORM_MAX_ROWS:
         return False
+    if not in_graph:
+        return rows * n_weights <= ((210e6 if norm else 110e6) if huffman else (150e6 if norm else 60e6))
     if rows == 1:
         return n_weights <= (28e6 if norm else 51e6 if huffman else 20e6)
     return rows * n_weights <= (18e6 if norm else 22e6)
@@ -487,7 +505,7 @@ def linear_grouped(input: Tensor, weights, biases=None, *, residuals=None, input
     mode, aux, eps = _ops.X_PLAIN, None, 0.0
     if input_norm is not None or input_gate is not None:
         fusable = not isinstance(first, NibbleWeight) and fuses_input(
-            x.size(0), sum(w.rem.numel() for w in weights), input_norm is not None, hasattr(first, 'LUT1'))
+            x.size(0), sum(w.rem.numel() for w in weights), input_norm is not None, hasattr(first, 'LUT1'), recorded())
         if input_norm is not None:
             gamma, eps = input_norm
             gamma = gamma.detach()

@@ -65,6 +65,11 @@ class Recording:
         return held
 
 
+def recorded() -> bool:
+    """Whether the current call is being recorded into a graph, or is a warm-up run of a program that will be."""
+    return getattr(_recording, "current", None) is not None or torch.cuda.is_current_stream_capturing()
+
+
 def _fresh(device, nbytes, counters) -> Tensor:
     ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
     ws[:counters].view(torch.int32).zero_()

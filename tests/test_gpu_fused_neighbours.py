@@ -158,3 +158,36 @@ def test_more_rows_or_other_codecs_run_the_unfused_kernels(cuda, algo):
     a, = linear_grouped(x, [mod], input_gate=gate)
     b, = linear_grouped(ops.silu_mul(gate, x), [mod])
     assert torch.equal(_bits(a), _bits(b))
+
+
+@pytest.mark.parametrize("recorder", ["torch", "package"])
+@pytest.mark.parametrize("rows,Ms,K", [(2, (4608,), 3584), (4, (1024, 512), 8192)])
+def test_eager_and_recorded_calls_give_the_same_bits(cuda, recorder, rows, Ms, K):
+    """Eager calls keep the transform inside where a graph gives it a launch of its own."""
+    from bf16_huffman_infer_amd.cudagraph_utils import GraphedCallable
+    from bf16_huffman_infer_amd.functional import fuses_input, linear_grouped
+    mods = [_cls("huffman").compress(gaussian_weight(M, K, seed=M)).cuda() for M in Ms]
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, K, generator=g).bfloat16().cuda()
+    gate = torch.randn(rows, K, generator=g).bfloat16().cuda()
+    gamma = (1 + 0.1 * torch.randn(K, generator=g)).bfloat16().cuda()
+    n = sum(Ms) * K
+    for norm in (True, False):
+        assert fuses_input(rows, n, norm, True, False) and not fuses_input(rows, n, norm, True, True)
+    outs = [torch.empty(rows, 2 * sum(Ms), dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+
+    def step(out):
+        out.copy_(torch.cat(linear_grouped(x, mods, input_norm=(gamma, 1e-6)) + linear_grouped(x, mods, input_gate=gate), -1))
+        return out
+    step(outs[0])
+    if recorder == "package":
+        graph = GraphedCallable(lambda: step(outs[1]), ())
+    else:
+        step(outs[1])
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            step(outs[1])
+    for _ in range(3):
+        outs[1].zero_()
+        graph.replay()
+        assert torch.equal(_bits(outs[0]), _bits(outs[1]))

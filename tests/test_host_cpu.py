@@ -334,3 +334,17 @@ def test_a_weight_whose_buffer_is_parametrized_reaches_the_kernel(monkeypatch, m
     torch.nn.utils.parametrize.register_parametrization(weight, "rem", Same())
     torch.nn.functional.linear(x, weight)
     assert len(seen) == 2 and all(t.data_ptr() == rem.data_ptr() for t in seen)
+
+
+# (rows, weights, norm, Huffman): inside a GEMV's launch in an eager call, in a graph; None: measured about equal
+@pytest.mark.parametrize("rows,n,norm,huffman,eager,in_graph", [
+    (1, 4608 * 3584, True, True, True, True), (2, 4608 * 3584, True, True, True, False), (4, 6144 * 4096, True, True, True, False),
+    (1, 24576 * 4096, True, True, True, False), (2, 24576 * 4096, True, True, True, False), (4, 24576 * 4096, True, True, None, False),
+    (2, 4096 * 12288, False, True, True, False), (4, 4096 * 12288, False, True, False, False),
+    (1, 3584 * 18944, False, True, True, False), (4, 3584 * 18944, False, True, False, False),
+    (1, 4096 * 12288, False, False, True, False), (4, 4096 * 12288, False, False, False, False),
+    (1, 3584 * 18944, False, False, False, False), (4, 24576 * 4096, True, False, False, False), (5, 128 * 128, True, True, False, False)])
+def test_transforms_go_inside_a_launch_where_that_was_faster(rows, n, norm, huffman, eager, in_graph):
+    from bf16_huffman_infer_amd.functional import fuses_input
+    assert eager is None or fuses_input(rows, n, norm, huffman, False) == eager
+    assert fuses_input(rows, n, norm, huffman, True) == in_graph
