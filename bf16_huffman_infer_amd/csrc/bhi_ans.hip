@@ -46,6 +46,7 @@ struct AnsCodec {
     using Cursor = AnsCursor;
     template <int RING> using TileCursor = AnsTileCursor<RING>;
     using Table = AnsTable;
+    static constexpr bool kHuffman = false;
     static constexpr bool kTransformsX = true;    // kernels with RMSNorm / SiLU*mul in front of the product are built
     static constexpr int kTableWords = kAnsTableWords;
     static __device__ __forceinline__ bool variant(const uint8_t* __restrict__) { return false; }
@@ -172,6 +173,13 @@ extern "C" int bhi_tile_bf16_ans(const bhi_gemv_member* weight, const void* X, i
     if (int rc = launch_tile<AnsCodec>(weight, X, split_k, Ks, batch, workspace, workspace_bytes, 0, true,
                                         (hipStream_t)stream)) return rc;
     return bhi_launch_status("tile_bf16_ans");
+}
+
+extern "C" int bhi_wide_bf16_ans(const bhi_gemv_member* weight, const void* X, int split_k, int Ks, int batch,
+                                 void* workspace, int64_t workspace_bytes, void* stream) {
+    if (int rc = launch_wide<AnsCodec>(weight, X, split_k, Ks, batch, workspace, workspace_bytes, 0, true,
+                                        (hipStream_t)stream)) return rc;
+    return bhi_launch_status("wide_bf16_ans");
 }
 
 extern "C" int bhi_gemm_bf16_ans_grouped(const bhi_gemv_member* members, int n_members, const void* X, int split_k,

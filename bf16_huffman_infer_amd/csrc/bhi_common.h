@@ -408,15 +408,16 @@ struct AnsCursor : RowRingT<0> {
         pos = 2;
     }
 
-    // one symbol: returns the second word of its table entry ((sym << 23) | rem), advances the state
-    __device__ __forceinline__ uint32_t symbol(const uint32_t* __restrict__ table) { return symbol(table, xl, xh); }
-    static __device__ __forceinline__ uint32_t symbol(const uint32_t* __restrict__ table, uint32_t& xl, uint32_t& xh) {
+    // A symbol's table entry {freq, (sym << 23) | rem}, by byte 0 of the state.
+    static __device__ __forceinline__ uint2 look(const uint32_t* __restrict__ table, uint32_t xl) {
         // byte 0 of the state, times eight, in one instruction (written as a mask and a shift
         // the compiler makes it two; eight symbols per step, the kernel is bound by VALU issue)
         uint32_t off;
         asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:DWORD src1_sel:BYTE_0"
             : "=v"(off) : "v"(3u), "v"(xl));
-        const uint2 ent = *(const uint2*)((const char*)table + off);       // {freq, (sym << 23) | rem}
+        return *(const uint2*)((const char*)table + off);
+    }
+    static __device__ __forceinline__ void advance(uint2 ent, uint32_t& xl, uint32_t& xh) {
         // state >> 8 in one instruction (the compiler splits a 64-bit shift by a constant into two)
         uint64_t y;
         asm("v_lshrrev_b64 %0, 8, %1" : "=v"(y) : "v"(((uint64_t)xh << 32) | xl));
@@ -424,8 +425,14 @@ struct AnsCursor : RowRingT<0> {
         xl = (uint32_t)lowp;
         // freq <= 256 and y >> 32 < 2**24: a 24-bit multiply-add (the state is valid: < 2**64)
         xh = __umul24(ent.x, (uint32_t)(y >> 32)) + (uint32_t)(lowp >> 32);
+    }
+    // one symbol: returns the second word of its table entry, advances the state
+    static __device__ __forceinline__ uint32_t symbol(const uint32_t* __restrict__ table, uint32_t& xl, uint32_t& xh) {
+        const uint2 ent = look(table, xl);
+        advance(ent, xl, xh);
         return ent.y;
     }
+    __device__ __forceinline__ uint32_t symbol(const uint32_t* __restrict__ table) { return symbol(table, xl, xh); }
 
     __device__ __forceinline__ void refill(uint32_t word) {
         const bool need = xh == 0u;

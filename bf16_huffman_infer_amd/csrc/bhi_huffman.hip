@@ -13,6 +13,7 @@ namespace bhi {
 struct HuffCodec {
     using Cursor = HuffCursor;
     template <int RING> using TileCursor = HuffTileCursor<RING>;
+    static constexpr bool kHuffman = true;
     static constexpr bool kTransformsX = true;    // kernels with RMSNorm / SiLU*mul in front of the product are built
     static constexpr int kTableWords = kTableEntries;
     using Table = PlainTable<kTableEntries>;
@@ -154,6 +155,13 @@ extern "C" int bhi_tile_bf16_huffman(const bhi_gemv_member* weight, const void* 
     return bhi_launch_status("tile_bf16_huffman");
 }
 
+extern "C" int bhi_wide_bf16_huffman(const bhi_gemv_member* weight, const void* X, int split_k, int Ks, int batch,
+                                 void* workspace, int64_t workspace_bytes, void* stream) {
+    if (int rc = launch_wide<HuffCodec>(weight, X, split_k, Ks, batch, workspace, workspace_bytes, (int64_t)kTableEntries * 4, false,
+                                        (hipStream_t)stream)) return rc;
+    return bhi_launch_status("wide_bf16_huffman");
+}
+
 extern "C" int bhi_gemm_bf16_huffman_grouped(const bhi_gemv_member* members, int n_members, const void* X, int split_k,
                                              int Ks, int batch, void* stream) {
     if (int rc = launch_mma<HuffCodec>(members, n_members, X, split_k, Ks, batch, nullptr, 0,
@@ -227,6 +235,19 @@ extern "C" int64_t bhi_tile_workspace_bytes(int split_k, int M, int Ks, int batc
     if (batch < kTileMinBatch || batch > kTileMaxBatch) return bhi_fail(BHI_EBATCH, "the tiled product takes 17 to 128 rows of X");
     if (int rc = check_shape(split_k, M, Ks, kTailPadWords, &s)) return rc;
     return tile_workspace_bytes(s, batch);
+}
+
+extern "C" int bhi_wide_slices(int split_k, int M, int Ks) {
+    Shape s;
+    if (int rc = check_shape(split_k, M, Ks, kTailPadWords, &s)) return rc;
+    return wide_slices(s);
+}
+
+extern "C" int64_t bhi_wide_workspace_bytes(int split_k, int M, int Ks, int batch) {
+    Shape s;
+    if (batch < kWideMinBatch || batch > kWideMaxBatch) return bhi_fail(BHI_EBATCH, "the wide product takes 17 to 640 rows of X");
+    if (int rc = check_shape(split_k, M, Ks, kTailPadWords, &s)) return rc;
+    return wide_workspace_bytes(s, batch);
 }
 
 extern "C" int64_t bhi_encode_capacity(int n_steps) {

@@ -869,3 +869,4 @@ static inline void launch_decode(const void* A_rem, const void* A_exp, void* Y, 
 
 #include "bhi_mma.h"
 #include "bhi_tile.h"
+#include "bhi_wide.h"

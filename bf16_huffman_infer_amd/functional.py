@@ -9,6 +9,7 @@ bytes inside ``rem``/``exp``/``offsets``/``LUT1`` follow the wave64 layout of th
 package's HIP kernels.
 """
 import contextlib
+import functools
 from typing import Optional
 
 import torch
@@ -783,6 +784,7 @@ def prefers_matrix_cores(rows: int, M: int, K: int) -> bool:
     return rows >= 3 and M >= 32768 and K >= 3584
 
 
+@functools.lru_cache(maxsize=1024)        # an eager call asks every time
 def prefers_tiles(rows: int, M: int, K: int, split_k: int = 1, huffman: bool = True) -> bool:
     """Whether ``rows`` > 16 rows of activations go through the tiled product (``bhi_tile.h``) rather than
     the matrix-core kernel (up to 32 rows) or decoding and a dense GEMM (above).  Measured on MI355X in
@@ -829,6 +831,53 @@ def prefers_tiles(rows: int, M: int, K: int, split_k: int = 1, huffman: bool = T
     return huffman or rows <= 80 or not (tasks == 1 and 4 * 4096 < M < 5 * 4096)
 
 
+@functools.lru_cache(maxsize=1024)
+def prefers_wide(rows: int, M: int, K: int, split_k: int = 1, huffman: bool = True) -> bool:
+    """Whether 17 to 640 rows of activations go through the wide product (``bhi_wide.h``) rather than what
+    :func:`prefers_tiles` and the paths behind it choose.  Its blocks of 64 weight rows, cut along K as long as
+    every block has a compute unit of its own, cover the units in rounds; what counts is how full the
+    last one is.  Measured on MI355X in recorded graphs, twelve shapes of 17 row counts and both codecs (us, the
+    other path / wide; more in ``bhi_wide.h``):
+
+    ================================  ===========  ===========  ===========  ===========  ===========
+    M x K (filled units)              32 rows      64 rows      96 rows      256 rows     640 rows
+    ================================  ===========  ===========  ===========  ===========  ===========
+    512x1024 (6 %) Huffman            10.0 / 10.4  12.1 / 11.1  12.3 / 12.2  12.7 / 15.9  13.1 / 27.1
+    1024x4096 (25 %) Huffman          15.0 / 14.6  18.2 / 16.0  17.3 / 17.6  21.7 / 25.2  27.3 / 45.4
+    2048x2048 (50 %) rANS             13.4 / 13.6  16.1 / 14.4  17.0 / 16.6  20.6 / 23.4  24.3 / 38.3
+    4608x3584 (56 %) Huffman          18.1 / 19.4  22.5 / 21.5  32.4 / 23.2  46.4 / 31.7  44.8 / 55.0
+    12288x4096 (75 %) Huffman         29.9 / 32.2  35.6 / 35.6  42.7 / 37.0  79.3 / 50.3  97.4 / 92.0
+    3584x3584 (88 %) rANS             18.9 / 18.1  21.8 / 18.8  30.3 / 21.8  29.8 / 29.9  42.0 / 48.0
+    4096x12288 (100 %) rANS           39.7 / 38.2  46.2 / 40.5  55.0 / 43.5  81.5 / 58.8   123 / 96.6
+    8192x8192 (100 %) Huffman         44.2 / 35.4  52.8 / 40.4  57.8 / 42.8   105 / 61.7   121 / 116
+    18944x3584 (two rounds, 58 %) H   38.2 / 49.8  45.2 / 54.8  61.4 / 57.1  86.0 / 79.3   122 / 145
+    18944x3584 (two rounds, 58 %) r   55.5 / 63.0  59.5 / 67.6  71.0 / 69.2  90.5 / 90.9   130 / 149
+    32768x2048 (two rounds, full) r   36.4 / 42.7  42.8 / 45.6  47.1 / 47.0  86.2 / 67.1   128 / 113
+    ================================  ===========  ===========  ===========  ===========  ===========
+    """
+    slices = _lib.load().bhi_wide_slices(split_k, M, K // split_k)
+    blocks = M // 64 * slices
+    rounds = -(-blocks // 256)
+    filled = blocks / (256 * rounds)
+    weights = M * K
+    useful = filled * weights              # a layer that leaves units idle needs more work per block to win
+    if rows > 128:
+        if rounds > 1 and filled < 0.75:
+            return rows <= (320 if huffman else 192)
+        return useful >= 8 << 20 and rows <= (256 if useful < 24 << 20 else _ops.WIDE_MAX_ROWS)
+    if rounds > 1:
+        return rows > 80
+    if rows <= 32:
+        return filled >= 0.85 and weights >= 32 << 20
+    if filled >= 0.85 and weights >= 8 << 20:
+        return True
+    if weights < 4 << 20:
+        return False
+    if useful < 8 << 20:
+        return 48 < rows <= (96 if filled >= 0.5 else 64)
+    return rows > (64 if slices == 1 else 48)
+
+
 def _fuses_above_32_rows(input: Tensor, bias: Optional[Tensor]) -> bool:
     """Decoding and ``F.linear`` pass gradients, forward-mode tangents, function transforms, autocast, dispatch
     modes and tracing on to the input (and the bias); a fused product does not, and takes over only where
@@ -844,18 +893,29 @@ def _fuses_above_32_rows(input: Tensor, bias: Optional[Tensor]) -> bool:
     return type(input) in (Tensor, nn.Parameter)
 
 
-def _tiled(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool:
+def _takes(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], first: int, last: int, rule) -> bool:
+    """Whether a fused product for ``first`` to ``last`` rows takes the place of what runs else: its operands fit
+    it, ``rule`` wants it, and above 32 rows nothing is asked for but the value."""
     rows = input.size(0)
-    if not _ops.TILE_MIN_ROWS <= rows <= _ops.TILE_MAX_ROWS or isinstance(weight, NibbleWeight):
+    if not first <= rows <= last or isinstance(weight, NibbleWeight):
         return False
     split_k, M, N = _ops._buffer(weight, 'rem').shape
+    if not rule(rows, M, split_k * N, split_k, not isinstance(weight, ANSWeight)):
+        return False
     if input.dtype != torch.bfloat16 or (bias is not None and bias.dtype != torch.bfloat16) or not input.is_cuda:
         return False
     if input.size(1) != split_k * N or input.numel() >= 2 ** 31:
         return False
-    if not prefers_tiles(rows, M, split_k * N, split_k, not isinstance(weight, ANSWeight)):
-        return False
     return rows <= GEMM_MAX_ROWS or ((bias is None or tuple(bias.shape) == (M,)) and _fuses_above_32_rows(input, bias))
+
+
+def _tiled(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool:
+    return _takes(input, weight, bias, _ops.TILE_MIN_ROWS, _ops.TILE_MAX_ROWS, prefers_tiles)
+
+
+def _wide(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool:
+    return (_takes(input, weight, bias, _ops.WIDE_MIN_ROWS, _ops.WIDE_MAX_ROWS, prefers_wide)
+            and _ops._buffer(weight, 'rem').shape[1] % 64 == 0 and (input.size(0) + 15) * input.size(1) < 2 ** 31)
 
 
 def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], fused) -> Tensor:
@@ -881,14 +941,15 @@ def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tens
             output = fused(input)
             if bias is not None:
                 output += bias[None, :]
-    elif matrix_cores and rows > MAX_FUSED_BATCH and _tiled(input, weight, bias):
-        # 17..128 rows where the rule says so: as below, sixteen weight rows at a time
+    elif matrix_cores and rows > MAX_FUSED_BATCH and (
+            product := _ops.wide_bf16 if _wide(input, weight, bias) else _ops.tile_bf16 if _tiled(input, weight, bias) else None):
+        # 17..640 rows where the rules say so: as below, sixteen weight rows at a time
         x = (input if rows <= GEMM_MAX_ROWS else input.contiguous()).view(-1, split_k, N).contiguous()
         if x.data_ptr() % 16:
             x = x.clone()
         _check_weight_call(weight.rem, weight.exp, x)
         output = torch.empty((rows, M), dtype=torch.bfloat16, device=x.device)
-        _ops.tile_bf16(weight, x, output, None if bias is None else bias.detach().contiguous())
+        product(weight, x, output, None if bias is None else bias.detach().contiguous())
     elif wide or (rows <= GEMM_MAX_ROWS and matrix_cores):
         # up to 32 rows that neither the GEMV nor the tiled product takes: decode inside the matrix-core kernel,
         # no BF16 weight in memory
@@ -903,7 +964,7 @@ def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tens
 
 def linear_huffman(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor] = None) -> Tensor:
     """``F.linear`` with a :class:`HuffmanWeight`: fused kernels up to 32 rows and, where they are faster,
-    up to 128, else decode + dense GEMM (reference ``functional.py:390-411``)."""
+    up to 640, else decode + dense GEMM (reference ``functional.py:390-411``)."""
     def fused(x):
         b = weight._buffers          # without nn.Module's attribute lookups, a microsecond of the call
         try:

@@ -639,6 +639,39 @@ def tile_bf16(weight, X: Tensor, Y: Tensor, bias=None) -> None:
     _lib.check(rc, name)
 
 
+WIDE_MIN_ROWS, WIDE_MAX_ROWS = 17, 640
+WIDE_COUNTER_BYTES = 1024            # of a workspace of the wide product: one per row block of a product cut along K
+
+
+def wide_bf16(weight, X: Tensor, Y: Tensor, bias=None) -> None:
+    """``Y = X @ W.T (+ bias)`` for 17 to 640 rows of ``X`` with ``W`` held compressed (:class:`HuffmanWeight` or
+    :class:`ANSWeight`, ``M`` a multiple of 64): decoded into matrix operands in LDS, which the wavefronts of a block
+    share.  Arguments as :func:`gemm_bf16`; ``X`` in the kernel's order and the partial sums of K slices lie in a
+    workspace of the (device, stream) or of the capture (:mod:`.workspace`)."""
+    lib = _lib.load()
+    rem = _buffer(weight, "rem")
+    split_k, M, Ks = _weight_dims(rem, _buffer(weight, "offsets"))
+    if X.dim() != 3 or X.shape[1] != split_k or X.shape[2] != Ks:
+        raise RuntimeError(f"X must be [rows, {split_k}, {Ks}], got {tuple(X.shape)}")
+    rows = X.shape[0]
+    if tuple(Y.shape) != (rows, M):
+        raise RuntimeError(f"Y must be [{rows}, {M}], got {tuple(Y.shape)}")
+    member = (_lib.GemvMember * 1)()
+    x_ptr = _req(X, torch.bfloat16, "X", rem)
+    name = "wide_bf16_huffman" if _fill_member(member[0], weight, Y, bias, rem) else "wide_bf16_ans"
+    device = rem.device
+    stream = _stream(rem)
+    with _on_device(rem.get_device()):
+        need = int(lib.bhi_wide_workspace_bytes(split_k, M, Ks, rows))
+        if need < 0:
+            _lib.check(need, name)
+        ws = workspace("wide", device, stream, need, WIDE_COUNTER_BYTES)
+        rc = getattr(lib, "bhi_" + name)(member, x_ptr, split_k, Ks, rows, ws.data_ptr(), need, stream)
+        if rc != 0:
+            ws[:WIDE_COUNTER_BYTES].zero_()
+    _lib.check(rc, name)
+
+
 def gemm_bf16_grouped(weights, X: Tensor, Ys, biases=None, residuals=None) -> None:
     """:func:`gemm_bf16` for up to four weights of one class (Huffman or rANS) and one ``split_k`` / ``Ks``
     that multiply the same ``X``: one grid when their rows together are enough for the kernel to

@@ -221,6 +221,17 @@ int bhi_tile_bf16_ans(const bhi_gemv_member* weight, const void* X, int split_k,
                       void* workspace, int64_t workspace_bytes, void* stream);
 int64_t bhi_tile_workspace_bytes(int split_k, int M, int Ks, int batch);
 
+/* The product for 17..640 rows of X (no counterpart in the reference, as above): one weight with M a multiple
+ * of 64 and no residual, X aligned to 16 bytes, Y to 8.  The workspace (16-byte aligned, bhi_wide_workspace_bytes: 1 KiB of
+ * counters under the rules above, X in the kernel's order, partial sums) is always needed.  A bias is
+ * added as by the tiled product.  bhi_wide_slices: how many blocks along K share 64 weight rows. */
+int bhi_wide_bf16_huffman(const bhi_gemv_member* weight, const void* X, int split_k, int Ks, int batch,
+                          void* workspace, int64_t workspace_bytes, void* stream);
+int bhi_wide_bf16_ans(const bhi_gemv_member* weight, const void* X, int split_k, int Ks, int batch,
+                      void* workspace, int64_t workspace_bytes, void* stream);
+int64_t bhi_wide_workspace_bytes(int split_k, int M, int Ks, int batch);
+int bhi_wide_slices(int split_k, int M, int Ks);
+
 /* bhi_gemm_bf16_huffman without a workspace argument -- no counterpart in the reference.  For
  * callers that cannot allocate device memory at all (code under stream capture that has no
  * workspace yet, serving loops and harnesses that forbid it): the partial sums and counters

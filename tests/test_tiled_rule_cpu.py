@@ -81,3 +81,30 @@ def test_tiled_product_is_chosen_where_it_was_faster(M, K, rows, huffman, rans):
     split_k, = get_block_size_n(torch.empty(1, K, device="meta"))
     assert huffman is None or prefers_tiles(rows, M, K, split_k, True) == huffman
     assert rans is None or prefers_tiles(rows, M, K, split_k, False) == rans
+
+
+def test_wide_product_is_cut_while_every_block_has_a_unit():
+    """Slices divide the tasks of a row group and leave at most 256 blocks; the workspace holds counters, whole
+    tiles of X and, where K is cut, whole rounds of eight tiles per slice."""
+    from bf16_huffman_infer_amd import _lib
+    lib = _lib.load()
+    for split_k, M, Ks in [(1, 128, 128), (1, 1024, 4096), (3, 4096, 4096), (4, 3584, 4736), (1, 18944, 3584), (1, 12288, 4096),
+                           (2, 65536, 2048), (5, 3328, 1280), (12, 128, 1024)]:
+        per_group = split_k * lib.bhi_chunks_per_group(M, Ks, split_k)
+        slices = lib.bhi_wide_slices(split_k, M, Ks)
+        assert slices == max([1] + [d for d in range(2, 9) if per_group % d == 0 and M // 64 * d <= 256])
+        for rows in (17, 128, 129, 144, 145, 320, 321, 640):
+            tiles = -(-rows // 16)
+            want = 1024 + tiles * 16 * split_k * Ks * 2 + (-(-tiles // 8) * 8 * 16 * M * 4 * slices if slices > 1 else 0)
+            assert lib.bhi_wide_workspace_bytes(split_k, M, Ks, rows) == want
+        assert lib.bhi_wide_workspace_bytes(split_k, M, Ks, 16) < 0 and lib.bhi_wide_workspace_bytes(split_k, M, Ks, 641) < 0
+
+
+def test_wide_rule():
+    """Sides of the measured table: small layers and long prompts on half-empty units stay where they were."""
+    from bf16_huffman_infer_amd.functional import prefers_wide
+    assert [r for r in (32, 33, 64, 96, 256, 640) if prefers_wide(r, 12288, 4096)] == [96, 256, 640]
+    assert [r for r in (32, 33, 96, 256, 640) if prefers_wide(r, 4096, 12288, 3)] == [32, 33, 96, 256, 640]
+    assert [r for r in (33, 80, 81, 192, 193, 320, 321) if prefers_wide(r, 18944, 3584)] == [81, 192, 193, 320]
+    assert [r for r in (33, 80, 81, 192, 193, 320) if prefers_wide(r, 18944, 3584, 1, False)] == [81, 192]
+    assert not any(prefers_wide(r, 512, 1024) for r in (17, 33, 64, 128, 300, 640))
