@@ -60,6 +60,7 @@ _SIGNATURES = {
     "bhi_gemm_bf16_ans_grouped": (_i32, [ctypes.POINTER(GemvMember), _i32, _vp, _i32, _i32, _i32, _vp]),
     "bhi_split_planes": (_i32, [_vp, _vp, _vp, _i32, _i32, _i32, _vp]),
     "bhi_pair_histogram": (_i32, [_vp, _i64, _vp, _vp]),
+    "bhi_pair_code": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp]),
     "bhi_place_streams": (_i32, [_vp, _i64, _vp, _vp, _i64, _i32, _vp, _i64, _vp]),
     "bhi_tile_bf16_huffman": (_i32, [ctypes.POINTER(GemvMember), _vp, _i32, _i32, _i32, _vp, _i64, _vp]),
     "bhi_tile_bf16_ans": (_i32, [ctypes.POINTER(GemvMember), _vp, _i32, _i32, _i32, _vp, _i64, _vp]),

@@ -85,9 +85,201 @@ void place_streams_kernel(const uint4* __restrict__ streams, long long stride, c
     for (uint32_t i = threadIdx.x; i < n; i += kBlockThreads) words[start + i] = src[i];
 }
 
+// The pair code of a matrix (huffman.py, LUTHuffmanEncoder.build_lut): optimal code lengths of at most eleven bits for the
+// most frequent pairs and ESC (package-merge), for four cut-offs; the cheapest, or an escape-free one that costs at
+// most 1/32 more; canonical codes; the encoder's and the decoder's table.
+//
+// One block: 65536 counts, up to 1537 symbols, ten merges each of which needs the one before.  As Python lists
+// this was 6.2 of the 17.7 ms that converting a 12288x4096 weight took (18.3 -> 12.4 ms in turn with it).  A merge is parallel: an element's
+// place is its own index plus the number of elements of the other list in front of it (a binary search), and since the
+// first k elements of a merged list are its first a leaves and its first k - a packages, all that has to be kept
+// of a merge is where its leaves went.
+constexpr int kCodeThreads = 1024, kMaxCoded = 1536, kCodeSymbols = kMaxCoded + 1;
+constexpr uint32_t kEscIndex = 65536;
+constexpr int kEscSideBits = 32, kEscFreeShift = 5;
+
+// Elements of the ascending a[0..n) that are smaller than v (OR_EQUAL: or equal to it).
+template <bool OR_EQUAL>
+__device__ __forceinline__ int count_below(const unsigned long long* a, int n, unsigned long long v) {
+    int lo = 0, hi = n;
+    while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (OR_EQUAL ? a[mid] <= v : a[mid] < v) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// counts: descending, with ids[i] the pair of counts[i]; pairs of one count in ascending order.
+// info: expected bits, code length of ESC, whether pairs escape.
+__global__ __launch_bounds__(kCodeThreads)
+void pair_code_kernel(const unsigned long long* __restrict__ counts, const long long* __restrict__ ids, uint32_t* __restrict__ enc,
+                      uint32_t* __restrict__ dec, long long* __restrict__ info) {
+    __shared__ unsigned long long leaves[kCodeSymbols], list[2][2 * kCodeSymbols], packs[kCodeSymbols];
+    __shared__ uint16_t place[kTableBits][kCodeSymbols];                  // of every leaf in the list of a merge
+    __shared__ uint16_t rank_of[kCodeSymbols];                            // of symbol i among the leaves
+    __shared__ uint8_t lengths[2][kCodeSymbols];                          // of the cut-off at hand and of the best one
+    __shared__ uint16_t id_of[kMaxCoded];
+    __shared__ unsigned long long sums[2];
+    __shared__ uint32_t seen[4], chosen[kTableBits], per_length[kTableBits + 2], first_code[kTableBits + 2];
+    const int tid = threadIdx.x;
+    if (tid < 2) sums[tid] = 0;
+    if (tid < 4) seen[tid] = 0;
+    __syncthreads();
+    {
+        const unsigned long long least[4] = {1, 2, 4, 16};
+        unsigned long long sum = 0;
+        uint32_t n[4] = {0, 0, 0, 0};
+        for (int i = tid; i < 65536; i += kCodeThreads) {
+            const unsigned long long c = counts[i];
+            sum += c;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) n[k] += c >= least[k] ? 1 : 0;
+        }
+        atomicAdd(&sums[0], sum);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) atomicAdd(&seen[k], n[k]);
+    }
+    for (int i = tid; i < kMaxCoded; i += kCodeThreads) id_of[i] = (uint16_t)ids[i];
+    for (int i = tid; i <= (int)kEscIndex; i += kCodeThreads) enc[i] = 0;
+    __syncthreads();
+    const unsigned long long total = sums[0];
+    const int present = (int)seen[0];
+
+    unsigned long long best_bits = 0, free_bits = 0;
+    int best = 0, last = 0, all_coded = 0;                                // symbols without ESC; 0: none yet
+    unsigned long long best_escapes = 0;
+    for (int cut = 0; cut < 4; ++cut) {
+        int m = min((int)seen[cut], kMaxCoded);
+        if (m == 0) m = 1;
+        if (m == last) continue;
+        last = m;
+        const int n = m + 1;
+        __syncthreads();
+        if (tid == 0) sums[1] = 0;
+        __syncthreads();
+        unsigned long long part = 0;
+        for (int i = tid; i < m; i += kCodeThreads) part += counts[i];
+        atomicAdd(&sums[1], part);
+        __syncthreads();
+        const unsigned long long escapes = total - sums[1], esc = escapes > 1 ? escapes : 1;
+        __syncthreads();
+        // leaves in ascending order, of one weight in the order of the symbols: ESC is the last symbol
+        for (int i = tid; i < m; i += kCodeThreads) packs[m - 1 - i] = counts[i];              // ascending
+        __syncthreads();
+        for (int i = tid; i < n; i += kCodeThreads) {
+            int r;
+            unsigned long long w;
+            if (i < m) {
+                w = packs[m - 1 - i];
+                const int below = count_below<false>(packs, m, w), up_to = count_below<true>(packs, m, w);
+                r = below + (i - (m - up_to)) + (esc < w ? 1 : 0);
+            } else {
+                w = esc;
+                r = count_below<true>(packs, m, esc);
+            }
+            rank_of[i] = (uint16_t)r;
+            leaves[r] = w;
+        }
+        __syncthreads();
+        for (int i = tid; i < n; i += kCodeThreads) list[0][i] = leaves[i];
+        int len = n, from = 0;
+        for (int merge = 1; merge < kTableBits; ++merge) {
+            __syncthreads();
+            const int half = len / 2;
+            for (int j = tid; j < half; j += kCodeThreads) packs[j] = list[from][2 * j] + list[from][2 * j + 1];
+            __syncthreads();
+            for (int i = tid; i < n; i += kCodeThreads) {                 // a leaf in front of packages of its weight
+                const int at = i + count_below<false>(packs, half, leaves[i]);
+                place[merge][i] = (uint16_t)at;
+                list[from ^ 1][at] = leaves[i];
+            }
+            for (int j = tid; j < half; j += kCodeThreads) list[from ^ 1][j + count_below<true>(leaves, n, packs[j])] = packs[j];
+            from ^= 1;
+            len = n + half;
+        }
+        __syncthreads();
+        if (tid == 0) {                                                   // leaves among the elements taken from every list
+            int k = 2 * n - 2;
+            for (int merge = kTableBits - 1; merge > 0; --merge) {
+                int lo = 0, hi = n;
+                while (lo < hi) {
+                    const int mid = (lo + hi) / 2;
+                    if (place[merge][mid] < k) lo = mid + 1;
+                    else hi = mid;
+                }
+                chosen[merge] = (uint32_t)lo;
+                k = 2 * (k - lo);
+            }
+            chosen[0] = (uint32_t)k;
+            sums[1] = 0;
+        }
+        __syncthreads();
+        part = 0;
+        for (int i = tid; i < n; i += kCodeThreads) {
+            uint32_t bits = 0;
+#pragma unroll
+            for (int merge = 0; merge < kTableBits; ++merge) bits += rank_of[i] < chosen[merge] ? 1 : 0;
+            lengths[0][i] = (uint8_t)bits;
+            part += i < m ? counts[i] * bits : escapes * (bits + kEscSideBits);
+        }
+        atomicAdd(&sums[1], part);
+        __syncthreads();
+        const unsigned long long bits = sums[1];
+        if (m == present) {                                               // the first cut-off, if any
+            all_coded = m;
+            free_bits = bits;
+        }
+        // an escape-free code stays unless a later one is cheaper by more than 1/32
+        const bool taken = best == 0 || bits < best_bits;
+        if (taken) best_bits = bits;
+        if (best == 0 || (taken && !(all_coded && free_bits <= best_bits + (best_bits >> kEscFreeShift)))) {
+            best = m;
+            best_escapes = escapes;
+            for (int i = tid; i < n; i += kCodeThreads) lengths[1][i] = lengths[0][i];
+        }
+    }
+    // canonical codes: shorter first, of one length in the order of the ids, ESC last
+    __syncthreads();
+    const int n = best + 1;
+    if (tid < kTableBits + 2) per_length[tid] = 0;
+    __syncthreads();
+    for (int i = tid; i < n; i += kCodeThreads) atomicAdd(&per_length[lengths[1][i]], 1u);
+    __syncthreads();
+    if (tid == 0) {
+        uint32_t code = 0;
+        for (int l = 1; l <= kTableBits; ++l) {
+            code = (code + per_length[l - 1]) << 1;
+            first_code[l] = code;
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += kCodeThreads) {
+        const uint32_t l = lengths[1][i], id = i < best ? id_of[i] : kEscIndex;
+        uint32_t before = 0;
+        for (int j = 0; j < best; ++j) before += lengths[1][j] == l && id_of[j] < id ? 1 : 0;
+        const uint32_t reversed = __brev(first_code[l] + before) >> (32 - l);
+        enc[id] = reversed | l << 16;
+        const uint32_t entry = l | (id == kEscIndex ? kEscFlag : (id & 0xFFu) << 7 | (id >> 8) << 23);
+        for (uint32_t at = reversed; at < (uint32_t)kTableEntries; at += 1u << l) dec[at] = entry;
+    }
+    if (tid == 0) {
+        info[0] = (long long)(all_coded && best == all_coded ? free_bits : best_bits);
+        info[1] = lengths[1][best];
+        info[2] = best_escapes > 0 ? 1 : 0;
+    }
+}
+
 }  // namespace bhi
 
 using namespace bhi;
+
+extern "C" int bhi_pair_code(const void* counts, const void* ids, void* enc, void* dec, void* info, void* stream) {
+    if (!counts || !ids || !enc || !dec || !info) return bhi_fail(BHI_EINVAL, "null pointer");
+    hipLaunchKernelGGL(pair_code_kernel, dim3(1), dim3(kCodeThreads), 0, (hipStream_t)stream, (const unsigned long long*)counts,
+                       (const long long*)ids, (uint32_t*)enc, (uint32_t*)dec, (long long*)info);
+    return bhi_launch_status("pair_code");
+}
 
 extern "C" int bhi_split_planes(const void* W, void* rem, void* exp, int split_k, int M, int Ks, void* stream) {
     if (!W || !rem || !exp) return bhi_fail(BHI_EINVAL, "null pointer");

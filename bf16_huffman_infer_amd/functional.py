@@ -196,7 +196,7 @@ class HuffmanWeight(nn.Module):
     def _codec_of(cls, counts: Tensor) -> LUTHuffmanEncoder:
         """The code for int64 ``[65536]`` pair counts."""
         codec = LUTHuffmanEncoder()
-        codec.build_lut(counts.cpu())
+        codec.build_lut(counts)
         return codec
 
     @staticmethod

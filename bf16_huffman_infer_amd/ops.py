@@ -312,6 +312,22 @@ def pair_histogram(exp: Tensor) -> Tensor:
     return counts
 
 
+def pair_code(counts: Tensor):
+    """The pair code for int64 ``[65536]`` counts on the GPU, at least one of them positive: (encoder's table int32
+    ``[65537]``, decoder's int32 ``[2048]``, int64 ``[3]``: expected bits, code length of ESC, whether pairs
+    escape), as :meth:`.huffman.LUTHuffmanEncoder.build_lut` lays them out."""
+    if counts.numel() != 65536:
+        raise RuntimeError("counts must hold 65536 entries")
+    values, ids = torch.sort(counts.flatten(), descending=True, stable=True)
+    enc = torch.empty(65537, dtype=torch.int32, device=counts.device)
+    dec = torch.empty(2048, dtype=torch.int32, device=counts.device)
+    info = torch.empty(3, dtype=torch.int64, device=counts.device)
+    with _on_device(counts.get_device()):
+        _lib.check(_lib.load().bhi_pair_code(_req(values, torch.int64, "counts"), ids.data_ptr(), enc.data_ptr(), dec.data_ptr(),
+                                             info.data_ptr(), _stream(counts)), "pair_code")
+    return enc, dec, info
+
+
 def place_streams(streams: Tensor, lengths: Tensor, starts: Tensor, words: Tensor) -> None:
     """Copies the first ``lengths[i]`` words of row ``i`` of ``streams`` to ``words[starts[i]:]``; ``starts`` is
     int64 ``[n]`` of any stride."""

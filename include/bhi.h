@@ -260,9 +260,13 @@ int bhi_gemm_workspace_reset(void* workspace, int64_t workspace_bytes, void* str
  * 1's, ... as the encoders take them.  bhi_pair_histogram: adds the occurrences of every pair of
  * neighbouring bytes to counts int64 [65536] (index first | second << 8).  bhi_place_streams: copies the
  * first lengths[i] (int32) words of row i of streams int32 [n_tasks, stride] to words + starts[i *
- * starts_stride] (int64); a row that does not fit words int32 [n_words] is left out. */
+ * starts_stride] (int64); a row that does not fit words int32 [n_words] is left out.
+ * bhi_pair_code: the pair code for 65536 counts, sorted: counts int64 [65536] descending, ids int64 the pair of each
+ * (ascending within a count), at least one count positive -> enc int32 [65537] as bhi_huffman_encode takes it,
+ * dec int32 [2048] (LUT1), info int64 [3]: expected bits, code length of ESC, whether pairs escape. */
 int bhi_split_planes(const void* W, void* rem, void* exp, int split_k, int M, int Ks, void* stream);
 int bhi_pair_histogram(const void* exp, int64_t bytes, void* counts, void* stream);
+int bhi_pair_code(const void* counts, const void* ids, void* enc, void* dec, void* info, void* stream);
 int bhi_place_streams(const void* streams, int64_t stride, const void* lengths, const void* starts, int64_t starts_stride,
                       int n_tasks, void* words, int64_t n_words, void* stream);
 

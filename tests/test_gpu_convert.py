@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from helpers import gaussian_weight, random_bits_weight
+from helpers import gaussian_weight, random_bits_weight, student_t_weight
 
 pytestmark = pytest.mark.gpu
 
@@ -127,3 +127,44 @@ def test_convert_compares_with_the_layer_itself(cuda):
     on_gpu.weight.data.copy_(w)
     module = convert(on_gpu, "layer")
     assert type(module) is CompressedLinear and not on_gpu.weight.is_cuda and torch.equal(on_gpu.weight.data, w)
+
+
+def _count_sets():
+    g = torch.Generator().manual_seed(11)
+    at = torch.randperm(65536, generator=g)
+    spread = (torch.rand(65536, generator=g).double() ** -3).clamp(max=1e9).long()
+    yield "one pair", torch.zeros(65536).long().index_fill(0, at[:1], 5)
+    yield "one pair, once", torch.zeros(65536).long().index_fill(0, at[:1], 1)
+    yield "two pairs of one count", torch.zeros(65536).long().index_fill(0, at[:2], 7)
+    for n in (3, 64, 65, 1000, 1535, 1536, 1537, 1538, 4000, 65536):
+        counts = torch.zeros(65536).long()
+        counts[at[:n]] = spread[at[:n]]
+        yield f"{n} pairs", counts
+        counts = counts.clone()
+        counts[at[:n]] = 1 + spread[at[:n]] % 3
+        yield f"{n} pairs of three counts", counts
+    yield "all once", torch.ones(65536).long()
+    steep = torch.zeros(65536).long()
+    steep[at[:40]] = 1 << torch.arange(40)                       # beyond 32 bits, far beyond eleven levels
+    yield "powers of two", steep
+    steep = steep.clone()
+    steep[at[40:3000]] = 1
+    yield "powers of two and a tail", steep
+
+
+def test_pair_code_on_the_gpu_is_the_host_one(cuda):
+    from bf16_huffman_infer_amd.huffman import LUTHuffmanEncoder
+    weights = [student_t_weight(256, 1024, seed=5), gaussian_weight(1024, 1024, seed=6)]
+    sets = list(_count_sets())
+    for w in weights:
+        e = ((w.view(torch.int16).int() >> 7) & 0xFF)
+        sets.append(("a weight", torch.bincount((e[:, 0::2] | e[:, 1::2] << 8).flatten(), minlength=65536)))
+    for name, counts in sets:
+        here, there = LUTHuffmanEncoder(), LUTHuffmanEncoder()
+        here.build_lut(counts)
+        there.build_lut(counts.cuda())
+        assert (here.enc_table == there.enc_table).all() and (here.dec_table == there.dec_table).all(), name
+        assert (here.code_lengths == there.code_lengths).all() and here.expected_bits == there.expected_bits, name
+    for refused in (torch.zeros(65536).long(), -torch.ones(65536).long(), torch.ones(100).long()):
+        with pytest.raises(AssertionError):
+            LUTHuffmanEncoder().build_lut(refused.cuda())
