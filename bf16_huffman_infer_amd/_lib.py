@@ -69,6 +69,7 @@ _SIGNATURES = {
     "bhi_wide_bf16_ans": (_i32, [ctypes.POINTER(GemvMember), _vp, _i32, _i32, _i32, _vp, _i64, _vp]),
     "bhi_wide_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32]),
     "bhi_wide_slices": (_i32, [_i32, _i32, _i32]),
+    "bhi_prefers_matrix_cores": (_i32, [_i32, _i32, _i32]),
     "bhi_gemm_workspace_bytes": (_i64, [_i32, _i32, _i32, _i32]),
     "bhi_gemm_bf16_huffman_static": (_i32, [ctypes.POINTER(GemvMember), _vp, _i32, _i32, _i32, _vp]),
     "bhi_gemm_static_workspace_bytes": (_i64, []),
@@ -108,6 +109,25 @@ def load() -> ctypes.CDLL:
             raise RuntimeError("bhi_gemv_member of the library and of the binding differ: rebuild the library")
         _lib = lib
     return _lib
+
+
+_eager = None
+
+
+def eager():
+    """The native step of eager calls (``csrc/bhi_torch.cpp``), which gets its entry points from :func:`load`."""
+    global _eager
+    if _eager is None:
+        lib = load()
+        try:
+            from . import _bhi_torch
+        except ImportError as e:
+            raise RuntimeError("_bhi_torch.so is missing or does not fit this torch: build the extension first "
+                               "(python -m bf16_huffman_infer_amd.csrc.build)") from e
+        _bhi_torch.bind(*(ctypes.cast(f, _vp).value for f in (lib.bhi_gemv_bf16_huffman_grouped, lib.bhi_gemv_bf16_ans_grouped,
+                                                              lib.bhi_prefers_matrix_cores)))
+        _eager = _bhi_torch
+    return _eager
 
 
 def check(rc: int, what: str) -> None:

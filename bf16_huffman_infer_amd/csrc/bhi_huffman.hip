@@ -230,6 +230,8 @@ extern "C" int64_t bhi_gemm_workspace_bytes(int split_k, int M, int Ks, int batc
     return mma_workspace_bytes(s, batch);
 }
 
+extern "C" int bhi_prefers_matrix_cores(int rows, int M, int K) { return mma_prefers(rows, M, K); }
+
 extern "C" int64_t bhi_tile_workspace_bytes(int split_k, int M, int Ks, int batch) {
     Shape s;
     if (batch < kTileMinBatch || batch > kTileMaxBatch) return bhi_fail(BHI_EBATCH, "the tiled product takes 17 to 128 rows of X");

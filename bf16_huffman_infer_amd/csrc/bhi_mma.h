@@ -434,6 +434,15 @@ static inline bhi::Shape mma_group_shape(const bhi::Shape& first, long long rows
     return s;
 }
 
+// Rows of X (at most eight) from which a layer goes through this kernel rather than the GEMV (both sides measured: the
+// table in functional.prefers_matrix_cores).
+static inline bool mma_prefers(int rows, int M, int K) {
+    if (rows >= 8 && K >= 11008) return true;
+    if (rows >= 6 && ((M >= 10240 && K >= 3584) || K >= 14336)) return true;
+    if (rows >= 4 && (K >= 16384 || (M >= 14336 && K >= 4096))) return true;
+    return rows >= 3 && M >= 32768 && K >= 3584;
+}
+
 // One member of a launch from the caller's description of it, not cut along K.
 static inline int fill_mma_member(bhi::MmaArgs& a, const bhi_gemv_member& m, int split_k, int Ks, int batch,
                                   int64_t table_bytes_expected, bool header_is_table) {

@@ -10,6 +10,8 @@ PKG = os.path.dirname(HERE)
 SOURCES = ["bhi_api.hip", "bhi_huffman.hip", "bhi_ans.hip", "bhi_nibble.hip", "bhi_reference.hip", "bhi_attention.hip",
            "bhi_convert.hip"]
 LIB = os.path.join(PKG, "libbhi_hip.so")
+TORCH_SOURCE = "bhi_torch.cpp"                       # host code alone: compiled against torch and Python, links no kernel
+TORCH_LIB = os.path.join(PKG, "_bhi_torch.so")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
@@ -44,6 +46,22 @@ def build(verbose: bool = True, defines=(), lib: str = LIB) -> str:
     return lib
 
 
+def build_torch(verbose: bool = True, lib: str = TORCH_LIB) -> str:
+    import sysconfig
+
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+          "-isystem", os.path.join(root, "include"), "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+          "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
+          os.path.join(HERE, TORCH_SOURCE), "-o", lib, "-L" + os.path.join(root, "lib"),
+          "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"], verbose)
+    return lib
+
+
 if __name__ == "__main__":
     build()
+    build_torch()
     sys.exit(0)

@@ -775,13 +775,7 @@ def prefers_matrix_cores(rows: int, M: int, K: int) -> bool:
     rows; 37888x3584: 39.1 / 39.6, 41.9 / 39.7, 44.4 / 39.8, 58.7 / 48.9).  The rANS kernels cross over
     at the same places (18944x3584 at 6 rows 37.7 / 36.0, 3584x18944 at 4 rows 34.7 / 33.9,
     37888x3584 at 3 rows 53.6 / 51.2)."""
-    if rows >= 8 and K >= 11008:
-        return True
-    if rows >= 6 and ((M >= 10240 and K >= 3584) or K >= 14336):
-        return True
-    if rows >= 4 and (K >= 16384 or (M >= 14336 and K >= 4096)):
-        return True
-    return rows >= 3 and M >= 32768 and K >= 3584
+    return bool(_lib.load().bhi_prefers_matrix_cores(rows, M, K))
 
 
 @functools.lru_cache(maxsize=1024)        # an eager call asks every time
@@ -962,9 +956,20 @@ def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tens
     return output if len(shape) == 2 else output.unflatten(0, shape[:-1])
 
 
+def _eager(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], huffman: bool) -> Optional[Tensor]:
+    """A call of the GEMV that nothing watches, in one native step (``bhi_torch.cpp``); None where the path through the
+    custom ops has to take it or to refuse it."""
+    if torch.compiler.is_compiling():
+        return None
+    return _lib.eager().linear(input, getattr(weight, '_buffers', None), bias, huffman)
+
+
 def linear_huffman(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor] = None) -> Tensor:
     """``F.linear`` with a :class:`HuffmanWeight`: fused kernels up to 32 rows and, where they are faster,
     up to 640, else decode + dense GEMM (reference ``functional.py:390-411``)."""
+    if (output := _eager(input, weight, bias, True)) is not None:
+        return output
+
     def fused(x):
         b = weight._buffers          # without nn.Module's attribute lookups, a microsecond of the call
         try:
@@ -978,6 +983,9 @@ def linear_huffman(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor] 
 
 def linear_ans(input: Tensor, weight: ANSWeight, bias: Optional[Tensor] = None) -> Tensor:
     """rANS counterpart of :func:`linear_huffman` (reference ``functional.py:447-466``)."""
+    if (output := _eager(input, weight, bias, False)) is not None:
+        return output
+
     def fused(x):
         b = weight._buffers          # as above
         try:

@@ -210,6 +210,9 @@ int bhi_gemm_bf16_ans_grouped(const bhi_gemv_member* members, int n_members, con
 /* Workspace bytes a call with these dimensions needs (0: none); negative on a rejected shape. */
 int64_t bhi_gemm_workspace_bytes(int split_k, int M, int Ks, int batch);
 
+/* Whether up to eight rows of X are faster through the product above than through the GEMV (0 or 1). */
+int bhi_prefers_matrix_cores(int rows, int M, int K);
+
 /* The product for 17..128 rows of X (no counterpart in the reference, which decodes to a BF16 matrix
  * and calls a dense GEMM): one weight as above, workspace under the same rules, its size from
  * bhi_tile_workspace_bytes (1 KiB of counters, then partial sums).  Above 32 rows a bias is added
