@@ -21,19 +21,20 @@
 // Measured on MI355X in recorded graphs (four to twelve copies of a weight in turn, us, before / now; before:
 // tile_kernel up to 128 rows where its rule takes it, decoding and library GEMM else):
 //
-//   M x K               33 rows      64 rows      96 rows      128 rows     192 rows     320 rows     512 rows
-//   4096x4096   Huff    18.5 / 18.1  20.5 / 18.8  25.0 / 21.5  28.3 / 22.9  40.0 / 28.6  36.1 / 36.0  40.9 / 45.0
-//   4608x3584   rANS    23.0 / 23.6  25.8 / 24.4  32.1 / 25.9  33.9 / 27.4  39.5 / 31.1  36.3 / 38.3  43.9 / 48.4
-//   12288x4096  Huff    31.7 / 34.0  35.6 / 35.6  42.7 / 37.0  47.5 / 40.7  69.9 / 45.8  79.3 / 55.5  84.7 / 77.6
-//   12288x4096  rANS    39.8 / 41.3  43.5 / 42.8  53.4 / 44.0  55.6 / 45.5  71.2 / 53.1  79.1 / 62.0  89.0 / 82.3
-//   4096x12288  Huff    35.4 / 34.0  40.1 / 35.5  48.8 / 38.7  57.2 / 42.3   103 / 50.3  91.3 / 64.0   105 / 80.9
-//   18944x3584  Huff    40.5 / 51.8  45.2 / 54.8  61.4 / 57.1  65.9 / 62.0  80.1 / 71.7  90.8 / 86.1   109 / 122
-//   3584x18944  Huff    53.8 / 41.2  59.8 / 44.1  65.1 / 47.0  68.0 / 51.8   131 / 62.2   142 / 75.2   212 / 102
-//   8192x8192   rANS    64.4 / 45.8  68.6 / 48.6  68.9 / 50.5  72.5 / 52.7  93.9 / 62.2  98.2 / 75.5   111 / 98.6
+//   M x K               33 rows      64 rows      96 rows      128 rows     192 rows     300 rows     512 rows
+//   4096x4096   Huff    18.6 / 18.1  20.4 / 18.3  24.9 / 21.6  28.9 / 22.7  40.1 / 28.1  35.8 / 33.4  41.7 / 45.0
+//   12288x4096  Huff    32.1 / 33.9  35.8 / 35.5  42.9 / 36.9  47.9 / 39.7  70.9 / 45.8  77.6 / 51.7  86.0 / 70.7
+//   12288x4096  rANS    41.0 / 42.7  43.6 / 43.7  54.7 / 44.3  56.9 / 45.4  72.5 / 50.2  80.8 / 58.5  90.5 / 76.7
+//   4096x12288  Huff    36.3 / 33.4  40.9 / 35.1  49.5 / 38.2  58.0 / 41.5   103 / 51.7  92.4 / 61.1   111 / 84.5
+//   18944x3584  Huff    41.9 / 52.4  45.6 / 54.9  61.6 / 56.6  66.3 / 63.1  79.4 / 73.5  95.4 / 87.0   110 / 118
+//   3584x18944  Huff    54.3 / 40.7  60.9 / 43.4  65.6 / 47.9  69.1 / 51.6   130 / 61.7   138 / 77.9   213 / 101
+//   8192x8192   rANS    65.7 / 44.6  69.4 / 46.5  71.0 / 49.8  73.2 / 51.5  96.5 / 58.6   103 / 74.8   117 / 100
 //
 // (functional.prefers_wide picks the sides.)  What bounds it now: up to 9 tiles the LDS pipe (lookups and weight reads,
-// 0.8 us a step), from 20 tiles on the loads of X, which every block reads whole (0.057 us per tile and step, 30
-// bytes a clock and unit), and the units without a block: 18944 rows are 296 blocks on 256 units.
+// 0.8 us a step), from 20 tiles on the loads of X, which every block reads whole (0.041 us per tile and step, 41
+// bytes a clock and unit; 0.057 us while a tile of X was one piece of memory, whose chunks all fell on the
+// same channels of the cache: 640 rows of 12288x4096 92 us instead of 84), and the units without a block: 18944
+// rows are 296 blocks on 256 units.
 #pragma once
 // (included by bhi_task.h users after bhi_tile.h, whose argument block and workspace rules it shares)
 
@@ -129,12 +130,12 @@ __device__ __forceinline__ void decode_wide(AnsCursor (&cur)[kWideGroups], const
     pair(std::integral_constant<int, 3>{});
 }
 
-// X in the order the matrix instructions take it: 1 KB per tile of sixteen rows and chunk of 32 columns (about 2.5 us: its
-// launch).  Rows past the batch repeat its last row.
-static __global__ __launch_bounds__(256) void pack_x_kernel(const uint16_t* __restrict__ X, u32x4v_t* __restrict__ out, int rows, int K, int pieces) {
+// X in the order the matrix instructions take it: 1 KB per tile of sixteen rows and chunk of 32 columns, the tiles of
+// a chunk side by side (about 2.5 us: its launch).  Rows past the batch repeat its last row.
+static __global__ __launch_bounds__(256) void pack_x_kernel(const uint16_t* __restrict__ X, u32x4v_t* __restrict__ out, int rows, int K, int tiles) {
     const int piece = (int)(blockIdx.x * 4 + threadIdx.x / kLanes), lane = threadIdx.x & (kLanes - 1);
-    if (piece >= pieces) return;
-    const int per_tile = K / 32, tile = piece / per_tile, chunk = piece % per_tile;
+    const int tile = piece % tiles, chunk = piece / tiles;
+    if (chunk >= K / 32) return;
     const int r = tile * kTileBatch + (lane & 15);
     out[(size_t)piece * kLanes + lane] = *(const u32x4v_t*)(X + (size_t)(r < rows ? r : rows - 1) * K + chunk * 32 + 8 * (lane >> 4));
 }
@@ -176,11 +177,11 @@ void wide_kernel(const uint16_t* __restrict__ X, const WideArgs wa) {
     }
 
     // buffer loads: place of tile and chunk as a scalar offset
-    const uint32_t tile_bytes = (uint32_t)K * (kTileBatch * 2u);
-    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, (int)(tile_bytes * (uint32_t)wa.tiles), 0x00020000);
+    const uint32_t chunk_bytes = (uint32_t)wa.tiles * 1024u;
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc((void*)X, 0, (int)(chunk_bytes * (uint32_t)(K / 32)), 0x00020000);
     uint32_t x_tile[NT];
 #pragma unroll
-    for (int n = 0; n < NT; ++n) x_tile[n] = (uint32_t)min(tile0 + n * kParts, wa.tiles - 1) * tile_bytes;
+    for (int n = 0; n < NT; ++n) x_tile[n] = (uint32_t)min(tile0 + n * kParts, wa.tiles - 1) * 1024u;
 
     // lane 4 b + i of a group's stream holds row i and columns 8 b .. 8 b + 7; the operand of a chunk of 32 columns wants
     // row r of sixteen and columns 8 q .. in lane 16 q + r.  Rows of odd q are stored four places on, so that eight
@@ -207,7 +208,7 @@ void wide_kernel(const uint16_t* __restrict__ X, const WideArgs wa) {
         auto x_load = [&](uint32_t x0, int c) __attribute__((always_inline)) {
 #pragma unroll
             for (int n = 0; n < N; ++n)
-                xf[c][n] = __builtin_amdgcn_raw_buffer_load_b128(xr, lane * 16 + c * 1024, (int)(x_tile[n] + x0), 0);
+                xf[c][n] = __builtin_amdgcn_raw_buffer_load_b128(xr, lane * 16, (int)(x_tile[n] + x0 + (uint32_t)c * chunk_bytes), 0);
         };
         auto fetch = [&](u32x4v_t (&f)[kQuads], int from, int c) __attribute__((always_inline)) {
 #pragma unroll
@@ -263,7 +264,7 @@ void wide_kernel(const uint16_t* __restrict__ X, const WideArgs wa) {
             for (int g = 0; g < kWideGroups; ++g) pending[g] = false;
             // step t is decoded while step t - 1 is multiplied
             auto one = [&](int i, int t) __attribute__((always_inline)) {
-                const uint32_t x_now = (uint32_t)(id.k * s.Ks + (id.t0 + t) * kStepCols) * (kTileBatch * 2u);
+                const uint32_t x_now = (uint32_t)(id.k * s.steps + id.t0 + t) * kWideChunks * chunk_bytes;
                 u32x4v_t f[2][kQuads];
                 fetch(f[0], par ^ 1, 0);
                 uint32_t lo[kWideGroups], hi[kWideGroups], nx[kWideGroups];
@@ -460,7 +461,7 @@ static inline int launch_wide(const bhi_gemv_member* weight, const void* X, int 
     a.partial = (float*)(packed + packed_bytes);
     const int K = split_k * Ks, pieces = wa.tiles * (K / 32);
     hipLaunchKernelGGL(pack_x_kernel, dim3((unsigned)((pieces + 3) / 4)), dim3(256), 0, stream, (const uint16_t*)X, (u32x4v_t*)packed,
-                       batch, K, pieces);
+                       batch, K, wa.tiles);
     const uint16_t* x = (const uint16_t*)packed;
     if (wide_split(wa.tiles, Codec::kHuffman) == 2) {
         switch ((wa.tiles + kWideWaves / 2 - 1) / (kWideWaves / 2)) {
