@@ -124,8 +124,9 @@ def eager():
         except ImportError as e:
             raise RuntimeError("_bhi_torch.so is missing or does not fit this torch: build the extension first "
                                "(python -m bf16_huffman_infer_amd.csrc.build)") from e
-        _bhi_torch.bind(*(ctypes.cast(f, _vp).value for f in (lib.bhi_gemv_bf16_huffman_grouped, lib.bhi_gemv_bf16_ans_grouped,
-                                                              lib.bhi_prefers_matrix_cores)))
+        _bhi_torch.bind(*(ctypes.cast(f, _vp).value for f in (
+            lib.bhi_gemv_bf16_huffman_grouped, lib.bhi_gemv_bf16_ans_grouped, lib.bhi_huffman_decode, lib.bhi_ans_decode,
+            lib.bhi_prefers_matrix_cores)))
         _eager = _bhi_torch
     return _eager
 

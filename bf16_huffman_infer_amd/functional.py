@@ -181,6 +181,8 @@ class HuffmanWeight(nn.Module):
 
     def get_weight(self) -> Tensor:
         """The original BF16 weight, bit for bit."""
+        if (weight := _eager_weight(self, True)) is not None:
+            return weight
         weight = self._empty_weight()
         huffman_decode(self.rem, self.exp, weight, self.offsets,
                        self.LUT1, self.LUT2, self.LUT3, self.LUT4, self.code_lengths)
@@ -312,6 +314,8 @@ class ANSWeight(HuffmanWeight):
         return linear_ans(*args, **(kwargs or {}))
 
     def get_weight(self) -> Tensor:
+        if (weight := _eager_weight(self, False)) is not None:
+            return weight
         weight = self._empty_weight()
         ans_decode(self.rem, self.exp, weight, self.offsets, self.LUT)
         return weight
@@ -962,6 +966,13 @@ def _eager(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], huffman
     if torch.compiler.is_compiling():
         return None
     return _lib.eager().linear(input, getattr(weight, '_buffers', None), bias, huffman)
+
+
+def _eager_weight(weight: HuffmanWeight, huffman: bool) -> Optional[Tensor]:
+    """The same for a weight that is decoded."""
+    if torch.compiler.is_compiling():
+        return None
+    return _lib.eager().weight(getattr(weight, '_buffers', None), huffman)
 
 
 def linear_huffman(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor] = None) -> Tensor:

@@ -99,3 +99,21 @@ def test_recorded_and_replayed(cuda):
             y.zero_()
             graph.replay()
             assert torch.equal(y, want) and torch.equal(lin(x), want)
+
+
+@pytest.mark.parametrize("algo", ["huffman", "ans"])
+def test_weight_back_in_one_step(cuda, algo):
+    from bf16_huffman_infer_amd.functional import _eager_weight
+    weight, huffman = _layer(algo).weight, algo == "huffman"
+    weight.get_weight()                                    # the library's first use of the device
+    want = gaussian_weight(384, 1024, seed=384)
+    y = _eager_weight(weight, huffman)
+    assert torch.equal(y.cpu().view(torch.int16), want.view(torch.int16)) and not y.requires_grad
+    with torch.device("cuda"):                             # a function mode: the custom op
+        assert _eager_weight(weight, huffman) is None and torch.equal(weight.get_weight(), y)
+    taken = []
+    torch.func.vmap(lambda v: (taken.append(_eager_weight(weight, huffman)), v)[1])(y)
+    assert taken == [None]
+    assert _eager_weight(_layer(algo).weight.cpu(), huffman) is None
+    del weight._buffers["exp"]
+    assert _eager_weight(weight, huffman) is None
