@@ -142,6 +142,18 @@ def test_split_edges(cuda, q_heads, kv_heads, max_len, positions):
         assert err <= 1.0, (p, err)
 
 
+@pytest.mark.parametrize("q_heads,kv_heads", [(28, 4), (16, 16)])
+@pytest.mark.parametrize("positions", [(128, 129, 143, 144, 191), (4095, 4096, 4143, 4144, 5999, 6143, 6144)])
+def test_shares_of_three_tiles(cuda, q_heads, kv_heads, positions):
+    """Splits of 129 to 192 slots: a wavefront has three matrix tiles, the last block's fewer or a part of one."""
+    from bf16_huffman_infer_amd import ops
+    qk, v, kc, vc, cos, sin = _case(q_heads, kv_heads, 8192, q_heads)
+    for p in positions:
+        err = _step_error(qk, v, cos, sin, p, kc, vc, q_heads, kv_heads,
+                          lambda pos: ops.decode_attention(qk, v, None, cos, sin, pos, kc, vc, eps=1e-6))
+        assert err <= 1.0, (p, err)
+
+
 @pytest.mark.parametrize("q_heads,kv_heads,max_len,positions", [(28, 4, 8192, (0, 63, 64, 255, 256, 257, 5000)), (3, 3, 300, (299,))])
 def test_entry_without_workspace(cuda, q_heads, kv_heads, max_len, positions):
     """The C entry that takes no workspace walks all slots in one block per q head."""
