@@ -962,15 +962,18 @@ def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tens
 
 def _eager(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], huffman: bool) -> Optional[Tensor]:
     """A call of the GEMV that nothing watches, in one native step (``bhi_torch.cpp``); None where the path through the
-    custom ops has to take it or to refuse it."""
-    if torch.compiler.is_compiling():
+    custom ops has to take it or to refuse it.  Whoever has put a wrapper in the place of this module's ops (to
+    count or to log calls) watches too."""
+    if torch.compiler.is_compiling() or gemv_bf16_grouped is not _ops.gemv_bf16_grouped or not (
+            gemv_bf16_huffman is _ops.gemv_bf16_huffman if huffman else gemv_bf16_ans is _ops.gemv_bf16_ans):
         return None
     return _lib.eager().linear(input, getattr(weight, '_buffers', None), bias, huffman)
 
 
 def _eager_weight(weight: HuffmanWeight, huffman: bool) -> Optional[Tensor]:
     """The same for a weight that is decoded."""
-    if torch.compiler.is_compiling():
+    if torch.compiler.is_compiling() or not (
+            huffman_decode is _ops.huffman_decode if huffman else ans_decode is _ops.ans_decode):
         return None
     return _lib.eager().weight(getattr(weight, '_buffers', None), huffman)
 
