@@ -16,6 +16,11 @@ int bhi_launch_status(const char* what) {
     return (int)e;
 }
 
+std::mutex& bhi_launches_mutex() {
+    static std::mutex m;
+    return m;
+}
+
 extern "C" uint64_t bhi_stream_capture_id(void* stream) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     unsigned long long id = 0;

@@ -460,6 +460,8 @@ static inline int launch_wide(const bhi_gemv_member* weight, const void* X, int 
     a.counters = (uint32_t*)workspace;
     a.partial = (float*)(packed + packed_bytes);
     const int K = split_k * Ks, pieces = wa.tiles * (K / 32);
+    // both launches before another thread's on this stream: its pack_x_kernel would write over this call's X
+    const std::lock_guard<std::mutex> in_a_row(bhi_launches_mutex());
     hipLaunchKernelGGL(pack_x_kernel, dim3((unsigned)((pieces + 3) / 4)), dim3(256), 0, stream, (const uint16_t*)X, (u32x4v_t*)packed,
                        batch, K, wa.tiles);
     const uint16_t* x = (const uint16_t*)packed;

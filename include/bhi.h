@@ -226,7 +226,9 @@ int64_t bhi_tile_workspace_bytes(int split_k, int M, int Ks, int batch);
 
 /* The product for 17..640 rows of X (no counterpart in the reference, as above): one weight with M a multiple
  * of 64 and no residual, X aligned to 16 bytes, Y to 8.  The workspace (16-byte aligned, bhi_wide_workspace_bytes: 1 KiB of
- * counters under the rules above, X in the kernel's order, partial sums) is always needed.  A bias is
+ * counters under the rules above, X in the kernel's order, partial sums) is always needed.  A call enqueues two
+ * launches that meet there, one right after the other also where several threads call on one stream: calls on
+ * one stream may share a workspace, calls on streams that may overlap may not.  A bias is
  * added as by the tiled product.  bhi_wide_slices: how many blocks along K share 64 weight rows. */
 int bhi_wide_bf16_huffman(const bhi_gemv_member* weight, const void* X, int split_k, int Ks, int batch,
                           void* workspace, int64_t workspace_bytes, void* stream);

@@ -102,3 +102,33 @@ def test_wide_product_rejections(cuda):
                                         (x.data_ptr() + 2, ws.data_ptr(), need, b"aligned")):
         assert lib.bhi_wide_bf16_huffman(member, x_ptr, 1, 1024, 40, ws_ptr, nbytes, None) != 0
         assert text in lib.bhi_last_error_string()
+
+
+def test_two_threads_on_one_stream_keep_their_own_x(cuda):
+    """Both use the workspace of the stream that they share; every result is compared."""
+    import threading
+    from bf16_huffman_infer_amd import ops
+    mods = [_cls(algo).compress(gaussian_weight(512, 1024, seed=i)).cuda() for i, algo in enumerate(("huffman", "ans"))]
+    g = torch.Generator().manual_seed(9)
+    xs = [[torch.randn(rows, 1, 1024, generator=g).bfloat16().cuda() for rows in sizes] for sizes in ((40, 150, 40), (40, 600, 65))]
+
+    def product(mod, x):
+        y = torch.empty(x.shape[0], 512, dtype=torch.bfloat16, device="cuda")
+        ops.wide_bf16(mod, x, y)
+        return y
+    want = [[product(mod, x) for x in mine] for mod, mine in zip(mods, xs)]
+    got, stream, start = [[], []], torch.cuda.current_stream(), threading.Barrier(2)
+
+    def calls(i):
+        with torch.cuda.stream(stream):
+            start.wait()
+            for _ in range(50):
+                got[i].append([product(mods[i], x) for x in xs[i]])
+    threads = [threading.Thread(target=calls, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i in range(2):
+        assert len(got[i]) == 50
+        assert all(torch.equal(y, w) for ys in got[i] for y, w in zip(ys, want[i]))
