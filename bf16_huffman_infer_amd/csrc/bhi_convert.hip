@@ -111,7 +111,8 @@ __device__ __forceinline__ int count_below(const unsigned long long* a, int n, u
 }
 
 // counts: descending, with ids[i] the pair of counts[i]; pairs of one count in ascending order.
-// info: expected bits, code length of ESC, whether pairs escape.
+// info: expected bits, code length of ESC, whether pairs escape; -1, 0, 0 and no tables for counts that are negative or
+// not descending: the places of the leaves below come from searches that rely on the order.
 __global__ __launch_bounds__(kCodeThreads)
 void pair_code_kernel(const unsigned long long* __restrict__ counts, const long long* __restrict__ ids, uint32_t* __restrict__ enc,
                       uint32_t* __restrict__ dec, long long* __restrict__ info) {
@@ -121,17 +122,20 @@ void pair_code_kernel(const unsigned long long* __restrict__ counts, const long 
     __shared__ uint8_t lengths[2][kCodeSymbols];                          // of the cut-off at hand and of the best one
     __shared__ uint16_t id_of[kMaxCoded];
     __shared__ unsigned long long sums[2];
-    __shared__ uint32_t seen[4], chosen[kTableBits], per_length[kTableBits + 2], first_code[kTableBits + 2];
+    __shared__ uint32_t unfit, seen[4], chosen[kTableBits], per_length[kTableBits + 2], first_code[kTableBits + 2];
     const int tid = threadIdx.x;
     if (tid < 2) sums[tid] = 0;
     if (tid < 4) seen[tid] = 0;
+    if (tid == 0) unfit = 0;
     __syncthreads();
     {
         const unsigned long long least[4] = {1, 2, 4, 16};
         unsigned long long sum = 0;
         uint32_t n[4] = {0, 0, 0, 0};
+        bool fits = true;
         for (int i = tid; i < 65536; i += kCodeThreads) {
             const unsigned long long c = counts[i];
+            fits = fits && (long long)c >= 0 && (i == 0 || counts[i - 1] >= c);
             sum += c;
 #pragma unroll
             for (int k = 0; k < 4; ++k) n[k] += c >= least[k] ? 1 : 0;
@@ -139,6 +143,12 @@ void pair_code_kernel(const unsigned long long* __restrict__ counts, const long 
         atomicAdd(&sums[0], sum);
 #pragma unroll
         for (int k = 0; k < 4; ++k) atomicAdd(&seen[k], n[k]);
+        if (!fits) atomicOr(&unfit, 1u);
+    }
+    __syncthreads();
+    if (unfit) {
+        if (tid < 3) info[tid] = tid == 0 ? -1 : 0;
+        return;
     }
     for (int i = tid; i < kMaxCoded; i += kCodeThreads) id_of[i] = (uint16_t)ids[i];
     for (int i = tid; i <= (int)kEscIndex; i += kCodeThreads) enc[i] = 0;

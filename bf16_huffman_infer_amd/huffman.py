@@ -128,7 +128,7 @@ class LUTHuffmanEncoder:
         # one copy to the host, and with it one wait
         words = torch.cat((enc, dec, info.view(torch.int32), torch.stack((counts.min(), counts.max())).view(torch.int32))).cpu().numpy()
         bits, esc_length, escapes, low, high = words[ESC_INDEX + 1 + (1 << TABLE_BITS):].copy().view(np.int64).tolist()
-        if low < 0 or high <= 0:
+        if low < 0 or high <= 0:                      # with a negative count the kernel left the tables alone
             return False
         self.enc_table[:] = words[:ESC_INDEX + 1].view(np.uint32)
         self.dec_table[:] = words[ESC_INDEX + 1:ESC_INDEX + 1 + (1 << TABLE_BITS)].view(np.uint32)

@@ -316,7 +316,8 @@ def pair_histogram(exp: Tensor) -> Tensor:
 def pair_code(counts: Tensor):
     """The pair code for int64 ``[65536]`` counts on the GPU, at least one of them positive: (encoder's table int32
     ``[65537]``, decoder's int32 ``[2048]``, int64 ``[3]``: expected bits, code length of ESC, whether pairs
-    escape), as :meth:`.huffman.LUTHuffmanEncoder.build_lut` lays them out."""
+    escape), as :meth:`.huffman.LUTHuffmanEncoder.build_lut` lays them out; where a count is negative, no tables and
+    -1 expected bits."""
     if counts.numel() != 65536:
         raise RuntimeError("counts must hold 65536 entries")
     values, ids = torch.sort(counts.flatten(), descending=True, stable=True)

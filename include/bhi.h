@@ -268,7 +268,8 @@ int bhi_gemm_workspace_reset(void* workspace, int64_t workspace_bytes, void* str
  * starts_stride] (int64); a row that does not fit words int32 [n_words] is left out.
  * bhi_pair_code: the pair code for 65536 counts, sorted: counts int64 [65536] descending, ids int64 the pair of each
  * (ascending within a count), at least one count positive -> enc int32 [65537] as bhi_huffman_encode takes it,
- * dec int32 [2048] (LUT1), info int64 [3]: expected bits, code length of ESC, whether pairs escape. */
+ * dec int32 [2048] (LUT1), info int64 [3]: expected bits, code length of ESC, whether pairs escape.  Counts that are
+ * negative or not descending give no tables and info -1, 0, 0. */
 int bhi_split_planes(const void* W, void* rem, void* exp, int split_k, int M, int Ks, void* stream);
 int bhi_pair_histogram(const void* exp, int64_t bytes, void* counts, void* stream);
 int bhi_pair_code(const void* counts, const void* ids, void* enc, void* dec, void* info, void* stream);

@@ -168,3 +168,17 @@ def test_pair_code_on_the_gpu_is_the_host_one(cuda):
     for refused in (torch.zeros(65536).long(), -torch.ones(65536).long(), torch.ones(100).long()):
         with pytest.raises(AssertionError):
             LUTHuffmanEncoder().build_lut(refused.cuda())
+
+
+@pytest.mark.parametrize("negative", [1, 3, 2000])
+def test_pair_code_of_counts_that_are_partly_negative(cuda, negative):
+    """Sorted, they are not in order for the kernel's unsigned searches: it looks at them first and builds nothing."""
+    from bf16_huffman_infer_amd import ops
+    from bf16_huffman_infer_amd.huffman import LUTHuffmanEncoder
+    counts = torch.zeros(65536).long()
+    counts[:3000] = torch.arange(3000, 0, -1)
+    counts[40000:40000 + negative] = -torch.arange(1, negative + 1)
+    for here in (counts, counts.cuda()):
+        with pytest.raises(AssertionError):
+            LUTHuffmanEncoder().build_lut(here)
+    assert ops.pair_code(counts.cuda())[2].tolist() == [-1, 0, 0]
