@@ -23,6 +23,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/bhi.h"
@@ -124,30 +125,27 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     if (!PyDict_Check(args[1]) || !prefers_matrix_cores) Py_RETURN_NONE;
     const bool huffman = args[3] == Py_True;
-    try {
-        const at::Tensor* x = plain(args[0], at::kBFloat16, -1);
-        if (!x || x->dim() < 2 || x->numel() == 0) Py_RETURN_NONE;
-        const int64_t K = x->size(-1), rows = x->numel() / K;
-        if (rows > BHI_MAX_BATCH || watched() || (c10::GradMode::is_enabled() && x->requires_grad())) Py_RETURN_NONE;
-        const int device = (int)x->get_device();
-        Weight w;
-        if (!here(device) || !gather(args[1], huffman, device, w)) Py_RETURN_NONE;
-        if (w.M % 128 != 0 || w.Ks % 128 != 0 || K != w.split_k * w.Ks || prefers_matrix_cores((int)rows, (int)w.M, (int)K)) Py_RETURN_NONE;
-        if (args[2] != Py_None) {
-            const at::Tensor* bias = plain(args[2], at::kBFloat16, device);
-            if (!bias || bias->dim() != 1 || bias->size(0) != w.M) Py_RETURN_NONE;
-            w.m.bias = bias->data_ptr();
-        }
-        c10::SmallVector<int64_t, 4> shape(x->sizes().begin(), x->sizes().end());
-        shape.back() = w.M;
-        at::Tensor y = at::empty(shape, x->options().requires_grad(false));
-        w.m.Y = y.data_ptr();
-        if (gemv[huffman ? 0 : 1](&w.m, 1, x->data_ptr(), (int)w.split_k, (int)w.Ks, (int)rows, stream_of(device)) != 0) Py_RETURN_NONE;
-        return THPVariable_Wrap(std::move(y));
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
+    HANDLE_TH_ERRORS                                    // torch's own exceptions: OutOfMemoryError among them
+    const at::Tensor* x = plain(args[0], at::kBFloat16, -1);
+    if (!x || x->dim() < 2 || x->numel() == 0) Py_RETURN_NONE;
+    const int64_t K = x->size(-1), rows = x->numel() / K;
+    if (rows > BHI_MAX_BATCH || watched() || (c10::GradMode::is_enabled() && x->requires_grad())) Py_RETURN_NONE;
+    const int device = (int)x->get_device();
+    Weight w;
+    if (!here(device) || !gather(args[1], huffman, device, w)) Py_RETURN_NONE;
+    if (w.M % 128 != 0 || w.Ks % 128 != 0 || K != w.split_k * w.Ks || prefers_matrix_cores((int)rows, (int)w.M, (int)K)) Py_RETURN_NONE;
+    if (args[2] != Py_None) {
+        const at::Tensor* bias = plain(args[2], at::kBFloat16, device);
+        if (!bias || bias->dim() != 1 || bias->size(0) != w.M) Py_RETURN_NONE;
+        w.m.bias = bias->data_ptr();
     }
+    c10::SmallVector<int64_t, 4> shape(x->sizes().begin(), x->sizes().end());
+    shape.back() = w.M;
+    at::Tensor y = at::empty(shape, x->options().requires_grad(false));
+    w.m.Y = y.data_ptr();
+    if (gemv[huffman ? 0 : 1](&w.m, 1, x->data_ptr(), (int)w.split_k, (int)w.Ks, (int)rows, stream_of(device)) != 0) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
 }
 
 PyObject* weight(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -157,23 +155,20 @@ PyObject* weight(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     if (!PyDict_Check(args[0]) || !decode_huffman) Py_RETURN_NONE;
     const bool huffman = args[1] == Py_True;
-    try {
-        Weight w;
-        if (watched() || !gather(args[0], huffman, -1, w)) Py_RETURN_NONE;
-        const int device = (int)w.rem->get_device();
-        if (!here(device) || w.rem->numel() == 0) Py_RETURN_NONE;
-        at::Tensor y = at::empty({w.M, w.split_k * w.Ks}, w.rem->options().dtype(at::kBFloat16).requires_grad(false));
-        const bhi_gemv_member& m = w.m;
-        const int split_k = (int)w.split_k, M = (int)w.M, Ks = (int)w.Ks;
-        const int rc = huffman ? decode_huffman(m.A_rem, m.A_exp, m.exp_words, y.data_ptr(), m.offsets, m.table, m.table_bytes, w.unread[0],
-                                                w.unread[1], w.unread[2], m.header, split_k, M, Ks, stream_of(device))
-                               : decode_ans(m.A_rem, m.A_exp, m.exp_words, y.data_ptr(), m.offsets, m.table, split_k, M, Ks, stream_of(device));
-        if (rc != 0) Py_RETURN_NONE;
-        return THPVariable_Wrap(std::move(y));
-    } catch (const std::exception& e) {
-        PyErr_SetString(PyExc_RuntimeError, e.what());
-        return nullptr;
-    }
+    HANDLE_TH_ERRORS
+    Weight w;
+    if (watched() || !gather(args[0], huffman, -1, w)) Py_RETURN_NONE;
+    const int device = (int)w.rem->get_device();
+    if (!here(device) || w.rem->numel() == 0) Py_RETURN_NONE;
+    at::Tensor y = at::empty({w.M, w.split_k * w.Ks}, w.rem->options().dtype(at::kBFloat16).requires_grad(false));
+    const bhi_gemv_member& m = w.m;
+    const int split_k = (int)w.split_k, M = (int)w.M, Ks = (int)w.Ks;
+    const int rc = huffman ? decode_huffman(m.A_rem, m.A_exp, m.exp_words, y.data_ptr(), m.offsets, m.table, m.table_bytes, w.unread[0],
+                                            w.unread[1], w.unread[2], m.header, split_k, M, Ks, stream_of(device))
+                           : decode_ans(m.A_rem, m.A_exp, m.exp_words, y.data_ptr(), m.offsets, m.table, split_k, M, Ks, stream_of(device));
+    if (rc != 0) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(y));
+    END_HANDLE_TH_ERRORS
 }
 
 // bind(gemv Huffman, gemv rANS, decode Huffman, decode rANS, prefers_matrix_cores): addresses of the library's entry points

@@ -117,3 +117,25 @@ def test_weight_back_in_one_step(cuda, algo):
     assert _eager_weight(_layer(algo).weight.cpu(), huffman) is None
     del weight._buffers["exp"]
     assert _eager_weight(weight, huffman) is None
+
+
+def test_short_of_memory_raises_torchs_own_error(cuda):
+    lin = _layer("huffman", M=131072, K=256)               # 2 MB of output, 67 MB of weight
+    x = torch.randn(8, 256).bfloat16().cuda()
+    with torch.no_grad():
+        want = lin(x)
+        torch.cuda.empty_cache()
+        limit = torch.cuda.memory_reserved() + (1 << 20)
+        torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(0).total_memory)
+        held = []
+        try:
+            with pytest.raises(torch.OutOfMemoryError):    # what the allocator still holds
+                for _ in range(64):
+                    held.append(torch.empty(1 << 21, dtype=torch.uint8, device="cuda"))
+            for call in (lambda: lin(x), lin.weight.get_weight):
+                with pytest.raises(torch.OutOfMemoryError):
+                    call()
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+        held.clear()
+        assert torch.equal(lin(x), want)
