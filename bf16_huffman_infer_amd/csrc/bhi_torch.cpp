@@ -66,15 +66,36 @@ bool watched() {
         || at::tracer::impl::is_dispatch_enabled() || at::hasCallbacks();
 }
 
+// Allocating and launching go on without the interpreter lock, as through ctypes and torch's own calls: an allocator that
+// frees and waits, or a launch into a full queue, stops no other thread.
+struct WithoutGil {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~WithoutGil() { PyEval_RestoreThread(state); }
+};
+
 // A weight module's buffers as a kernel takes them (m.Y is left open).  False where they are not what the ops accept.
 struct Weight {
     int64_t split_k, M, Ks;
     const at::Tensor* rem;
+    PyObject* held[kLut + 1] = {};                  // the module may be given other buffers while the lock is released
     const void* unread[3];                          // LUT2..LUT4: carried by the op's signature
     bhi_gemv_member m;
+    Weight() = default;
+    Weight(const Weight&) = delete;
+    ~Weight() {
+        for (PyObject* o : held) Py_XDECREF(o);
+    }
 };
 bool gather(PyObject* buffers, bool huffman, int device, Weight& w) {
-    auto buffer = [&](Name name, at::ScalarType type) { return plain(PyDict_GetItem(buffers, names[name]), type, device); };
+    auto buffer = [&](Name name, at::ScalarType type) -> const at::Tensor* {
+        PyObject* const o = PyDict_GetItem(buffers, names[name]);
+        const at::Tensor* const t = plain(o, type, device);
+        if (t) {
+            Py_INCREF(o);
+            w.held[name] = o;
+        }
+        return t;
+    };
     w.rem = buffer(kRem, at::kByte);
     if (!w.rem || w.rem->dim() != 3) return false;
     if (device < 0) device = (int)w.rem->get_device();                       // the rest lies where rem does
@@ -141,9 +162,15 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
     }
     c10::SmallVector<int64_t, 4> shape(x->sizes().begin(), x->sizes().end());
     shape.back() = w.M;
-    at::Tensor y = at::empty(shape, x->options().requires_grad(false));
-    w.m.Y = y.data_ptr();
-    if (gemv[huffman ? 0 : 1](&w.m, 1, x->data_ptr(), (int)w.split_k, (int)w.Ks, (int)rows, stream_of(device)) != 0) Py_RETURN_NONE;
+    at::Tensor y;
+    int rc;
+    {
+        const WithoutGil released;
+        y = at::empty(shape, x->options().requires_grad(false));
+        w.m.Y = y.data_ptr();
+        rc = gemv[huffman ? 0 : 1](&w.m, 1, x->data_ptr(), (int)w.split_k, (int)w.Ks, (int)rows, stream_of(device));
+    }
+    if (rc != 0) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -160,12 +187,17 @@ PyObject* weight(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (watched() || !gather(args[0], huffman, -1, w)) Py_RETURN_NONE;
     const int device = (int)w.rem->get_device();
     if (!here(device) || w.rem->numel() == 0) Py_RETURN_NONE;
-    at::Tensor y = at::empty({w.M, w.split_k * w.Ks}, w.rem->options().dtype(at::kBFloat16).requires_grad(false));
     const bhi_gemv_member& m = w.m;
     const int split_k = (int)w.split_k, M = (int)w.M, Ks = (int)w.Ks;
-    const int rc = huffman ? decode_huffman(m.A_rem, m.A_exp, m.exp_words, y.data_ptr(), m.offsets, m.table, m.table_bytes, w.unread[0],
-                                            w.unread[1], w.unread[2], m.header, split_k, M, Ks, stream_of(device))
-                           : decode_ans(m.A_rem, m.A_exp, m.exp_words, y.data_ptr(), m.offsets, m.table, split_k, M, Ks, stream_of(device));
+    at::Tensor y;
+    int rc;
+    {
+        const WithoutGil released;
+        y = at::empty({w.M, w.split_k * w.Ks}, w.rem->options().dtype(at::kBFloat16).requires_grad(false));
+        rc = huffman ? decode_huffman(m.A_rem, m.A_exp, m.exp_words, y.data_ptr(), m.offsets, m.table, m.table_bytes, w.unread[0],
+                                      w.unread[1], w.unread[2], m.header, split_k, M, Ks, stream_of(device))
+                     : decode_ans(m.A_rem, m.A_exp, m.exp_words, y.data_ptr(), m.offsets, m.table, split_k, M, Ks, stream_of(device));
+    }
     if (rc != 0) Py_RETURN_NONE;
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS

@@ -139,3 +139,26 @@ def test_short_of_memory_raises_torchs_own_error(cuda):
             torch.cuda.set_per_process_memory_fraction(1.0)
         held.clear()
         assert torch.equal(lin(x), want)
+
+
+@pytest.mark.parametrize("algo", ["huffman", "ans"])
+def test_launches_without_the_interpreter_lock(cuda, algo):
+    """In the place of the library's entry points stands the interpreter's own question whether this thread holds the
+    lock: 0, which the step takes for a launch, where it does not."""
+    import ctypes
+    from bf16_huffman_infer_amd import _lib
+    lin, huffman = _layer(algo), algo == "huffman"
+    x = torch.randn(1, 1024).bfloat16().cuda()
+    with torch.no_grad():
+        want = lin(x)
+        asked = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+        lib, step = _lib.load(), _lib.eager()
+        prefers = ctypes.cast(lib.bhi_prefers_matrix_cores, ctypes.c_void_p).value
+        step.bind(asked, asked, asked, asked, prefers)
+        try:
+            taken = [step.linear(x, lin.weight._buffers, None, huffman), step.weight(lin.weight._buffers, huffman)]
+        finally:
+            step.bind(*(ctypes.cast(f, ctypes.c_void_p).value for f in (
+                lib.bhi_gemv_bf16_huffman_grouped, lib.bhi_gemv_bf16_ans_grouped, lib.bhi_huffman_decode, lib.bhi_ans_decode)), prefers)
+        assert taken[0] is not None and taken[1] is not None
+        assert torch.equal(lin(x), want)
