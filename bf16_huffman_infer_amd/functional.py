@@ -139,6 +139,9 @@ def mv_ans(A_rem: Tensor, A_exp: Tensor, X: Tensor, offsets: Tensor, LUT: Tensor
     return Y
 
 
+_MV_HUFFMAN, _MV_ANS = mv_huffman, mv_ans           # what nobody has put a wrapper in the place of
+
+
 class HuffmanWeight(nn.Module):
     """A BF16 weight ``[M, K]`` stored as a raw sign/mantissa plane plus a Huffman-coded
     exponent stream.  Passing the module as the weight of ``F.linear`` runs the fused
@@ -962,16 +965,18 @@ def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tens
 
 def _eager(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], huffman: bool) -> Optional[Tensor]:
     """A call of the GEMV that nothing watches, in one native step (``bhi_torch.cpp``); None where the path through the
-    custom ops has to take it or to refuse it.  Whoever has put a wrapper in the place of this module's ops (to
-    count or to log calls) watches too."""
+    custom ops has to take it or to refuse it.  Whoever has put a wrapper in the place of this module's
+    ``mv_huffman`` / ``mv_ans`` or of the ops that they and a call with a bias run, ``gemv_bf16_huffman`` /
+    ``gemv_bf16_ans`` and ``gemv_bf16_grouped`` (to count or to log calls), watches too."""
     if torch.compiler.is_compiling() or gemv_bf16_grouped is not _ops.gemv_bf16_grouped or not (
-            gemv_bf16_huffman is _ops.gemv_bf16_huffman if huffman else gemv_bf16_ans is _ops.gemv_bf16_ans):
+            mv_huffman is _MV_HUFFMAN and gemv_bf16_huffman is _ops.gemv_bf16_huffman if huffman
+            else mv_ans is _MV_ANS and gemv_bf16_ans is _ops.gemv_bf16_ans):
         return None
     return _lib.eager().linear(input, getattr(weight, '_buffers', None), bias, huffman)
 
 
 def _eager_weight(weight: HuffmanWeight, huffman: bool) -> Optional[Tensor]:
-    """The same for a weight that is decoded."""
+    """The same for a weight that is decoded, by ``huffman_decode`` / ``ans_decode``."""
     if torch.compiler.is_compiling() or not (
             huffman_decode is _ops.huffman_decode if huffman else ans_decode is _ops.ans_decode):
         return None
