@@ -1,10 +1,12 @@
 """ctypes binding of libbhi_hip.so (the C ABI declared in include/bhi.h).
 
 The library is built in-tree by ``python -m bf16_huffman_infer_amd.csrc.build``.  There
-is no fallback: if it is missing every op of this package raises.
+is no fallback: if it is missing every op of this package raises.  The native step of eager calls
+(:func:`eager`) is host code only, and the ops take its calls where it is missing.
 """
 import ctypes
 import os
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbhi_hip.so")
@@ -115,20 +117,24 @@ _eager = None
 
 
 def eager():
-    """The native step of eager calls (``csrc/bhi_torch.cpp``), which gets its entry points from :func:`load`."""
+    """The native step of eager calls (``csrc/bhi_torch.cpp``), which gets its entry points from :func:`load`.  It is
+    host code that the custom ops do without: where it is missing or does not fit this torch, None, and a
+    warning the first time."""
     global _eager
     if _eager is None:
         lib = load()
         try:
             from . import _bhi_torch
         except ImportError as e:
-            raise RuntimeError("_bhi_torch.so is missing or does not fit this torch: build the extension first "
-                               "(python -m bf16_huffman_infer_amd.csrc.build)") from e
-        _bhi_torch.bind(*(ctypes.cast(f, _vp).value for f in (
-            lib.bhi_gemv_bf16_huffman_grouped, lib.bhi_gemv_bf16_ans_grouped, lib.bhi_huffman_decode, lib.bhi_ans_decode,
-            lib.bhi_prefers_matrix_cores)))
-        _eager = _bhi_torch
-    return _eager
+            _eager = False
+            warnings.warn(f"eager calls of compressed linears go through the custom ops, some 10 us of host time each: {e}; build the "
+                          "extension (python -m bf16_huffman_infer_amd.csrc.build)", RuntimeWarning, stacklevel=2)
+        else:
+            _bhi_torch.bind(*(ctypes.cast(f, _vp).value for f in (
+                lib.bhi_gemv_bf16_huffman_grouped, lib.bhi_gemv_bf16_ans_grouped, lib.bhi_huffman_decode, lib.bhi_ans_decode,
+                lib.bhi_prefers_matrix_cores)))
+            _eager = _bhi_torch
+    return _eager or None
 
 
 def check(rc: int, what: str) -> None:

@@ -972,7 +972,8 @@ def _eager(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], huffman
             mv_huffman is _MV_HUFFMAN and gemv_bf16_huffman is _ops.gemv_bf16_huffman if huffman
             else mv_ans is _MV_ANS and gemv_bf16_ans is _ops.gemv_bf16_ans):
         return None
-    return _lib.eager().linear(input, getattr(weight, '_buffers', None), bias, huffman)
+    step = _lib.eager()
+    return None if step is None else step.linear(input, getattr(weight, '_buffers', None), bias, huffman)
 
 
 def _eager_weight(weight: HuffmanWeight, huffman: bool) -> Optional[Tensor]:
@@ -980,7 +981,8 @@ def _eager_weight(weight: HuffmanWeight, huffman: bool) -> Optional[Tensor]:
     if torch.compiler.is_compiling() or not (
             huffman_decode is _ops.huffman_decode if huffman else ans_decode is _ops.ans_decode):
         return None
-    return _lib.eager().weight(getattr(weight, '_buffers', None), huffman)
+    step = _lib.eager()
+    return None if step is None else step.weight(getattr(weight, '_buffers', None), huffman)
 
 
 def linear_huffman(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor] = None) -> Tensor:

@@ -58,7 +58,8 @@ def _stream(t: Tensor) -> int:
             with torch.cuda.device(index):
                 _lib.check(_lib.load().bhi_device_init(), "device_init")
             _ready_devices.add(index)
-            _lib.eager().ready(index)
+            if (step := _lib.eager()) is not None:
+                step.ready(index)
     return torch._C._cuda_getCurrentRawStream(index)
 
 
