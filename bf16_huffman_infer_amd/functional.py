@@ -857,6 +857,8 @@ def prefers_wide(rows: int, M: int, K: int, split_k: int = 1, huffman: bool = Tr
     ================================  ===========  ===========  ===========  ===========  ===========
     """
     slices = _lib.load().bhi_wide_slices(split_k, M, K // split_k)
+    if slices < 1 or M < 128 or M % 128 != 0:     # refused by the library, or by the operand check of every fused call
+        return False
     blocks = M // 64 * slices
     rounds = -(-blocks // 256)
     filled = blocks / (256 * rounds)
@@ -901,11 +903,11 @@ def _takes(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], first: 
     if not first <= rows <= last or isinstance(weight, NibbleWeight):
         return False
     split_k, M, N = _ops._buffer(weight, 'rem').shape
-    if not rule(rows, M, split_k * N, split_k, not isinstance(weight, ANSWeight)):
-        return False
     if input.dtype != torch.bfloat16 or (bias is not None and bias.dtype != torch.bfloat16) or not input.is_cuda:
         return False
-    if input.size(1) != split_k * N or input.numel() >= 2 ** 31:
+    if split_k < 1 or input.size(1) != split_k * N or input.numel() >= 2 ** 31:
+        return False
+    if not rule(rows, M, split_k * N, split_k, not isinstance(weight, ANSWeight)):
         return False
     return rows <= GEMM_MAX_ROWS or ((bias is None or tuple(bias.shape) == (M,)) and _fuses_above_32_rows(input, bias))
 
@@ -916,7 +918,7 @@ def _tiled(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool
 
 def _wide(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor]) -> bool:
     return (_takes(input, weight, bias, _ops.WIDE_MIN_ROWS, _ops.WIDE_MAX_ROWS, prefers_wide)
-            and _ops._buffer(weight, 'rem').shape[1] % 64 == 0 and (input.size(0) + 15) * input.size(1) < 2 ** 31)
+            and (input.size(0) + 15) * input.size(1) < 2 ** 31)
 
 
 def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], fused) -> Tensor:

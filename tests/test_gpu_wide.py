@@ -132,3 +132,23 @@ def test_two_threads_on_one_stream_keep_their_own_x(cuda):
     for i in range(2):
         assert len(got[i]) == 50
         assert all(torch.equal(y, w) for ys in got[i] for y, w in zip(ys, want[i]))
+
+
+@pytest.mark.parametrize("algo", ["huffman", "ans"])
+@pytest.mark.parametrize("M", [4, 32, 64, 96])
+def test_heights_that_fused_calls_refuse_are_decoded(cuda, algo, M):
+    """Weights that the package's conversion does not make, but the library takes: the first rows of one that it makes."""
+    from bf16_huffman_infer_amd.functional import CompressedLinear, check_layout
+    whole = gaussian_weight(128, 256, seed=M)
+    kwargs = {n: t.cpu() for n, t in _cls(algo).compress_split_n(whole, n=1).kwargs().items()}
+    assert not kwargs["offsets"][0].view(-1, 4)[:, 1:].any()                    # one task per row group, in their order
+    words = int(kwargs["offsets"][0, M])
+    kwargs.update(rem=kwargs["rem"][:, :M].contiguous(), offsets=kwargs["offsets"][:, :M].contiguous(),
+                  exp=torch.cat((kwargs["exp"][:words], torch.zeros(2048, dtype=torch.int32))))
+    weight = _cls(algo)(**kwargs)
+    check_layout(weight)
+    lin = CompressedLinear(weight, None).cuda()
+    assert torch.equal(lin.weight.get_weight().cpu(), whole[:M])
+    for rows in (129, 200, 640):
+        x = torch.randn(rows, 256, generator=torch.Generator().manual_seed(rows)).bfloat16().cuda()
+        _check(lin(x), x, whole[:M])

@@ -108,3 +108,18 @@ def test_wide_rule():
     assert [r for r in (33, 80, 81, 192, 193, 320, 321) if prefers_wide(r, 18944, 3584)] == [81, 192, 193, 320]
     assert [r for r in (33, 80, 81, 192, 193, 320) if prefers_wide(r, 18944, 3584, 1, False)] == [81, 192]
     assert not any(prefers_wide(r, 512, 1024) for r in (17, 33, 64, 128, 300, 640))
+
+
+# in front of the rules: what the package's own conversion does not make (it wants M % 128 == 0), but check_layout and the library take
+@pytest.mark.parametrize("M", [4, 32, 60, 96, 192, 8256, 12224])
+@pytest.mark.parametrize("rows", [17, 40, 128, 200, 640])
+def test_wide_rule_leaves_heights_that_fused_calls_refuse(M, rows):
+    from bf16_huffman_infer_amd.functional import prefers_wide
+    for K, split_k in ((1024, 1), (4096, 1), (12288, 3)):
+        assert not prefers_wide(rows, M, K, split_k, True) and not prefers_wide(rows, M, K, split_k, False)
+
+
+def test_wide_rule_leaves_widths_that_the_library_refuses():
+    from bf16_huffman_infer_amd.functional import prefers_wide
+    for M, K, split_k in ((128, 100, 1), (128, 64, 1), (16384, 4000, 1), (16384, 8192, 3), (128, 1 << 20, 1)):
+        assert not any(prefers_wide(rows, M, K, split_k) for rows in (17, 40, 200, 640)), (M, K, split_k)
