@@ -907,7 +907,8 @@ def _takes(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], first: 
         return False
     if split_k < 1 or input.size(1) != split_k * N or input.numel() >= 2 ** 31:
         return False
-    if not rule(rows, M, split_k * N, split_k, not isinstance(weight, ANSWeight)):
+    # whole numbers: under torch.jit.trace these are tensors, which the rules would keep
+    if not rule(int(rows), int(M), int(split_k * N), int(split_k), not isinstance(weight, ANSWeight)):
         return False
     return rows <= GEMM_MAX_ROWS or ((bias is None or tuple(bias.shape) == (M,)) and _fuses_above_32_rows(input, bias))
 

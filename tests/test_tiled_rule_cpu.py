@@ -123,3 +123,23 @@ def test_wide_rule_leaves_widths_that_the_library_refuses():
     from bf16_huffman_infer_amd.functional import prefers_wide
     for M, K, split_k in ((128, 100, 1), (128, 64, 1), (16384, 4000, 1), (16384, 8192, 3), (128, 1 << 20, 1)):
         assert not any(prefers_wide(rows, M, K, split_k) for rows in (17, 40, 200, 640)), (M, K, split_k)
+
+
+def test_rules_are_asked_with_whole_numbers():
+    """Under torch.jit.trace sizes are tensors, and the rules remember what they were asked."""
+    import types
+    from bf16_huffman_infer_amd.functional import _takes
+    asked, x = [], torch.zeros(24, 512, dtype=torch.bfloat16)
+    weight = types.SimpleNamespace(rem=torch.zeros(2, 128, 256, dtype=torch.uint8))
+
+    def rule(*args):
+        asked.append(args)
+        return True
+
+    def step(v, rem):
+        of_gpu = types.SimpleNamespace(size=v.size, numel=v.numel, dtype=v.dtype, is_cuda=True)
+        assert type(v.size(0)) is torch.Tensor
+        assert _takes(of_gpu, types.SimpleNamespace(rem=rem), None, 17, 32, rule)
+        return v + 1
+    torch.jit.trace(step, (x, weight.rem), check_trace=False)
+    assert asked and all(type(a) in (int, bool) for args in asked for a in args) and asked[0][:4] == (24, 128, 512, 2)
