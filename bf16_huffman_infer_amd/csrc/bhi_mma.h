@@ -229,7 +229,7 @@ void mma_kernel(const uint16_t* __restrict__ X, int first1, int first2, int firs
             // Every load of a window is unconditional, and a step's operands are requested again as soon as it has used
             // them, so that the compiler can count what is in flight: with a second set that was copied, and
             // loads behind branches, each window ended with a wait for all of them (12288x4096 at 16 rows 25.3 us,
-            // 24.0 so; the 8-row step of a Qwen2.5-7B layer 118.1 -> 117.4).  A row prefetch without room
+            // 24.0 so; at 8 rows no difference beyond the noise).  A row prefetch without room
             // goes to the block's first rows, which are cached; the very last window's X is the task's first again.
             uint32_t rows[S];
             bool pending = cur.template room<S>();

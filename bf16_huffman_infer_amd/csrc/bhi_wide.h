@@ -2,8 +2,8 @@
 // every wavefront multiplies all of them with its own part of X.
 //
 // What bounds the range.  tile_kernel keeps a wavefront's decoded weights in its registers, so every wavefront
-// reads all of X from LDS for sixteen weight rows; from 65 rows those reads and the table lookups fill the LDS
-// pipe (77 rows of 4096x12288: 2800 of 3900 clocks a step), and its windows of X end at 128 rows.  Decoding to
+// reads all of X from LDS for sixteen weight rows; from 65 rows those reads and the table lookups take most of a
+// step (77 rows of 4096x12288: 2800 of 3900 clocks, counted from the instructions), and its windows of X end at 128 rows.  Decoding to
 // BF16 and a library GEMM moves the weight through memory twice (12288x4096: 32 us to write it, 37-47 us to
 // read and multiply it at 144 to 512 rows).
 //
@@ -30,11 +30,14 @@
 //   3584x18944  Huff    54.3 / 40.7  60.9 / 43.4  65.6 / 47.9  69.1 / 51.6   130 / 61.7   138 / 77.9   213 / 101
 //   8192x8192   rANS    65.7 / 44.6  69.4 / 46.5  71.0 / 49.8  73.2 / 51.5  96.5 / 58.6   103 / 74.8   117 / 100
 //
-// (functional.prefers_wide picks the sides.)  What bounds it now: up to 9 tiles the LDS pipe (lookups and weight reads,
-// 0.8 us a step), from 20 tiles on the loads of X, which every block reads whole (0.041 us per tile and step, 41
-// bytes a clock and unit; 0.057 us while a tile of X was one piece of memory, whose chunks all fell on the
-// same channels of the cache: 640 rows of 12288x4096 92 us instead of 84), and the units without a block: 18944
-// rows are 296 blocks on 256 units.
+// (functional.prefers_wide picks the sides.)  What bounds it now, by counters (share of the time that a compute unit
+// with a block has the LDS pipe / matrix cores / VALU / address unit of its vector memory busy): 77 rows of 4096x12288
+// 44 / 12 / 22 / 54 %, and wavefronts wait half of their time for memory or LDS: nothing is full, a step is as long
+// as its chain of lookups between two barriers at two wavefronts per SIMD; 300 rows of 11008x4096 rANS
+// 58 / 35 / 43 / 61 %; 640 rows of 12288x4096 36 / 53 / 25 / 81 %: the loads of X, which every block reads whole
+// (0.041 us per tile and step, 41 bytes a clock and unit; 0.057 us while a tile of X was one piece of memory, whose
+// chunks all fell on the same channels of the cache: 92 us instead of 84).  Beside that the units without a block:
+// 11008 rows are 172 blocks for 256 units, 18944 are 296.
 #pragma once
 // (included by bhi_task.h users after bhi_tile.h, whose argument block and workspace rules it shares)
 
@@ -131,7 +134,8 @@ __device__ __forceinline__ void decode_wide(AnsCursor (&cur)[kWideGroups], const
 }
 
 // X in the order the matrix instructions take it: 1 KB per tile of sixteen rows and chunk of 32 columns, the tiles of
-// a chunk side by side (about 2.5 us: its launch).  Rows past the batch repeat its last row.
+// a chunk side by side.  Under a trace, which adds 1 to 2 us, 2.3 us for 40 rows of 4096 columns, 3.2 for 77 of 12288,
+// 5.4 for 300 of 4096 and 6.3 for 640: its launch and one round trip, and a tenth of the call.  Rows past the batch repeat its last row.
 static __global__ __launch_bounds__(256) void pack_x_kernel(const uint16_t* __restrict__ X, u32x4v_t* __restrict__ out, int rows, int K, int tiles) {
     const int piece = (int)(blockIdx.x * 4 + threadIdx.x / kLanes), lane = threadIdx.x & (kLanes - 1);
     const int tile = piece % tiles, chunk = piece / tiles;

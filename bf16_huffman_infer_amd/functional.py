@@ -826,7 +826,8 @@ def prefers_tiles(rows: int, M: int, K: int, split_k: int = 1, huffman: bool = T
         # a small layer's weight stays in the caches between the decoder and the GEMM
         return huffman or rows <= 48 or M * K >= 7 << 18
     # Above, the library's kernel gains on this one with every row.  With one task per row group and four to
-    # five wavefronts for a unit, blocks of six or eight leave a quarter of the units idle.
+    # five wavefronts for a unit, blocks of six or eight leave a quarter of the units idle (F.linear asks prefers_wide
+    # first, which takes all of these).
     if M * K < 16 << 20:
         return False
     return huffman or rows <= 80 or not (tasks == 1 and 4 * 4096 < M < 5 * 4096)
@@ -855,6 +856,10 @@ def prefers_wide(rows: int, M: int, K: int, split_k: int = 1, huffman: bool = Tr
     18944x3584 (two rounds, 58 %) r   55.5 / 63.0  59.5 / 67.6  71.0 / 69.2  90.5 / 90.9   130 / 149
     32768x2048 (two rounds, full) r   36.4 / 42.7  42.8 / 45.6  47.1 / 47.0  86.2 / 67.1   128 / 113
     ================================  ===========  ===========  ===========  ===========  ===========
+
+    The limits lie between neighbouring measured shapes and row counts and have no other reason.  Of the entries here and
+    in ``bhi_wide.h`` four are left to the slower path: 512x1024 at 64 rows, 1024x4096 at 32, rANS 3584x3584 at 32
+    (by 0.4 to 1.0 us) and 4096x4096 at 300 (by 2.4).
     """
     slices = _lib.load().bhi_wide_slices(split_k, M, K // split_k)
     if slices < 1 or M < 128 or M % 128 != 0:     # refused by the library, or by the operand check of every fused call
@@ -947,7 +952,8 @@ def _linear_compressed(input: Tensor, weight: HuffmanWeight, bias: Optional[Tens
                 output += bias[None, :]
     elif matrix_cores and rows > MAX_FUSED_BATCH and (
             product := _ops.wide_bf16 if _wide(input, weight, bias) else _ops.tile_bf16 if _tiled(input, weight, bias) else None):
-        # 17..640 rows where the rules say so: as below, sixteen weight rows at a time
+        # 17..640 rows where the rules say so: as below, but the matrix instructions take sixteen weight rows, in the
+        # wide product out of LDS, where a block has decoded 64
         x = (input if rows <= GEMM_MAX_ROWS else input.contiguous()).view(-1, split_k, N).contiguous()
         if x.data_ptr() % 16:
             x = x.clone()

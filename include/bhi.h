@@ -182,7 +182,8 @@ int bhi_rms_norm(const void* X, const void* gamma, void* out, int rows, int K, f
 int bhi_silu_mul(const void* gate, const void* up, void* out, int64_t n, void* stream);
 
 /* Fused decode + matrix product for 1..32 rows of X (meant for 9..16; up to 8 the GEMV
- * entry points are faster, above 16 mostly bhi_tile_bf16_*): Y = X W^T (+ bias) with the weights going from the decoder's
+ * entry points are faster, above 16 mostly bhi_tile_bf16_* and
+ * bhi_wide_bf16_*): Y = X W^T (+ bias) with the weights going from the decoder's
  * registers straight into matrix-core instructions.  Replaces the reference's path above
  * eight rows, huffman_decode / ans_decode to a BF16 matrix followed by a dense GEMM
  * (functional.py:405-407, 460-462; kernel.cu:510-587, 851-919), which writes and re-reads

@@ -110,6 +110,37 @@ def test_wide_rule():
     assert not any(prefers_wide(r, 512, 1024) for r in (17, 33, 64, 128, 300, 640))
 
 
+# (M, K, Huffman, rows where the wide product was faster by more than 2 %, rows where the other path was): every such entry of the
+# tables in prefers_wide and bhi_wide.h but the four that prefers_wide names as left to the slower side
+WIDE_MEASURED = [
+    (512, 1024, True, [], [32, 256, 640]),
+    (1024, 4096, True, [64], [256, 640]),
+    (2048, 2048, False, [64, 96], [256, 640]),
+    (4608, 3584, True, [64, 96, 256], [32, 640]),
+    (12288, 4096, True, [96, 128, 192, 256, 300, 512, 640], [32, 33]),
+    (3584, 3584, False, [64, 96], [640]),
+    (4096, 12288, False, [32, 64, 96, 256, 640], []),
+    (8192, 8192, True, [32, 64, 96, 256, 640], []),
+    (18944, 3584, True, [96, 128, 192, 256, 300], [32, 33, 64, 512, 640]),
+    (18944, 3584, False, [96], [32, 64, 640]),
+    (32768, 2048, False, [256, 640], [32, 64]),
+    (4096, 4096, True, [33, 64, 96, 128, 192], [512]),
+    (12288, 4096, False, [96, 128, 192, 300, 512], [33]),
+    (4096, 12288, True, [33, 64, 96, 128, 192, 300, 512], []),
+    (3584, 18944, True, [33, 64, 96, 128, 192, 300, 512], []),
+    (8192, 8192, False, [33, 64, 96, 128, 192, 300, 512], []),
+]
+
+
+@pytest.mark.parametrize("M,K,huffman,wide,other", WIDE_MEASURED)
+def test_wide_product_is_chosen_where_it_was_faster(M, K, huffman, wide, other):
+    from bf16_huffman_infer_amd.functional import prefers_wide
+    from bf16_huffman_infer_amd.utils import get_block_size_n
+    split_k, = get_block_size_n(torch.empty(1, K, device="meta"))
+    assert [r for r in wide if not prefers_wide(r, M, K, split_k, huffman)] == []
+    assert [r for r in other if prefers_wide(r, M, K, split_k, huffman)] == []
+
+
 # in front of the rules: what the package's own conversion does not make (it wants M % 128 == 0), but check_layout and the library take
 @pytest.mark.parametrize("M", [4, 32, 60, 96, 192, 8256, 12224])
 @pytest.mark.parametrize("rows", [17, 40, 128, 200, 640])
