@@ -139,7 +139,9 @@ def mv_ans(A_rem: Tensor, A_exp: Tensor, X: Tensor, offsets: Tensor, LUT: Tensor
     return Y
 
 
-_MV_HUFFMAN, _MV_ANS = mv_huffman, mv_ans           # what nobody has put a wrapper in the place of
+# what the names of these functions mean while nobody has put a wrapper in their place
+_MV_HUFFMAN, _MV_ANS, _GEMV_HUFFMAN, _GEMV_ANS, _GEMV_GROUPED = (
+    mv_huffman, mv_ans, gemv_bf16_huffman, gemv_bf16_ans, gemv_bf16_grouped)
 
 
 class HuffmanWeight(nn.Module):
@@ -977,9 +979,9 @@ def _eager(input: Tensor, weight: HuffmanWeight, bias: Optional[Tensor], huffman
     custom ops has to take it or to refuse it.  Whoever has put a wrapper in the place of this module's
     ``mv_huffman`` / ``mv_ans`` or of the ops that they and a call with a bias run, ``gemv_bf16_huffman`` /
     ``gemv_bf16_ans`` and ``gemv_bf16_grouped`` (to count or to log calls), watches too."""
-    if torch.compiler.is_compiling() or gemv_bf16_grouped is not _ops.gemv_bf16_grouped or not (
-            mv_huffman is _MV_HUFFMAN and gemv_bf16_huffman is _ops.gemv_bf16_huffman if huffman
-            else mv_ans is _MV_ANS and gemv_bf16_ans is _ops.gemv_bf16_ans):
+    if torch.compiler.is_compiling() or gemv_bf16_grouped is not _GEMV_GROUPED or not (
+            mv_huffman is _MV_HUFFMAN and gemv_bf16_huffman is _GEMV_HUFFMAN if huffman
+            else mv_ans is _MV_ANS and gemv_bf16_ans is _GEMV_ANS):
         return None
     step = _lib.eager()
     return None if step is None else step.linear(input, getattr(weight, '_buffers', None), bias, huffman)
