@@ -3,7 +3,8 @@ to find at zero and leaves at zero, followed by partial results.
 
 Launches that may overlap must not share one, so a workspace belongs to
 
-* the (device, stream) of eager launches, which run one after the other;
+* the (device, stream) of eager launches, which run one after the other, whichever threads enqueue them (the library
+  enqueues the launches of one call in a row);
 * the CAPTURE of recorded launches, not to the stream they were recorded on: graphs recorded one
   after the other on one stream (torch records every graph on the same one) may be replayed
   side by side, and none may depend on another having run first.
